@@ -201,6 +201,9 @@ struct hg_ctx {
   unsigned long long* rs_d;
   int* nan_d;
   unsigned long long* gs_info;
+  // workspace of the gauss_seidel solves (a context with one of them)
+  double* sor_ws = nullptr;
+  long sor_doubles = 0;
   hg::JacobiWork jw{};
   double* jdiff_host_dummy = nullptr;
   // pinned host mirrors
@@ -672,7 +675,8 @@ void SolveRowsIterative(hg_ctx* c, int32_t solver, hg::Rows rows, const double* 
     return;
   }
   if (solver == HG_SOLVER_GAUSS_SEIDEL)
-    hg::LaunchGsWavefront(c->st, nx, ny, rows, k, x, tol, limit, omega, c->gs_info);
+    hg::LaunchSor(c->st, nx, ny, rows, k, x, tol, limit, omega, c->gs_info, c->sor_ws,
+                  c->sor_doubles);
   else if (solver == HG_SOLVER_LU_RELAXED)
     hg::LaunchLuRelaxed(c->st, nx, ny, rows, k, x, w.xa, w.xb, tol, limit, omega, c->gs_info);
   else
@@ -1159,6 +1163,12 @@ hg_status hg_create(const hg_config* cfg_in, hg_ctx** out) {
     c->rs_d = (unsigned long long*)c->Alloc(1);
     c->nan_d = (int*)c->Alloc(1);
     c->gs_info = (unsigned long long*)c->Alloc(2);
+    if (cfg.linear_solver_pressure == HG_SOLVER_GAUSS_SEIDEL ||
+        cfg.linear_solver_velocity == HG_SOLVER_GAUSS_SEIDEL ||
+        (cfg.heat_enable && cfg.linear_solver_heat == HG_SOLVER_GAUSS_SEIDEL)) {
+      c->sor_doubles = hg::SorWorkspace(cfg.nx, cfg.ny);
+      if (c->sor_doubles > 0) c->sor_ws = c->Alloc(c->sor_doubles);
+    }
     c->jw.xa = c->Alloc(nc);
     c->jw.xb = c->Alloc(nc);
     c->jw.diff = (unsigned long long*)c->Alloc(cfg.lu_relaxed_num_iters_limit + 2);

@@ -179,6 +179,13 @@ void LaunchLuWavefront(hipStream_t st, int nx, int ny, Rows a, const double* k0,
 // info[1] = final max|corr| (as double bits).
 void LaunchGsWavefront(hipStream_t st, int nx, int ny, Rows a, const double* k, double* x,
                        double tol, int limit, double omega, unsigned long long* info);
+// The same with many sweeps in flight (sor.hip), bit for bit, on a workspace
+// of `ws_doubles` doubles; with fewer than SorWorkspace(nx, ny) it keeps
+// fewer sweeps in flight, and without room for two (or where the shorter side
+// exceeds 1024 or the longer is under 8) it runs LaunchGsWavefront.
+long SorWorkspace(int nx, int ny);
+void LaunchSor(hipStream_t st, int nx, int ny, Rows a, const double* k, double* x, double tol,
+               int limit, double omega, unsigned long long* info, double* ws, long ws_doubles);
 // LuDecompositionRelaxed (linear.hpp:578-651) from zero, every iteration in
 // one persistent workgroup: res receives the solution; corr and f are
 // scratch cell arrays; info as for LaunchGsWavefront.

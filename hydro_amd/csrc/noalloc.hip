@@ -127,8 +127,9 @@ hg_status hg_stencil_solve_noalloc(int32_t nx, int32_t ny, const double* s, cons
       hg::LaunchLuRb(st, nx, ny, rows, k, k, a1, a2, a0, a0, x, a3);
       break;
     case HG_SOLVER_GAUSS_SEIDEL:
-      hg::LaunchGsWavefront(st, nx, ny, rows, k, x, opts->tolerance, limit,
-                            opts->relaxation_factor, info);
+      // the solver's workspace: what the scratch array holds behind the header
+      hg::LaunchSor(st, nx, ny, rows, k, x, opts->tolerance, limit, opts->relaxation_factor, info,
+                    a0, long((kScratchBytes - off_arr) / 8));
       break;
     case HG_SOLVER_LU_RELAXED:
       hg::LaunchLuRelaxed(st, nx, ny, rows, k, x, a0, a1, opts->tolerance, limit,

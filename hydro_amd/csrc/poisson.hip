@@ -74,6 +74,7 @@ hg_status hg_stencil_solve(int32_t nx, int32_t ny, const double* s, const double
     std::unique_ptr<void, std::function<void(void*)>> guard(
         (void*)st, [](void* p) { (void)hipStreamDestroy((hipStream_t)p); });
     DevBuf ds(N), dw(N), dc(N), de(N), dn(N), dk(N), dx(N), dx2(N), dz(N), dout(N), dtmp(N);
+    std::unique_ptr<DevBuf> sor_ws;
     DevBuf info(2), jdiff(size_t(std::max(opts->max_iters, 0)) + 2), jstate(2);
     const double* src[6] = {s, w, c, e, n, k};
     double* dst[6] = {ds.p, dw.p, dc.p, de.p, dn.p, dk.p};
@@ -98,8 +99,10 @@ hg_status hg_stencil_solve(int32_t nx, int32_t ny, const double* s, const double
         result = dout.p;
         break;
       case HG_SOLVER_GAUSS_SEIDEL: {
-        hg::LaunchGsWavefront(st, nx, ny, rows, dk.p, dx.p, opts->tolerance, opts->max_iters,
-                              opts->relaxation_factor, (unsigned long long*)info.p);
+        const long nws = hg::SorWorkspace(nx, ny);
+        sor_ws.reset(new DevBuf(size_t(nws)));
+        hg::LaunchSor(st, nx, ny, rows, dk.p, dx.p, opts->tolerance, opts->max_iters,
+                      opts->relaxation_factor, (unsigned long long*)info.p, sor_ws->p, nws);
         unsigned long long h[2];
         HG_CHECK(hipMemcpyAsync(h, info.p, 16, hipMemcpyDeviceToHost, st));
         HG_CHECK(hipStreamSynchronize(st));
