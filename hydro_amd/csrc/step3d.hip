@@ -435,13 +435,24 @@ __global__ void KMomentumRows(G g, FaceExpr e, MomCell m, int write_coefs, Rows 
     for (int q = 0; q < 7; ++q) A.t[q][c] = (q == 3) ? cen / m.relax : (Has(g, c, q) ? row[q] : 0.);
 }
 
-// ---- Jacobi (linear.hpp:750-783): one sweep x -> xn with the max |corr|
-// folded into diff[s] (non-negative doubles order as their bit patterns).
+// ---- Jacobi (linear.hpp:750-783): one sweep x -> xn with its max |corr|.
+// A sweep's maximum is kept in kJacSlots parts: a block folds its cells' and
+// adds one atomic maximum to part blockIdx % kJacSlots (non-negative doubles
+// order as their bit patterns).  One atomic per wave on a single address
+// serialised: 16.1 us per sweep at 48 x 40 x 36, of which the sweep itself is
+// about 3.  Sweep s uses row s % 4 of the parts; it reads the row of s - 1 and
+// clears that of s + 1, which s - 3 used.
+constexpr int kJacSlots = 64, kJacRows = 4;
+__device__ __forceinline__ unsigned long long* JacRow(unsigned long long* diff, int s) {
+  return diff + (s & (kJacRows - 1)) * kJacSlots;
+}
 // The stop rule after sweep s (state = {done, iters, buffer holding the
-// result}): converged (iters = s) or over the limit (iters = s + 1).
-__device__ __forceinline__ bool JacobiStop(const unsigned long long* diff, int s, double tol,
-                                           int limit, int& iters) {
-  const double d = __longlong_as_double((long long)diff[s]);
+// result}): converged (iters = s) or over the limit (iters = s + 1).  Every
+// wave folds the parts itself.
+__device__ __forceinline__ bool JacobiStop(unsigned long long* diff, int s, double tol, int limit,
+                                           int& iters) {
+  double d = __longlong_as_double((long long)JacRow(diff, s)[threadIdx.x & 63]);
+  for (int o = 32; o > 0; o >>= 1) d = fmax(d, __shfl_xor(d, o, 64));
   if (!(d > tol)) {
     iters = s;
     return true;
@@ -452,12 +463,27 @@ __device__ __forceinline__ bool JacobiStop(const unsigned long long* diff, int s
   }
   return false;
 }
+__device__ __forceinline__ void JacobiPut(double m, unsigned long long* row) {
+  __shared__ double red[kB / 64];
+  for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o, 64));
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < kB / 64; ++w) m = fmax(m, red[w]);
+    if (m > 0.)
+      atomicMax(&row[blockIdx.x % kJacSlots], (unsigned long long)__double_as_longlong(m));
+  }
+}
+__device__ __forceinline__ void JacobiClearNext(unsigned long long* diff, int s) {
+  if (blockIdx.x == 0 && threadIdx.x < kJacSlots) JacRow(diff, s + 1)[threadIdx.x] = 0ull;
+}
 // Sweep s first applies the stop rule of sweep s - 1 (complete: its kernel
 // has finished), so no separate check runs between sweeps: every block
-// takes the same decision from diff[s - 1], and block 0 records it.
-__global__ void KJacobiSweep(G g, Rows A, const double* __restrict__ k, const double* __restrict__ x,
-                             double* __restrict__ xn, double omega, unsigned long long* diff,
-                             int s, int* state, double tol, int limit) {
+// takes the same decision from that sweep's parts, and block 0 records it.
+__global__ void __launch_bounds__(kB)
+KJacobiSweep(G g, Rows A, const double* __restrict__ k, const double* __restrict__ x,
+             double* __restrict__ xn, double omega, unsigned long long* diff, int s, int* state,
+             double tol, int limit) {
   if (state[0]) return;  // decided after sweep s - 2 or earlier
   int iters = 0;
   if (s > 0 && JacobiStop(diff, s - 1, tol, limit, iters)) {
@@ -468,6 +494,7 @@ __global__ void KJacobiSweep(G g, Rows A, const double* __restrict__ k, const do
     }
     return;
   }
+  JacobiClearNext(diff, s);
   const long c = blockIdx.x * long(blockDim.x) + threadIdx.x;
   double m = 0.;
   if (c < g.nc) {
@@ -479,16 +506,13 @@ __global__ void KJacobiSweep(G g, Rows A, const double* __restrict__ k, const do
     m = fabs(corr);
     xn[c] = x[c] + corr * omega;
   }
-  for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o, 64));
-  if ((threadIdx.x & 63) == 0 && m > 0.)
-    atomicMax(&diff[s], (unsigned long long)__double_as_longlong(m));
+  JacobiPut(m, JacRow(diff, s));
 }
-// the stop rule after the last sweep s of a batch
-__global__ void KJacobiCheck(const unsigned long long* diff, int s, double tol, int limit,
-                             int* state) {
+// the stop rule after the last sweep s of a batch (one wave)
+__global__ void KJacobiCheck(unsigned long long* diff, int s, double tol, int limit, int* state) {
   if (state[0]) return;
   int iters = 0;
-  if (JacobiStop(diff, s, tol, limit, iters)) {
+  if (JacobiStop(diff, s, tol, limit, iters) && threadIdx.x == 0) {
     state[0] = 1;
     state[1] = iters;
     state[2] = (s + 1) & 1;  // sweep s wrote buffer (s + 1) & 1
@@ -499,21 +523,24 @@ __global__ void KJacobiCheck(const unsigned long long* diff, int s, double tol, 
 // sides, each from zero with its own stop rule) in one kernel per sweep:
 // the seven row entries of a cell are loaded once for the components still
 // running, and each component's update is the single-component sweep's,
-// operation for operation.  Component d keeps its max |corr| in
-// diff[d * stride + s] and its state (done, iters, buffer) at state[4 d].
+// operation for operation.  Component d keeps its parts of max |corr| in
+// diff[d * kJacRows * kJacSlots ..] and its state (done, iters, buffer) at
+// state[4 d].
 struct Jac3 {
   const double* k[3];
   const double* x[3];  // sweep s's input iterate, per component
   double* xn[3];       // its output
 };
-__global__ void KJacobiSweep3(G g, Rows A, Jac3 J, double omega, unsigned long long* diff,
-                              int stride, int s, int* state, double tol, int limit) {
+__global__ void __launch_bounds__(kB)
+KJacobiSweep3(G g, Rows A, Jac3 J, double omega, unsigned long long* diff, int s, int* state,
+              double tol, int limit) {
   bool act[3];
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
     act[d] = !state[4 * d];  // decided after sweep s - 2 or earlier: off
     int iters = 0;
-    if (act[d] && s > 0 && JacobiStop(diff + long(d) * stride, s - 1, tol, limit, iters)) {
+    unsigned long long* row = diff + d * kJacRows * kJacSlots;
+    if (act[d] && s > 0 && JacobiStop(row, s - 1, tol, limit, iters)) {
       if (blockIdx.x == 0 && threadIdx.x == 0) {
         state[4 * d] = 1;
         state[4 * d + 1] = iters;
@@ -521,6 +548,7 @@ __global__ void KJacobiSweep3(G g, Rows A, Jac3 J, double omega, unsigned long l
       }
       act[d] = false;
     }
+    if (act[d]) JacobiClearNext(row, s);
   }
   if (!act[0] && !act[1] && !act[2]) return;  // uniform over the grid
   const long c = blockIdx.x * long(blockDim.x) + threadIdx.x;
@@ -550,22 +578,21 @@ __global__ void KJacobiSweep3(G g, Rows A, Jac3 J, double omega, unsigned long l
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
     if (!act[d]) continue;
-    double v = m[d];
-    for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
-    if ((threadIdx.x & 63) == 0 && v > 0.)
-      atomicMax(&diff[long(d) * stride + s], (unsigned long long)__double_as_longlong(v));
+    JacobiPut(m[d], JacRow(diff + d * kJacRows * kJacSlots, s));
+    __syncthreads();  // its LDS is used again
   }
 }
-// the stop rule after the last sweep s of a batch, for each component
-__global__ void KJacobiCheck3(const unsigned long long* diff, int stride, int s, double tol,
-                              int limit, int* state) {
-  const int d = threadIdx.x;
-  if (d >= 3 || state[4 * d]) return;
-  int iters = 0;
-  if (JacobiStop(diff + long(d) * stride, s, tol, limit, iters)) {
-    state[4 * d] = 1;
-    state[4 * d + 1] = iters;
-    state[4 * d + 2] = (s + 1) & 1;  // sweep s wrote buffer (s + 1) & 1
+// the stop rule after the last sweep s of a batch, for each component (one
+// wave)
+__global__ void KJacobiCheck3(unsigned long long* diff, int s, double tol, int limit, int* state) {
+  for (int d = 0; d < 3; ++d) {
+    if (state[4 * d]) continue;
+    int iters = 0;
+    if (JacobiStop(diff + d * kJacRows * kJacSlots, s, tol, limit, iters) && threadIdx.x == 0) {
+      state[4 * d] = 1;
+      state[4 * d + 1] = iters;
+      state[4 * d + 2] = (s + 1) & 1;  // sweep s wrote buffer (s + 1) & 1
+    }
   }
 }
 
@@ -987,7 +1014,6 @@ struct hg3_ctx {
   double *cb, *cr, *cz, *cp, *cq, *cx;
   CgScal* cs;
   CgScal* cs_h;
-  int jlimit = 0;
   bool p_converged = true;  // the last pressure solve met its tolerance (cg, fcg_mg)
   int fluid_iter = 0, cd_iter = 0;
   double last_ind = 1.;
@@ -1236,7 +1262,7 @@ int SolveJacobi(hg3_ctx* c, const Rows& R, const double* k, double* x) {
   const hg_config& cfg = c->cfg;
   const int limit = cfg.lu_relaxed_num_iters_limit;
   const double tol = cfg.lu_relaxed_tolerance, omega = cfg.lu_relaxed_relaxation_factor;
-  H3_CHECK(hipMemsetAsync(c->jdiff, 0, size_t(limit + 2) * 8, c->st));
+  H3_CHECK(hipMemsetAsync(c->jdiff, 0, size_t(kJacSlots) * 8, c->st));
   H3_CHECK(hipMemsetAsync(c->jstate, 0, 4 * sizeof(int), c->st));
   H3_CHECK(hipMemsetAsync(c->corr, 0, size_t(c->nc) * 8, c->st));
   double* buf[2] = {c->corr, c->corr2};
@@ -1246,7 +1272,7 @@ int SolveJacobi(hg3_ctx* c, const Rows& R, const double* k, double* x) {
     for (int b = 0; b < batch; ++b, ++s)
       KJacobiSweep<<<Grid(c->nc), kB, 0, c->st>>>(c->g, R, k, buf[s & 1], buf[(s + 1) & 1], omega,
                                                    c->jdiff, s, c->jstate, tol, limit);
-    KJacobiCheck<<<1, 1, 0, c->st>>>(c->jdiff, s - 1, tol, limit, c->jstate);
+    KJacobiCheck<<<1, 64, 0, c->st>>>(c->jdiff, s - 1, tol, limit, c->jstate);
     H3_CHECK(hipMemcpyAsync(c->state_h, c->jstate, 4 * sizeof(int), hipMemcpyDeviceToHost, c->st));
     c->Sync();
     if (c->state_h[0]) break;
@@ -1263,8 +1289,7 @@ void SolveVelocityJacobi3(hg3_ctx* c, const Rows& R, int iters[3]) {
   const hg_config& cfg = c->cfg;
   const int limit = cfg.lu_relaxed_num_iters_limit;
   const double tol = cfg.lu_relaxed_tolerance, omega = cfg.lu_relaxed_relaxation_factor;
-  const int stride = limit + 2;
-  H3_CHECK(hipMemsetAsync(c->jdiff, 0, size_t(3) * stride * 8, c->st));
+  H3_CHECK(hipMemsetAsync(c->jdiff, 0, size_t(3) * kJacRows * kJacSlots * 8, c->st));
   H3_CHECK(hipMemsetAsync(c->jstate, 0, 12 * sizeof(int), c->st));
   for (int d = 0; d < 3; ++d)
     H3_CHECK(hipMemsetAsync(c->jbuf[d][0], 0, size_t(c->nc) * 8, c->st));
@@ -1278,10 +1303,10 @@ void SolveVelocityJacobi3(hg3_ctx* c, const Rows& R, int iters[3]) {
         J.x[d] = c->jbuf[d][s & 1];
         J.xn[d] = c->jbuf[d][(s + 1) & 1];
       }
-      KJacobiSweep3<<<Grid(c->nc), kB, 0, c->st>>>(c->g, R, J, omega, c->jdiff, stride, s,
-                                                    c->jstate, tol, limit);
+      KJacobiSweep3<<<Grid(c->nc), kB, 0, c->st>>>(c->g, R, J, omega, c->jdiff, s, c->jstate, tol,
+                                                    limit);
     }
-    KJacobiCheck3<<<1, 64, 0, c->st>>>(c->jdiff, stride, s - 1, tol, limit, c->jstate);
+    KJacobiCheck3<<<1, 64, 0, c->st>>>(c->jdiff, s - 1, tol, limit, c->jstate);
     H3_CHECK(hipMemcpyAsync(c->state_h, c->jstate, 12 * sizeof(int), hipMemcpyDeviceToHost, c->st));
     c->Sync();
     if (c->state_h[0] && c->state_h[4] && c->state_h[8]) break;
@@ -1653,9 +1678,8 @@ hg_status hg3_create(const hg3_config* cfg3, hg3_ctx** out) {
     c->cq = c->Alloc(nc);
     c->cx = c->Alloc(nc);
     c->cs = (CgScal*)c->Alloc(long(sizeof(CgScal) / 8 + 1));
-    c->jlimit = std::max(1, cfg.lu_relaxed_num_iters_limit);
-    // three components' max |corr| per sweep and states (done, iters, buffer)
-    c->jdiff = (unsigned long long*)c->Alloc(3L * (c->jlimit + 2));
+    // three components' parts of max |corr| and states (done, iters, buffer)
+    c->jdiff = (unsigned long long*)c->Alloc(3L * kJacRows * kJacSlots);
     c->jstate = (int*)c->Alloc(6);
     if (cfg.linear_solver_velocity == HG_SOLVER_JACOBI)
       for (int d = 0; d < 3; ++d)
