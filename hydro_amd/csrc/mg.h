@@ -1,9 +1,10 @@
 // mg.h -- FP32 cell-centred multigrid V-cycle for the pressure operator.
 //
 // Face-form operator (A p)_c = sum_f k_f (p_c - p_nb).  Coarse levels halve
-// both dimensions while they stay even: coarse face coefficient = mean of
-// the two fine faces it covers (rediscretisation; in 2D k_f = A/(d a_f) does
-// not scale with h), restriction = sum of the four children's residuals,
+// both dimensions (the last cell of an odd side stays alone): coarse face
+// coefficient = mean of the two fine faces it covers (rediscretisation; in 2D
+// k_f = A/(d a_f) does not scale with h; the last faces by their own lengths
+// and distances), restriction = sum of the four children's residuals,
 // prolongation = cell-centred bilinear weighted by the coarse face
 // coefficients (injection across walls and strong density jumps), smoother =
 // Chebyshev-damped Jacobi sweeps before and after the coarse correction (two
@@ -29,6 +30,7 @@ constexpr int kMidY = 4;    // tile height of the coarser levels' fused kernels
 template <class M>
 struct MgLevelT {
   int nx, ny;
+  M lx, ly;       // distance ratio of the last inner face to the finer level's, in x and y
   TileGrid tg;    // 64 x 4 tiles
   TileGrid mid;   // 64 x kMidY tiles
   TileGrid tall;  // 64 x kTallY tiles

@@ -18,8 +18,8 @@ namespace hg {
 
 namespace {
 
-constexpr int kCoarsestMax = 1024;
-constexpr int kTinyMax = 64;          // coarsest grid solved by one wave
+constexpr int kTinyMax = 64;          // coarsest grid, solved by one wave
+constexpr int kCoarsestMax = kTinyMax;
 constexpr int kInKernelMax = 2048;    // levels handled by the one-workgroup cycle
 // Jacobi-PCG iterations on the coarsest grid: a partial solve.  The V-cycle
 // is applied inside flexible CG, which tolerates the inexact coarse solve;
@@ -48,19 +48,28 @@ __device__ __forceinline__ M Ax(int nx, int ny, const M* __restrict__ kx,
 }
 
 // Coarse cell (I, J) of a level: its west and south face coefficients (and
-// the east / north one on the last column / row), each the mean of the two
-// fine faces it covers, and its inverse diagonal.
+// the east / north one on the last column / row), each the sum of the fine
+// faces it covers (two, or one in a last row or column of its own) times
+// the ratio of the distances between the cells either side, fine over coarse
+// (1/2; lx / ly at the last inner face, CoarseRatio), and its inverse
+// diagonal.
 template <class M>
-__device__ __forceinline__ void CoarsenCell(int nxf, const M* __restrict__ kxf,
-                                            const M* __restrict__ kyf, int nxc, int nyc,
-                                            M* __restrict__ kxc, M* __restrict__ kyc,
+__device__ __forceinline__ void CoarsenCell(int nxf, int nyf, const M* __restrict__ kxf,
+                                            const M* __restrict__ kyf, int nxc, int nyc, M lx,
+                                            M ly, M* __restrict__ kxc, M* __restrict__ kyc,
                                             M* __restrict__ dinvc, int I, int J) {
-  auto fx = [&](int i, int j) { return kxf[i + (nxf + 1) * j]; };
-  auto fy = [&](int i, int j) { return kyf[i + nxf * j]; };
-  const M kw = 0.5f * (fx(2 * I, 2 * J) + fx(2 * I, 2 * J + 1));
-  const M ke = 0.5f * (fx(2 * I + 2, 2 * J) + fx(2 * I + 2, 2 * J + 1));
-  const M ks = 0.5f * (fy(2 * I, 2 * J) + fy(2 * I + 1, 2 * J));
-  const M kn = 0.5f * (fy(2 * I, 2 * J + 2) + fy(2 * I + 1, 2 * J + 2));
+  const bool two_i = 2 * I + 1 < nxf, two_j = 2 * J + 1 < nyf;
+  auto fx = [&](int i) {
+    return kxf[i + (nxf + 1) * (2 * J)] + (two_j ? kxf[i + (nxf + 1) * (2 * J + 1)] : M(0));
+  };
+  auto fy = [&](int j) {
+    return kyf[2 * I + nxf * j] + (two_i ? kyf[2 * I + 1 + nxf * j] : M(0));
+  };
+  const M half = 0.5f;
+  const M kw = (I == nxc - 1 ? lx : half) * fx(2 * I);
+  const M ke = (I == nxc - 2 ? lx : half) * fx(min(2 * I + 2, nxf));
+  const M ks = (J == nyc - 1 ? ly : half) * fy(2 * J);
+  const M kn = (J == nyc - 2 ? ly : half) * fy(min(2 * J + 2, nyf));
   kxc[I + (nxc + 1) * J] = kw;
   kyc[I + nxc * J] = ks;
   if (I == nxc - 1) kxc[I + 1 + (nxc + 1) * J] = ke;
@@ -71,12 +80,13 @@ __device__ __forceinline__ void CoarsenCell(int nxf, const M* __restrict__ kxf,
 
 template <class M>
 __global__ void __launch_bounds__(256)
-KCoarsen(int nxf, const M* __restrict__ kxf, const M* __restrict__ kyf, int nxc,
-         int nyc, M* __restrict__ kxc, M* __restrict__ kyc, M* __restrict__ dinvc) {
+KCoarsen(int nxf, int nyf, const M* __restrict__ kxf, const M* __restrict__ kyf, int nxc,
+         int nyc, M lx, M ly, M* __restrict__ kxc, M* __restrict__ kyc, M* __restrict__ dinvc) {
   const long n = long(nxc) * nyc;
   for (long c = blockIdx.x * long(blockDim.x) + threadIdx.x; c < n;
        c += long(gridDim.x) * blockDim.x)
-    CoarsenCell(nxf, kxf, kyf, nxc, nyc, kxc, kyc, dinvc, int(c % nxc), int(c / nxc));
+    CoarsenCell(nxf, nyf, kxf, kyf, nxc, nyc, lx, ly, kxc, kyc, dinvc, int(c % nxc),
+                int(c / nxc));
 }
 
 // Levels 0..count-1 of a chain of small grids: level k (>= 1) coarsened from
@@ -86,6 +96,7 @@ template <class M>
 struct ChainSet {
   int count;
   int nx[kMaxChain], ny[kMaxChain];
+  M lx[kMaxChain], ly[kMaxChain];
   M *kx[kMaxChain], *ky[kMaxChain], *dinv[kMaxChain];
 };
 
@@ -95,8 +106,8 @@ KCoarsenChain(ChainSet<M> cs) {
   for (int k = 1; k < cs.count; ++k) {
     const int nxc = cs.nx[k], nyc = cs.ny[k];
     for (int c = threadIdx.x; c < nxc * nyc; c += blockDim.x)
-      CoarsenCell(cs.nx[k - 1], cs.kx[k - 1], cs.ky[k - 1], nxc, nyc, cs.kx[k], cs.ky[k],
-                  cs.dinv[k], c % nxc, c / nxc);
+      CoarsenCell(cs.nx[k - 1], cs.ny[k - 1], cs.kx[k - 1], cs.ky[k - 1], nxc, nyc, cs.lx[k],
+                  cs.ly[k], cs.kx[k], cs.ky[k], cs.dinv[k], c % nxc, c / nxc);
     __threadfence_block();
     __syncthreads();
   }
@@ -463,7 +474,10 @@ KUp(int nx, int ny, TileGrid tg, const M* __restrict__ kx, const M* __restrict__
       M corr = ec;
       if (BILINEAR) {
         const int sx = c.i & 1, sy_ = c.j & 1;
-        const M wx = sw[sx ? 1 : 0][pj][pi], wy = sw[sy_ ? 3 : 2][pj][pi];
+        // (a last cell that is its parent's only child in x or y lies at the
+        // parent's centre in that direction)
+        const M wx = (!sx && c.i == nx - 1) ? M(0) : sw[sx ? 1 : 0][pj][pi];
+        const M wy = (!sy_ && c.j == ny - 1) ? M(0) : sw[sy_ ? 3 : 2][pj][pi];
         const int xi = pi + (sx ? 1 : -1), yj = pj + (sy_ ? 1 : -1);
         corr = Bilinear(ec, se[pj][xi], se[yj][pi], se[yj][xi], wx, wy);
       }
@@ -637,8 +651,10 @@ KCoarseCycle(CoarseSetT<M> cs, SweepWeights w, const int* done) {
         const M cs_ = cs.ky[l + 1][I + nxc * J], cn = cs.ky[l + 1][I + nxc * (J + 1)];
         const M kmax = fmax(fmax(cw, ce), fmax(cs_, cn));
         if (kmax > 0.f) {
-          wx[l][m] = fmin(1.f, 4.f * ((i & 1) ? ce : cw) / kmax);
-          wy[l][m] = fmin(1.f, 4.f * ((j & 1) ? cn : cs_) / kmax);
+          // (zero too where the cell is its parent's only child, see KUp)
+          const bool onex = !(i & 1) && i == nx - 1, oney = !(j & 1) && j == cs.ny[l] - 1;
+          wx[l][m] = onex ? M(0) : fmin(1.f, 4.f * ((i & 1) ? ce : cw) / kmax);
+          wy[l][m] = oney ? M(0) : fmin(1.f, 4.f * ((j & 1) ? cn : cs_) / kmax);
         }
       }
     }
@@ -715,7 +731,10 @@ KCoarseCycle(CoarseSetT<M> cs, SweepWeights w, const int* done) {
       const int I = C % nxc, J = C / nxc;
       M sum = 0.f;
 #pragma unroll
-      for (int q = 0; q < 4; ++q) sum += xa[2 * I + (q & 1) + nx * (2 * J + (q >> 1))];
+      for (int q = 0; q < 4; ++q) {
+        const int i = 2 * I + (q & 1), j = 2 * J + (q >> 1);
+        sum += (i < nx && j < ny) ? xa[i + nx * j] : M(0);
+      }
       rc[C] = sum;
     }
     __syncthreads();
@@ -808,13 +827,35 @@ inline int Blocks1D(long n) { return int(std::min<long>((n + 255) / 256, 4096));
 
 }  // namespace
 
+// Ratio of the distance between the last two cells of a line of `nf` to that
+// between the last two of its coarse line, where the last fine cell is `rho`
+// times as long as the others; rho becomes the coarse line's.  An even line's
+// last coarse cell is a pair, an odd one's the last fine cell alone.
+static double CoarseRatio(int nf, double& rho) {
+  if (nf % 2 == 0) {
+    const double r = 2. / (3. + rho);
+    rho = 0.5 * (1. + rho);
+    return r;
+  }
+  const double r = (1. + rho) / (2. + rho);
+  rho = 0.5 * rho;
+  return r;
+}
+
 template <class M>
 MgPrecondT<M>::MgPrecondT(int nx, int ny, M* kx0, M* ky0, M* dinv0) {
+  // the FP64 levels are a comparison on grids with even sides
+  if (std::is_same<M, double>::value &&
+      ((nx & 1) || (ny & 1) || long(nx) * ny <= kTinyMax || nx < 4 || ny < 4))
+    throw std::runtime_error("MgPrecond64: a grid with an odd or tiny side is not supported");
   int cx = nx, cy = ny;
+  double rx = 1., ry = 1., lx = 0.5, ly = 0.5;
   while (true) {
     MgLevelT<M> L;
     L.nx = cx;
     L.ny = cy;
+    L.lx = M(lx);
+    L.ly = M(ly);
     L.tg = MakeTileGrid(cx, cy);
     L.mid = MakeTileGrid(cx, cy, kMidY);
     L.tall = MakeTileGrid(cx, cy, kTallY);
@@ -832,32 +873,32 @@ MgPrecondT<M>::MgPrecondT(int nx, int ny, M* kx0, M* ky0, M* dinv0) {
     HG_CHECK(hipMalloc(&L.xa, n * sizeof(M)));
     HG_CHECK(hipMalloc(&L.xb, n * sizeof(M)));
     lv_.push_back(L);
-    if ((cx & 1) || (cy & 1) || n <= kTinyMax || cx < 4 || cy < 4) break;
-    cx /= 2;
-    cy /= 2;
+    // every grid halves (an odd side's last cell stays alone) down to at most
+    // kTinyMax cells.  A hierarchy that stopped at the first odd side relaxed
+    // that level instead: 300 x 180 (which halves twice) took 176 FCG
+    // iterations per solve, 300 x 181 about 700.
+    if (n <= kTinyMax) break;
+    lx = CoarseRatio(cx, rx);
+    ly = CoarseRatio(cy, ry);
+    cx = (cx + 1) / 2;
+    cy = (cy + 1) / 2;
   }
   HG_CHECK(hipMalloc(&never_done_, sizeof(int)));
   HG_CHECK(hipMemset(never_done_, 0, sizeof(int)));
-  const long nlast = long(lv_.back().nx) * lv_.back().ny;
-  if (nlast > kCoarsestMax)
-    coarse_sweeps = -1;  // coarsest too large for one workgroup: relax with grid kernels
-  // levels 1.. of at most kInKernelMax cells go to the one-workgroup cycle
-  // when the hierarchy ends on a tiny grid
-  if (nlast <= kTinyMax && lv_.size() > 1) {
-    for (int l = 1; l < int(lv_.size()); ++l)
-      if (long(lv_[l].nx) * lv_[l].ny <= kInKernelMax) {
-        first_in_kernel_ = l;
-        break;
-      }
-  }
-  // (a chain from <= kInKernelMax cells down to <= kTinyMax has at most
-  // kCcLevels + 1 levels; anything else stays on the grid kernels)
-  if (first_in_kernel_ > 0 && int(lv_.size()) - first_in_kernel_ > kCcLevels + 1)
-    first_in_kernel_ = -1;
-  if (first_in_kernel_ > 0) {
+  // the levels from the first below the finest that the one-workgroup cycle
+  // has room for: at most kInKernelMax cells, kCcThreads on the next, a
+  // chain of at most kCcLevels + 1 levels within its LDS (lines of odd sides
+  // shrink by less than four per level)
+  for (int l = 1; l < int(lv_.size()); ++l) {
     long cells = 0;
-    for (int l = first_in_kernel_; l < int(lv_.size()); ++l) cells += long(lv_[l].nx) * lv_[l].ny;
-    if (cells > kLdsCells) first_in_kernel_ = -1;  // cannot happen: 2048 * 4/3 < kLdsCells
+    for (int m = l; m < int(lv_.size()); ++m) cells += long(lv_[m].nx) * lv_[m].ny;
+    const long n0 = long(lv_[l].nx) * lv_[l].ny;
+    const long n1 = cells - n0 > 0 ? long(lv_[l + 1].nx) * lv_[l + 1].ny : 0;
+    if (n0 <= kInKernelMax && n1 <= kCcThreads && cells <= kLdsCells &&
+        int(lv_.size()) - l <= kCcLevels + 1) {
+      first_in_kernel_ = l;
+      break;
+    }
   }
 }
 
@@ -884,8 +925,8 @@ void MgPrecondT<M>::Build(hipStream_t st) {
     MgLevelT<M>& F = lv_[l - 1];
     MgLevelT<M>& C = lv_[l];
     if (long(C.nx) * C.ny <= kChainCells && lv_.size() - (l - 1) <= size_t(kMaxChain)) break;
-    KCoarsen<M><<<Blocks1D(long(C.nx) * C.ny), 256, 0, st>>>(F.nx, F.kx, F.ky, C.nx, C.ny, C.kx,
-                                                          C.ky, C.dinv);
+    KCoarsen<M><<<Blocks1D(long(C.nx) * C.ny), 256, 0, st>>>(
+        F.nx, F.ny, F.kx, F.ky, C.nx, C.ny, C.lx, C.ly, C.kx, C.ky, C.dinv);
   }
   if (l < lv_.size()) {
     ChainSet<M> cs{};
@@ -894,6 +935,8 @@ void MgPrecondT<M>::Build(hipStream_t st) {
       MgLevelT<M>& L = lv_[l - 1 + k];
       cs.nx[k] = L.nx;
       cs.ny[k] = L.ny;
+      cs.lx[k] = L.lx;
+      cs.ly[k] = L.ly;
       cs.kx[k] = L.kx;
       cs.ky[k] = L.ky;
       cs.dinv[k] = L.dinv;
@@ -932,49 +975,30 @@ void MgPrecondT<M>::Cycle(int l, const double* r64, float* z, M* out, hipStream_
     return;
   }
   const bool coarsest = (l == int(lv_.size()) - 1);
-  const int blocks = L.tg.blocks();
-  if (coarsest && coarse_sweeps > 0) {
-    // r of the coarsest level is always FP32 (lv_.size() > 1 is guaranteed for
-    // fine grids; a single-level hierarchy relaxes the FP64 residual below)
-    if (l > 0) {
-      KCoarsest<M><<<1, kCoarsestMax, 0, st>>>(L.nx, L.ny, L.kx, L.ky, L.dinv, L.r, omega,
-                                                coarse_sweeps, out, done);
-      return;
-    }
+  if (coarsest && l > 0) {
+    // (a chain the one-workgroup cycle does not take: a long thin grid)
+    KCoarsest<M><<<1, kCoarsestMax, 0, st>>>(L.nx, L.ny, L.kx, L.ky, L.dinv, L.r, omega,
+                                              coarse_sweeps, out, done);
+    return;
   }
   if (coarsest) {
-    // the level's result goes to z (FP32) on a single-level hierarchy
-    M* target = out;
-    if (l == 0) {
-      if constexpr (std::is_same<M, float>::value)
-        target = z;
-      else
-        throw std::runtime_error("MgPrecond64: a single-level hierarchy is not supported");
-    }
-    if (l == 0)
+    // a single level (at most kTinyMax cells): eight Jacobi sweeps into z
+    // (FP32), ping-ponging between xa and xb
+    if constexpr (std::is_same<M, float>::value) {
+      const int blocks = L.tg.blocks();
       KSmoothFirst<double, M><<<blocks, kTileThreads, 0, st>>>(L.nx, L.ny, L.tg, r64, L.dinv,
                                                                omega, L.xa, done);
-    else
-      KSmoothFirst<M, M><<<blocks, kTileThreads, 0, st>>>(L.nx, L.ny, L.tg, L.r, L.dinv, omega,
-                                                          L.xa, done);
-    // no coarser level (odd or tiny grids): seven more Jacobi sweeps ending
-    // in the target, ping-ponging between xa and xb
-    M* cur = L.xa;
-    const int nsw = 7;
-    for (int s = 0; s < nsw; ++s) {
-      M* dst = (s == nsw - 1) ? target : (cur == L.xa ? L.xb : L.xa);
-      if (dst == cur) dst = (cur == L.xa) ? L.xb : L.xa;
-      if (l == 0)
+      M* cur = L.xa;
+      const int nsw = 7;
+      for (int s = 0; s < nsw; ++s) {
+        M* dst = (s == nsw - 1) ? z : (cur == L.xa ? L.xb : L.xa);
         KJacobi<double, M><<<blocks, kTileThreads, 0, st>>>(L.nx, L.ny, L.tg, L.kx, L.ky, L.dinv,
                                                             r64, cur, omega, dst, done);
-      else
-        KJacobi<M, M><<<blocks, kTileThreads, 0, st>>>(L.nx, L.ny, L.tg, L.kx, L.ky, L.dinv, L.r,
-                                                       cur, omega, dst, done);
-      cur = dst;
+        cur = dst;
+      }
+    } else {
+      throw std::runtime_error("MgPrecond64: a single-level hierarchy is not supported");
     }
-    if (cur != target)
-      HG_CHECK(hipMemcpyAsync(target, cur, size_t(L.nx) * L.ny * sizeof(M),
-                              hipMemcpyDeviceToDevice, st));
     return;
   }
   MgLevelT<M>& C = lv_[l + 1];

@@ -76,3 +76,26 @@ def test_fp64_vcycle_same_iterations(gpu, problem):
           f"{s64.iterations} it {s64.ms:.3f} ms", flush=True)
     assert s32.converged and s64.converged
     assert abs(s32.iterations - s64.iterations) <= 1
+
+
+# sides that are odd at the first, a middle or every halving, lines that
+# shrink to one cell, grids around the one-workgroup cycle's limits
+@pytest.mark.parametrize("nx,ny", [(8, 8), (9, 9), (2, 50), (3, 700), (45, 45), (46, 45), (64, 33),
+                                   (65, 32), (97, 150), (129, 130), (333, 217), (510, 509)])
+def test_multigrid_any_side(gpu, nx, ny):
+    """fcg_mg on grids of any sides: the true residual meets the tolerance,
+    in tens of iterations where the Jacobi-PCG takes hundreds."""
+    n = max(nx, ny)
+    kx, ky, _ = workloads.poisson_problem(n, seed=5)
+    kx = kx.reshape(n, n + 1)[:ny, :nx + 1].copy()
+    ky = ky.reshape(n + 1, n)[:ny + 1, :nx].copy()
+    kx[:, -1] = 0.0
+    ky[-1, :] = 0.0
+    rhs = np.random.default_rng(1).normal(size=nx * ny)
+    print(f"case: fcg_mg {nx}x{ny}", flush=True)
+    p, st = Poisson(nx, ny, kx.reshape(-1), ky.reshape(-1)).solve(rhs, solver="fcg_mg", tol=1e-8,
+                                                                 precision=1)
+    b = rhs - rhs.mean()
+    res = np.linalg.norm(b - apply(kx, ky, p, nx, ny)) / np.linalg.norm(b)
+    assert st.converged and res <= 1.05e-8
+    assert st.iterations <= 100
