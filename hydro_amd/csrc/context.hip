@@ -674,15 +674,18 @@ void SolveRowsIterative(hg_ctx* c, int32_t solver, hg::Rows rows, const double* 
     *iters = it;
     return;
   }
-  if (solver == HG_SOLVER_GAUSS_SEIDEL)
-    hg::LaunchSor(c->st, nx, ny, rows, k, x, tol, limit, omega, c->gs_info, c->sor_ws,
-                  c->sor_doubles);
-  else if (solver == HG_SOLVER_LU_RELAXED)
-    hg::LaunchLuRelaxed(c->st, nx, ny, rows, k, x, w.xa, w.xb, tol, limit, omega, c->gs_info);
-  else
-    throw HgError(HG_ERR_UNSUPPORTED, "not an iterative row solver");
-  HG_CHECK(hipMemcpyAsync(c->info_h, c->gs_info, 16, hipMemcpyDeviceToHost, c->st));
-  c->Sync();
+  for (bool retry : {false, true}) {
+    if (solver == HG_SOLVER_GAUSS_SEIDEL)
+      hg::LaunchSor(c->st, nx, ny, rows, k, x, tol, limit, omega, c->gs_info, c->sor_ws,
+                    c->sor_doubles, retry);
+    else if (solver == HG_SOLVER_LU_RELAXED)
+      hg::LaunchLuRelaxed(c->st, nx, ny, rows, k, x, w.xa, w.xb, tol, limit, omega, c->gs_info);
+    else
+      throw HgError(HG_ERR_UNSUPPORTED, "not an iterative row solver");
+    HG_CHECK(hipMemcpyAsync(c->info_h, c->gs_info, 16, hipMemcpyDeviceToHost, c->st));
+    c->Sync();
+    if (c->info_h[0] != hg::kSorRetry) break;
+  }
   *iters = int(c->info_h[0]);
   std::memcpy(diff, &c->info_h[1], 8);
 }

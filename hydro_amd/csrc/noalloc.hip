@@ -126,11 +126,22 @@ hg_status hg_stencil_solve_noalloc(int32_t nx, int32_t ny, const double* s, cons
       Zero(st, a0, long(N));
       hg::LaunchLuRb(st, nx, ny, rows, k, k, a1, a2, a0, a0, x, a3);
       break;
-    case HG_SOLVER_GAUSS_SEIDEL:
+    case HG_SOLVER_GAUSS_SEIDEL: {
       // the solver's workspace: what the scratch array holds behind the header
-      hg::LaunchSor(st, nx, ny, rows, k, x, opts->tolerance, limit, opts->relaxation_factor, info,
-                    a0, long((kScratchBytes - off_arr) / 8));
+      const long ws = long((kScratchBytes - off_arr) / 8);
+      unsigned long long h[2] = {0, 0};
+      for (bool retry : {false, true}) {
+        hg::LaunchSor(st, nx, ny, rows, k, x, opts->tolerance, limit, opts->relaxation_factor,
+                      info, a0, ws, retry);
+        if (!check(hipMemcpyAsync(h, info, 16, hipMemcpyDeviceToHost, st)) ||
+            !check(hipStreamSynchronize(st)))
+          return Fail(HG_ERR_HIP, "iteration info readback failed");
+        if (h[0] != hg::kSorRetry) break;
+      }
+      iters = int(h[0]);
+      std::memcpy(&diff, &h[1], 8);
       break;
+    }
     case HG_SOLVER_LU_RELAXED:
       hg::LaunchLuRelaxed(st, nx, ny, rows, k, x, a0, a1, opts->tolerance, limit,
                           opts->relaxation_factor, info);
@@ -165,7 +176,7 @@ hg_status hg_stencil_solve_noalloc(int32_t nx, int32_t ny, const double* s, cons
     default:
       break;
   }
-  if (solver == HG_SOLVER_GAUSS_SEIDEL || solver == HG_SOLVER_LU_RELAXED) {
+  if (solver == HG_SOLVER_LU_RELAXED) {
     unsigned long long h[2] = {0, 0};
     if (!check(hipMemcpyAsync(h, info, 16, hipMemcpyDeviceToHost, st)) ||
         !check(hipStreamSynchronize(st)))

@@ -101,11 +101,15 @@ hg_status hg_stencil_solve(int32_t nx, int32_t ny, const double* s, const double
       case HG_SOLVER_GAUSS_SEIDEL: {
         const long nws = hg::SorWorkspace(nx, ny);
         sor_ws.reset(new DevBuf(size_t(nws)));
-        hg::LaunchSor(st, nx, ny, rows, dk.p, dx.p, opts->tolerance, opts->max_iters,
-                      opts->relaxation_factor, (unsigned long long*)info.p, sor_ws->p, nws);
         unsigned long long h[2];
-        HG_CHECK(hipMemcpyAsync(h, info.p, 16, hipMemcpyDeviceToHost, st));
-        HG_CHECK(hipStreamSynchronize(st));
+        for (bool retry : {false, true}) {
+          hg::LaunchSor(st, nx, ny, rows, dk.p, dx.p, opts->tolerance, opts->max_iters,
+                        opts->relaxation_factor, (unsigned long long*)info.p, sor_ws->p, nws,
+                        retry);
+          HG_CHECK(hipMemcpyAsync(h, info.p, 16, hipMemcpyDeviceToHost, st));
+          HG_CHECK(hipStreamSynchronize(st));
+          if (h[0] != hg::kSorRetry) break;
+        }
         iters = int(h[0]);
         std::memcpy(&diff, &h[1], 8);
         break;

@@ -32,11 +32,14 @@
 // -ffp-contract=off.
 //
 // What bounds it: the instructions of a step (about 140 per thread for two
-// cells, 52 of them FP64), with 2 Q a <= 2048 cells per step on one CU.
-// Per sweep, against the sweep-at-a-time kernel (101 and 701 sweeps): 64 x 64
-// 3.6 against 34.6 us, 256 x 128 15.3 against 177 us, 333 x 217 43 against
-// 534 us, 37 x 900 27 against 274 us.  1024 threads beat 512 and 256 (256 x
-// 128: 15.3, 19.7, 30.9 us).
+// cells, 52 of them FP64), with 2 Q a <= 2048 cells per step on one CU; and
+// where the long side has room for several workgroups (KSorChain, below) the
+// b / (G P) steps of a sweep, plus once per solve the a + b to fill the
+// pipeline.  Per sweep, against the sweep-at-a-time kernel (101 sweeps unless
+// noted): 64x64 3.6 against 34.6 us; 256x128 at 701 sweeps 3.7 (one
+// workgroup 15.3) against 177 us; 333x217 13 (43) against 534 us.
+// For one workgroup 1024 threads beat 512 and 256 (256x128: 15.3, 19.7, 30.9
+// us); for each of several 512 (256x128: 3.7; 1024: 7.2, 256: 4.8 us).
 #include <algorithm>
 
 #include "kernels.h"
@@ -49,11 +52,31 @@ constexpr int kSorThreads = 1024;
 constexpr int kSorMaxQ = 32;
 constexpr int kSorHeader = 32;  // doubles before the arrays: [0] the result's ring slot
 
+// (several workgroups, below)
+constexpr int kLag = 20;
+constexpr int kSpin = 1 << 20;
+constexpr int kNever = 0x7fffffff;
+
+constexpr int kSorMaxG = 64, kSorMaxStages = 1024;
+constexpr long kChainMaxDoubles = 1L << 26;  // of the workspace
+// Workspace header, in doubles: the smallest sweep that ended the solve
+// (int `stop`), then a 64-byte line of progress per workgroup, then the max
+// |corr| of the sweep each stage last found to end it.
+constexpr int kChainProgress = 8, kChainRec = kChainProgress + 8 * kSorMaxG;
+constexpr int kChainHeader = kChainRec + kSorMaxStages;
+
+struct SorChain {
+  int a, b, ap;           // short and long side, line padded to waves
+  int Q, G, span, le;     // thread groups per workgroup, workgroups, log rows
+  int limit, tail;
+};
+
 struct SorPlan {
   bool ok = false;
   bool tr = false;   // threads along y (the short side), marching along x
   int a = 0, b = 0;  // short and long side
   int Q = 0, rounds = 0;
+  int G = 1, span = 0, le = 0;  // several workgroups (G > 1): see KSorChain
   long doubles = 0;
 };
 
@@ -82,6 +105,35 @@ SorPlan PlanSor(int nx, int ny, int limit, long max_doubles) {
   return p;
 }
 
+// The several-workgroup plan: 512 threads (1024 where a line needs them),
+// as many workgroups as keep kLag steps between them.  A log keeps what the
+// tail may read: a + b rows of a line, up to b + span steps after its end (a
+// workgroup is at most the sum of the lags, under b, ahead of another).
+SorPlan PlanChain(int nx, int ny, int limit, long max_doubles) {
+  SorPlan p;
+  p.tr = ny < nx;
+  p.a = std::min(nx, ny);
+  p.b = std::max(nx, ny);
+  const long n = long(nx) * ny;
+  const int ap = (p.a + 63) / 64 * 64;
+  if (ap > kSorThreads) return p;
+  p.Q = std::max(512 / ap, 1);
+  const int P = 2 * p.Q;
+  int g = std::min(std::min(p.b / (2 * P + kLag), kSorMaxG), kSorMaxStages / P);
+  g = std::min(g, limit / P + 1);
+  for (; g >= 2; --g) {
+    p.span = p.b / g;
+    p.le = p.a + 2 * p.b + p.span + 64;
+    p.doubles = kChainHeader + 7 * n + long(g) * p.le * p.a;
+    if (p.doubles <= std::min(max_doubles, kChainMaxDoubles)) {
+      p.G = g;
+      p.ok = true;
+      break;
+    }
+  }
+  return p;
+}
+
 // Barrier between steps.  It orders the LDS exchange and leaves the loads in
 // flight; of the global stores it waits for those of two steps before and
 // earlier (a step issues at most 3 + 2 loads and 2 stores per wave, vector
@@ -90,6 +142,13 @@ SorPlan PlanSor(int nx, int ny, int limit, long max_doubles) {
 // issued at the earliest.  The workgroup's waves share one L1.
 __device__ __forceinline__ void StepBarrier() {
   asm volatile("s_waitcnt vmcnt(10)" ::: "memory");
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+  asm volatile("" ::: "memory");
+}
+
+__device__ __forceinline__ void ChainBarrier() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
@@ -106,7 +165,11 @@ struct SorRow {
 // Rows into the skewed order, zero where the neighbour is outside the grid.
 __global__ void __launch_bounds__(256)
 KSorPack(int nx, int ny, Rows r, const double* __restrict__ k, int tr, double2* __restrict__ oc,
-         double2* __restrict__ xn, double2* __restrict__ ck) {
+         double2* __restrict__ xn, double2* __restrict__ ck, double* head) {
+  if (blockIdx.x == 0 && head) {  // no sweep has ended, no steps done
+    int* const h = reinterpret_cast<int*>(head);
+    for (int z = threadIdx.x; z < 2 * kChainRec; z += 256) h[z] = z == 0 ? kNever : 0;
+  }
   const int a = tr ? ny : nx, b = tr ? nx : ny;
   const int d = blockIdx.x * 256 + threadIdx.x;  // skewed index, so that stores coalesce
   if (d >= a * b) return;
@@ -133,7 +196,7 @@ KSorUnpack(int nx, int ny, int tr, const double* __restrict__ ring,
   const int i = c % nx, j = c / nx;
   const int t = tr ? j : i, m = tr ? i : j;
   const int row = t + m >= b ? t + m - b : t + m;
-  const long slot = reinterpret_cast<const long long*>(head)[0];
+  const long slot = head ? reinterpret_cast<const long long*>(head)[0] : 0;
   x[c] = ring[slot * nx * ny + long(row) * a + t];
 }
 
@@ -322,26 +385,366 @@ KSorPipe(int a, int b, int Q, int rounds, const double2* __restrict__ oc,
   }
 }
 
+// ---- several workgroups -----------------------------------------------------
+// The same pipeline over G workgroups: workgroup g runs stages g P .. g P +
+// P - 1 (its threads' lines padded to whole waves, so that q is uniform in a
+// wave), the last stage of one feeding the first of the next through memory,
+// and the last workgroup's the first's, a round (b steps) later.  All
+// workgroups count the same virtual steps: workgroup g's first stage starts
+// at step g span, where G span <= b, so a line is span - 2 P >= kLag steps
+// further on in the workgroup before than its reader needs.
+//
+// What a first stage reads was written kLag + 1 or more steps before, into the
+// writer's log (row = step mod le).  Steps go in groups of four.  At a
+// group's start the first stage's waves issue the loads for the next group;
+// at its end the workgroup publishes the steps before the group, whose stores
+// are complete (vmcnt) in every wave.  A reader so needs progress that was
+// published about 12 steps ago and normally does not wait; it polls when it
+// must, a bounded number of times, after which the solve is marked failed
+// (stop = -1) and every workgroup leaves; the caller then runs the
+// one-workgroup kernel.
+// Log and flags are written and read with agent-scope accesses: the
+// workgroups are on different XCDs, each with its own L2.
+//
+// A sweep's workgroup applies the stop rule and lowers `stop`; every
+// workgroup runs on to the virtual step by which all earlier sweeps were
+// decided too.  Only the lines between workgroups are kept, so the result is
+// found by a second launch (tail) of one workgroup, which repeats the sweeps
+// from the last logged one before the stop to the stop -- unless the solve
+// ran to its last sweep, which is written as it is computed.
+__device__ __forceinline__ double AgentLoad(const double* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ int AgentLoad(const int* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+template <bool TR, int MAXT>
+__global__ void __launch_bounds__(MAXT)
+KSorChain(SorChain ch, const double2* __restrict__ oc, const double2* __restrict__ xn,
+          const double2* __restrict__ ck, double* head, double* logs, double* out, double tol,
+          double omega, unsigned long long* __restrict__ info) {
+  extern __shared__ double2 lds2[];  // as KSorPipe's; maxima [stage][4 rounds]
+  __shared__ int lstop;
+  int* const stop = reinterpret_cast<int*>(head);
+  int* const progress = reinterpret_cast<int*>(head + kChainProgress);
+  unsigned long long* const rec = reinterpret_cast<unsigned long long*>(head + kChainRec);
+  const int a = ch.a, b = ch.b, Q = ch.Q, P = 2 * Q, W = a + 2, le = ch.le, span = ch.span;
+  const long log_n = long(le) * a;
+  int G = ch.G, wg = blockIdx.x, limit = ch.limit;
+  // where the first stage's input comes from: the log of workgroup `src`, the
+  // values for this workgroup's step T in row T + shift; the zero start where
+  // T - t < from
+  int src = wg == 0 ? G - 1 : wg - 1, start = wg * span;
+  int shift = wg == 0 ? (G - 1) * span + 2 * P - b - 1 : 2 * P - span - 1;
+  int from = wg == 0 ? b : -1;
+  if (ch.tail) {
+    const int s = *stop;
+    if (s < 0) {
+      if (threadIdx.x == 0) info[0] = ~0ull;
+      return;
+    }
+    const int st = s % (G * P);
+    if (threadIdx.x == 0) {
+      const unsigned long long bits = rec[st];
+      info[0] = (unsigned long long)(!(__longlong_as_double((long long)bits) > tol) ? s : s + 1);
+      info[1] = bits;
+    }
+    if (s == limit) return;  // already written
+    // sweeps s - p .. s again, p the stage within its workgroup, from the
+    // sweep before them: logged by the workgroup before (a round earlier for
+    // the first), or the zero start.  Its cell (t, m) is in log row src span
+    // + 2 (P - 1) + t + rs b + m, and is read as the next cell of m - 1 at
+    // step t + m - 1.
+    const int p = st % P, w = st / P, rd = s / (G * P);
+    const int rs = w == 0 ? rd - 1 : rd;
+    src = w == 0 ? G - 1 : w - 1;
+    shift = src * span + 2 * (P - 1) + rs * b + 1;
+    from = rs < 0 ? kNever : -1;
+    G = 1;
+    wg = 0;
+    start = 0;
+    limit = p;
+  }
+  const bool wait = !ch.tail;
+  // (there is nothing to wait for before a workgroup's start)
+  if (threadIdx.x == 0 && wait)
+    __hip_atomic_store(progress + 16 * wg, start, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const int tid = threadIdx.x;
+  double2* const val = lds2;
+  unsigned long long* const sd = reinterpret_cast<unsigned long long*>(lds2 + 2 * Q * W);
+  for (int z = tid; z < 2 * Q * W; z += blockDim.x) val[z] = double2{0., 0.};
+  for (int z = tid; z < 4 * P; z += blockDim.x) sd[z] = 0ull;
+  if (tid == 0) lstop = kNever;
+  __syncthreads();
+  const int q = __builtin_amdgcn_readfirstlane(tid / ch.ap);
+  const int t = tid - q * ch.ap;
+  const bool live = t < a, first = q == 0, last = q == Q - 1;
+  const int ptot = G * P;  // sweeps per round
+  // the step within the pipeline's round, and the cell's place: m == 0 when
+  // tm == ez (see KSorPipe for m == 1, 2, b - 1); rd the lane's round
+  int ez = t + 4 * q, rd = 0;
+  while (ez >= b) {
+    ez -= b;
+    --rd;
+  }
+  if (ez > 0) --rd;
+  int tm = 0;
+  // the round in which a stage of these runs the last sweep (-1: none does)
+  auto LimRound = [&](int stage) {
+    const int d = limit - (wg * P + stage);
+    return d >= 0 && d % ptot == 0 ? d / ptot : -1;
+  };
+  const int limA = LimRound(2 * q), limB = LimRound(2 * q + 1);
+  int row = ((-4 * q) % b + b) % b;  // skewed row of the first stage's cells
+  int pr1 = row >= 1 ? row - 1 : row - 1 + b, pr2 = row >= 2 ? row - 2 : row - 2 + b;
+  SorRow c[4];
+  const unsigned t16 = unsigned(live ? t : 0) * 16u;
+  auto Load = [&](SorRow& o, int r) {
+    const size_t base = size_t(unsigned(r)) * unsigned(a) * 16u;
+    o.oc = *reinterpret_cast<const double2*>(reinterpret_cast<const char*>(oc) + base + t16);
+    o.xn = *reinterpret_cast<const double2*>(reinterpret_cast<const char*>(xn) + base + t16);
+    o.ck = *reinterpret_cast<const double2*>(reinterpret_cast<const char*>(ck) + base + t16);
+  };
+  Load(c[0], row);
+  Load(c[3], pr1);
+  Load(c[2], pr2);
+  const double* const in = logs + src * log_n;
+  double* const mylog = logs + wg * log_n;
+  // first stage: its input for the group's four steps, and for the next
+  // group's (next cell of the line, line after's cell)
+  double2 cur[4], nxt[4];
+  auto Fetch = [&](double2 (&g)[4], int T) {
+    // rows below 0 are never used
+    int r = T + shift;
+    r = r < 0 ? 0 : r % le;
+    const int tc = live ? t : 0, tx = t < a - 1 ? tc + 1 : tc;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const double* const lr = in + long(r) * a;
+      g[i].x = AgentLoad(lr + tc);
+      g[i].y = AgentLoad(lr + tx);
+      if (++r == le) r = 0;
+    }
+  };
+  int seen = 0, ahead = 0, ahead_stop = kNever;
+  // the source's steps below `need` are complete, or the solve has ended
+  // (false: gave up)
+  auto Await = [&](int need) {
+    if (!wait) return true;
+    seen = max(seen, ahead);
+    for (int k = 0; seen < need; ++k) {
+      seen = AgentLoad(progress + 16 * src);
+      if (seen >= need) break;
+      if (AgentLoad(stop) != kNever) return true;
+      if (k == kSpin) {
+        __hip_atomic_fetch_min(stop, -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return false;
+      }
+    }
+    return true;
+  };
+  double ownA = 0., ownB = 0., oldA = 0., h1 = 0., h2 = 0., dA = 0., dB = 0.;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) cur[i] = nxt[i] = double2{0., 0.};
+  bool ok = true;
+  if (first) {
+    // step T uses row T + shift: for the steps start - 1 (the first cell's
+    // old value) .. start + 3
+    ok = Await(start + 4 + shift);
+    if (ok) {
+      Fetch(cur, start);
+      if (t == 0 && from < 0 && start - 1 + shift >= 0)
+        oldA = AgentLoad(in + long((start - 1 + shift) % le) * a);
+    }
+  }
+  double2* const mine = val + q * W + t;
+  auto Cell = [&](const SorRow& r, double own, double cross, double xold, double nold, double old,
+                  double& dmax) {
+    const double po = r.oc.x * own, pc = r.oc.y * cross;
+    const double px = r.xn.x * xold, pn = r.xn.y * nold;
+    double sum = po + pc;
+    sum += TR ? pn : px;
+    sum += TR ? px : pn;
+    const double value = -(r.ck.y + sum) / r.ck.x;
+    const double corr = value - old;
+    dmax = fmax(dmax, fabs(corr));
+    return old + corr * omega;
+  };
+  auto Decide = [&](int stage, int r) {
+    const int slot = 4 * stage + (r & 3), s = wg * P + stage + ptot * r;
+    const unsigned long long bits = sd[slot];
+    sd[slot] = 0ull;
+    const double diff = __longlong_as_double((long long)bits);
+    if (!ch.tail && s <= limit && (!(diff > tol) || s == limit)) {
+      if (s < __hip_atomic_fetch_min(stop, s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+        rec[s % ptot] = bits;
+    }
+  };
+  // virtual step by which sweep s is decided and every earlier one too
+  auto DoneStep = [&](int s) {
+    const int st = s % ptot;
+    return (st / P) * span + 2 * (st % P) + (s / ptot) * b + a + b;
+  };
+  const int end = DoneStep(limit) + 4;
+  int lrow = start % le, done_steps = start;
+  for (int T = start;; T += 4) {
+    // ---- the next group's input
+    if (first && ok) {
+      ok = Await(T + 8 + shift);
+      if (ok) Fetch(nxt, T + 4);
+      if (wait) {
+        ahead = AgentLoad(progress + 16 * src);
+        if (tid == 0) ahead_stop = AgentLoad(stop);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int nrow = row + 1 == b ? 0 : row + 1;
+      Load(c[(i + 1) & 3], nrow);
+      const int tm1 = tm + 1 == b ? 0 : tm + 1;
+      if (live) {
+        const SorRow &ca = c[i & 3], &cb = c[(i + 2) & 3];
+        const double2* const pv = mine + ((i & 1) ^ 1) * Q * W;
+        const double2 west = pv[0];
+        const double eastA = pv[2].x;
+        double nextA, crossA;
+        if (first) {
+          const int u = T + i - t;  // (from >= 0 only where start is 0)
+          nextA = u + 1 >= from ? cur[i].x : 0.;
+          crossA = (u >= from && t < a - 1) ? cur[i].y : 0.;
+        } else {
+          nextA = pv[1 - W].y;
+          crossA = pv[2 - W].y;
+        }
+        // the last line's ends: decide the sweeps that finished a step ago
+        if (t == a - 1 && rd > 0) {
+          if (tm == ez) Decide(2 * q, rd - 1);
+          if (tm == (ez + 2 >= b ? ez + 2 - b : ez + 2)) Decide(2 * q + 1, rd - 1);
+        }
+        const bool m0 = tm == ez, mend = tm1 == ez;
+        const int tb1 = tm >= 1 ? tm - 1 : tm - 1 + b, tb2 = tm >= 2 ? tm - 2 : tm - 2 + b;
+        const bool mb1 = tb1 == ez, mb2 = tb2 == ez;
+        const double xA = Cell(ca, m0 ? 0. : ownA, west.x, crossA, mend ? 0. : nextA, oldA, dA);
+        const double xB = Cell(cb, mb2 ? 0. : ownB, west.y, eastA, mb1 ? 0. : h1, h2, dB);
+        mine[(i & 1) * Q * W + 1] = double2{xA, xB};
+        if (last && wait) {  // (the tail reads the logs)
+          int r = lrow + i;
+          if (r >= le) r -= le;
+          __hip_atomic_store(mylog + long(r) * a + t, xB, __ATOMIC_RELAXED,
+                             __HIP_MEMORY_SCOPE_AGENT);
+        }
+        if (limA >= 0 && rd == limA) out[long(row) * a + t] = xA;
+        if (limB >= 0) {
+          const int rdB = (m0 || mb1) ? rd - 1 : rd;  // (m == 0, 1: still the round before)
+          if (rdB == limB) out[long(pr2) * a + t] = xB;
+        }
+        if (mend) {
+          if (rd >= 0)
+            atomicMax(&sd[8 * q + (rd & 3)], (unsigned long long)__double_as_longlong(dA));
+          dA = 0.;
+          ++rd;
+        }
+        if (mb1) {
+          if (rd > 0)
+            atomicMax(&sd[8 * q + 4 + ((rd - 1) & 3)],
+                      (unsigned long long)__double_as_longlong(dB));
+          dB = 0.;
+        }
+        oldA = nextA;
+        h2 = h1;
+        h1 = xA;
+        ownA = xA;
+        ownB = xB;
+      }
+      pr2 = pr1;
+      pr1 = row;
+      row = nrow;
+      tm = tm1;
+      if (i == 3) {
+        // a wave with the last stage issues 16 vector memory operations per
+        // group, of which at most 12 may be outstanding here: its log stores
+        // before this group are complete
+        asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
+        if (tid == 0) lstop = ok ? ahead_stop : -1;
+      }
+      ChainBarrier();
+    }
+    lrow += 4;
+    if (lrow >= le) lrow -= le;
+    done_steps = T + 4;
+    if (tid == 0 && wait)
+      __hip_atomic_store(progress + 16 * wg, T, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (first) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) cur[i] = nxt[i];
+    }
+    const int s = lstop;
+    const int stop_at = s == kNever ? end : s < 0 ? 0 : min(end, DoneStep(s) + 4);
+    ChainBarrier();  // lstop is not written again before every thread read it
+    if (T >= stop_at) break;
+  }
+  // what the last two groups wrote: the others need no more than this for the
+  // sweeps up to the stop (and see the stop if they want more)
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (tid == 0 && wait)
+    __hip_atomic_store(progress + 16 * wg, done_steps, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 }  // namespace
 
+// Several workgroups where they hold more sweeps than one does.  Measured per
+// sweep, one | several (stages held): 64x128 5.7 | 4.5 us (32 | 48), 64x256
+// 10.2 | 5.2 us (32 | 112), 256x128 at 700 sweeps 15.3 | 3.7 us (16 | 56),
+// 333x217 at 100 43.5 | 13.2 us (8 | 52); with fewer stages they lose: 32x128
+// 3.7 | 4.2 us (64 | 48), 16x256 4.0 | 5.2 us (128 | 112), as the lines are
+// padded to waves.
+static bool UseChain(const SorPlan& one, const SorPlan& many) {
+  return many.ok && (!one.ok || many.G * many.Q > one.Q);
+}
+
 long SorWorkspace(int nx, int ny) {
-  const SorPlan p = PlanSor(nx, ny, 1 << 30, 1L << 60);
-  return p.ok ? p.doubles : 0;
+  const SorPlan p = PlanSor(nx, ny, 1 << 30, 1L << 60), c = PlanChain(nx, ny, 1 << 30, 1L << 60);
+  return std::max(p.ok ? p.doubles : 0, c.ok ? c.doubles : 0);
 }
 
 void LaunchSor(hipStream_t st, int nx, int ny, Rows a, const double* k, double* x, double tol,
-               int limit, double omega, unsigned long long* info, double* ws, long ws_doubles) {
+               int limit, double omega, unsigned long long* info, double* ws, long ws_doubles,
+               bool retry) {
   const SorPlan p = PlanSor(nx, ny, limit, ws ? ws_doubles : 0);
-  if (!p.ok) {
+  const SorPlan c = PlanChain(nx, ny, limit, ws ? ws_doubles : 0);
+  const bool many = !retry && UseChain(p, c);
+  if (!p.ok && !many) {
     LaunchGsWavefront(st, nx, ny, a, k, x, tol, limit, omega, info);
     return;
   }
   const long n = long(nx) * ny;
-  double2* oc = reinterpret_cast<double2*>(ws + kSorHeader);
+  const int tr = p.tr ? 1 : 0;
+  double2* oc = reinterpret_cast<double2*>(ws + (many ? kChainHeader : kSorHeader));
   double2 *xn = oc + n, *ck = xn + n;
   double* ring = reinterpret_cast<double*>(ck + n);
   const unsigned grid = unsigned((n + 255) / 256);
-  KSorPack<<<grid, 256, 0, st>>>(nx, ny, a, k, p.tr ? 1 : 0, oc, xn, ck);
+  KSorPack<<<grid, 256, 0, st>>>(nx, ny, a, k, tr, oc, xn, ck, many ? ws : nullptr);
+  if (many) {
+    SorChain ch{c.a, c.b, (c.a + 63) / 64 * 64, c.Q, c.G, c.span, c.le, limit, 0};
+    const int threads = c.Q * ch.ap;
+    const size_t lds = size_t(2) * c.Q * (c.a + 2) * sizeof(double2) + size_t(8) * c.Q * 8;
+    double *out = ring, *logs = out + n;
+    for (int tail = 0; tail < 2; ++tail) {
+      ch.tail = tail;
+      const unsigned g = tail ? 1u : unsigned(c.G);
+      auto launch = [&](auto kernel) {
+        kernel<<<g, threads, lds, st>>>(ch, oc, xn, ck, ws, logs, out, tol, omega, info);
+      };
+      if (threads > 512)
+        launch(tr ? KSorChain<true, 1024> : KSorChain<false, 1024>);
+      else
+        launch(tr ? KSorChain<true, 512> : KSorChain<false, 512>);
+    }
+    KSorUnpack<<<grid, 256, 0, st>>>(nx, ny, tr, out, nullptr, x);
+    return;
+  }
   const int threads = (p.Q * p.a + 63) / 64 * 64;
   const size_t lds = size_t(2) * p.Q * (p.a + 2) * sizeof(double2) +
                      size_t(p.rounds) * 2 * p.Q * 8 + 16;
@@ -351,7 +754,7 @@ void LaunchSor(hipStream_t st, int nx, int ny, Rows a, const double* k, double* 
   else
     KSorPipe<false><<<1, threads, lds, st>>>(p.a, p.b, p.Q, p.rounds, oc, xn, ck, ring, tol,
                                              limit, omega, ws, info);
-  KSorUnpack<<<grid, 256, 0, st>>>(nx, ny, p.tr ? 1 : 0, ring, ws, x);
+  KSorUnpack<<<grid, 256, 0, st>>>(nx, ny, tr, ring, ws, x);
 }
 
 }  // namespace hg

@@ -26,7 +26,8 @@ def rows(nx, ny, seed):
 
 
 SIZES = [(1, 1), (3, 7), (1, 8), (8, 8), (9, 8), (2, 50), (16, 16), (31, 33), (64, 64), (65, 64),
-         (57, 64), (128, 20), (40, 333), (1024, 12), (9, 1030), (513, 600), (1030, 1027)]
+         (57, 64), (128, 20), (40, 333), (1024, 12), (9, 1030), (513, 600), (1030, 1027), (64, 256),
+         (256, 65), (217, 333), (30, 700)]
 
 
 @pytest.mark.parametrize("nx,ny", SIZES)
