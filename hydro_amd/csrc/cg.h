@@ -85,6 +85,7 @@ class CgSolver {
   float *e32_ = nullptr, *zprev32_ = nullptr;
   double* part_ = nullptr;   // block partials
   void* scal_ = nullptr;     // device scalars (CgScalars)
+  void* words_ = nullptr;    // exchange and z words of the one-launch Jacobi-PCG
   void* host_scal_ = nullptr;  // pinned mirror
   int blocks_;
   int last_fcg_iters_ = 5;  // iterations of the last flexible solve
@@ -99,6 +100,9 @@ class CgSolver {
   CgResult SolveFlexible(const double* b, double* x, double tol, int max_iters, bool project,
                          Precond* pc, bool warm);
   void Prepare(const double* b, double* x, bool project, bool warm);
+  template <class T>
+  bool WholePcg(const T* kx, const T* ky, const T* dinv, const T* r, T* x, T* xsave,
+                int max_iters);
   int JacobiPcg64(double* x, int max_iters);
   int InnerFp32(double tol_inner, int max_iters, Precond* pc, bool* pc_failed);
   double ResidualFp64(const double* b, const double* x, double* r);  // returns ||r||^2

@@ -3,7 +3,8 @@
 // New solvers (no reference counterpart), values of linear_solver_pressure:
 //   "cg"           Jacobi-preconditioned CG, FP64 throughout (the plain
 //                  FP64 path); with precision "mixed", FP32 inner CG under
-//                  FP64 iterative refinement.
+//                  FP64 iterative refinement.  Grids of up to 262144 cells
+//                  run a solve in one launch (KPcgWhole).
 //   "fcg_learned"  flexible CG (Notay's FCG(1)) with FP64 Krylov vectors,
 //                  residuals, dot products and updates, preconditioned by an
 //                  FP32 multigrid V-cycle plus, once trained, the learned
@@ -284,6 +285,299 @@ KPcgStart(Walk w, const T* __restrict__ r, const T* __restrict__ dinv, T* __rest
   });
   double v[2] = {srz, srr};
   PutPartials<2>(v, pt.upd[1]);
+}
+
+// ---- Jacobi-PCG of a small grid in one launch ---------------------------------
+// Up to 64 workgroups hold the whole solve: each a contiguous range of cells,
+// K per thread, with x, r, z and the operator in registers and p, on the range
+// and the rows before and after it, in LDS.  The iteration is KPcgSpmv's and
+// KPcgUpdate's; where those end a kernel, the workgroups exchange their partial
+// dots (Exchange), and with (r, z) the z of the rows around a range (Halo).
+//
+// It is bound by the two exchanges, each a round trip between XCDs behind two
+// sums over the workgroup, against two launches per iteration of which each
+// begins with a fold over all partials.  Time per iteration, FP64, before and
+// after: 64x64 10.0 and 3.0 us, 128x128 9.9 and 3.4, 255x255 10.2 and 4.6,
+// 255x511 11.5 and 6.0, 512x512 15.2 and 7.4.  z sent with the dots instead of
+// after them saves about 1 us of that, sums by lane shifts instead of shuffles
+// through LDS 1.5 us, 1024 threads instead of 512 0.4 us.
+//
+// 64 workgroups: a quarter of the CUs, since kernels of four queues may run at
+// once and every workgroup waits for the others of its kernel (and one wave
+// reads all their partials).  The waits are bounded: a solve that waited too
+// long leaves sc->done 0 and the start's x in xsave.
+constexpr int kWholeMaxWg = 64;
+constexpr int kWholeThreads = 1024;
+constexpr long kWholeMaxCells = 4L * kWholeThreads * kWholeMaxWg;
+constexpr int kWholeLds = 8000;  // doubles
+constexpr int kWholeSpin = 1 << 17;
+// exchange words [2 parities][4][64], the count of finished workgroups, the
+// tags used so far
+constexpr int kWholeDone = 2 * 4 * kWholeMaxWg, kWholeEpoch = kWholeDone + 1;
+constexpr int kWholeWords = kWholeEpoch + 1;
+
+// A value travels as one (T = float) or two words that each hold 32 bits of it
+// under the exchange's number `tag`, so that it needs no flag behind it.
+using Word = unsigned long long;
+__device__ __forceinline__ Word TagLoad(const Word* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void TagStore(Word* p, unsigned tag, unsigned v) {
+  __hip_atomic_store(p, Word(tag) << 32 | v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ double FromWords(Word lo, Word hi) {
+  return __hiloint2double(int(unsigned(hi)), int(unsigned(lo)));
+}
+
+// Sum over the lanes of each row of 16 in its last lane (R = 4 steps), over
+// the wave in lane 63 (R = 6), in a fixed order.
+template <int R>
+__device__ __forceinline__ double DppSum(double v) {
+  auto Step = [&](auto ctrl, auto rows) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), ctrl.value, rows.value, 0xf,
+                                               true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), ctrl.value, rows.value, 0xf,
+                                               true);
+    v += __hiloint2double(hi, lo);
+  };
+  using std::integral_constant;
+  Step(integral_constant<int, 0x111>{}, integral_constant<int, 0xf>{});  // row_shr:1
+  Step(integral_constant<int, 0x112>{}, integral_constant<int, 0xf>{});
+  Step(integral_constant<int, 0x114>{}, integral_constant<int, 0xf>{});
+  Step(integral_constant<int, 0x118>{}, integral_constant<int, 0xf>{});
+  if constexpr (R == 6) {
+    Step(integral_constant<int, 0x142>{}, integral_constant<int, 0xa>{});  // row_bcast:15
+    Step(integral_constant<int, 0x143>{}, integral_constant<int, 0xc>{});  // row_bcast:31
+  }
+  return v;
+}
+__device__ __forceinline__ double LaneOf(double v, int lane) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                          __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+
+// Sums v over all workgroups, in a fixed order; `extra` = post(sums), formed
+// in one wave.  Words of a parity are written again two exchanges later, when
+// every workgroup has read them.  `others` runs in the other waves while the
+// first waits for the sums.  False, in the whole workgroup: gave up.
+template <int NV, class Post, class Others>
+__device__ __forceinline__ bool Exchange(double (&v)[NV], double& extra, unsigned tag,
+                                         Word* words, int* gave_up, Post&& post,
+                                         Others&& others) {
+  constexpr int kWaves = kWholeThreads / 64;  // at most 16: one row of lanes
+  __shared__ double red[NV][kWaves];
+  __shared__ double tot[NV + 1];
+  const int lane = threadIdx.x & 63, W = gridDim.x;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+#pragma unroll
+  for (int q = 0; q < NV; ++q) {
+    const double s = DppSum<6>(v[q]);
+    if (lane == 63) red[q][wave] = s;
+  }
+  __syncthreads();
+  bool ok = true;
+  if (wave == 0) {
+#pragma unroll
+    for (int q = 0; q < NV; ++q)
+      v[q] = LaneOf(DppSum<4>(lane < kWaves ? red[q][lane] : 0.), 15);
+    if (W > 1) {
+      Word* const mine = words + (tag & 1) * 4 * kWholeMaxWg;
+      if (lane == 0) {
+#pragma unroll
+        for (int q = 0; q < NV; ++q) {
+          TagStore(mine + 2 * q * kWholeMaxWg + blockIdx.x, tag, unsigned(__double2loint(v[q])));
+          TagStore(mine + (2 * q + 1) * kWholeMaxWg + blockIdx.x, tag,
+                   unsigned(__double2hiint(v[q])));
+        }
+      }
+      Word g[2 * NV];
+      for (int n = 0;; ++n) {
+        bool all = true;
+#pragma unroll
+        for (int i = 0; i < 2 * NV; ++i) g[i] = TagLoad(mine + i * kWholeMaxWg + min(lane, W - 1));
+#pragma unroll
+        for (int i = 0; i < 2 * NV; ++i) all = all && unsigned(g[i] >> 32) == tag;
+        if (__all(all)) break;
+        if (n == kWholeSpin) {
+          ok = false;
+          break;
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < NV; ++q)
+        v[q] = LaneOf(DppSum<6>(lane < W ? FromWords(g[2 * q], g[2 * q + 1]) : 0.), 63);
+    }
+    const double e = post(v);
+    if (lane == 0) {
+#pragma unroll
+      for (int q = 0; q < NV; ++q) tot[q] = v[q];
+      tot[NV] = e;
+    }
+  } else {
+    ok = others();
+  }
+  if (!ok) *gave_up = 1;
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < NV; ++q) v[q] = tot[q];
+  extra = tot[NV];
+  return *gave_up == 0;
+}
+
+template <class T, int K>
+__global__ void __launch_bounds__(kWholeThreads)
+KPcgWhole(int nx, int ny, int C, const T* __restrict__ kx, const T* __restrict__ ky,
+          const T* __restrict__ dinv, const T* __restrict__ r0, T* __restrict__ x,
+          T* __restrict__ xsave, Word* zw, Word* words, CgScalars* sc) {
+  extern __shared__ double whole_lds[];
+  __shared__ int gave_up;
+  T* const ps = reinterpret_cast<T*>(whole_lds);  // p of the cells c0 - nx ..
+  T* const zs = ps + C + 2 * nx;                  // z of the rows before and after
+  constexpr int NT = kWholeThreads;
+  const int n = nx * ny, c0 = blockIdx.x * C, c1 = min(c0 + C, n);
+  const double stop_rr = sc->tol2 * sc->bb;
+  const int max_iter = sc->max_iter;
+  // (the last workgroup that finishes a solve sets the next solve's)
+  const unsigned epoch = unsigned(TagLoad(words + kWholeEpoch));
+  unsigned tag = epoch;
+  T xv[K], r[K], zv[K], q[K], d[K], kw[K], ke[K], ks[K], kn[K], di[K];
+  bool in[K], edge[K], hw[K], he[K];
+  double dots[2] = {0., 0.}, quot;
+  if (threadIdx.x == 0) gave_up = 0;
+  for (int h = threadIdx.x; h < C + 4 * nx; h += NT) ps[h] = T(0);
+  ++tag;
+  auto PutZ = [&](int i) {
+    if (!edge[i]) return;
+    Word* const w = zw + c0 + threadIdx.x + i * NT;
+    if constexpr (sizeof(T) == 8) {
+      TagStore(w, tag, unsigned(__double2loint(zv[i])));
+      TagStore(w + n, tag, unsigned(__double2hiint(zv[i])));
+    } else {
+      TagStore(w, tag, __float_as_uint(zv[i]));
+    }
+  };
+  // z of the rows around the range, by all waves but the first
+  auto Halo = [&]() {
+    for (int h = int(threadIdx.x) - 64; h < 2 * nx; h += NT - 64) {
+      const int c = h < nx ? c0 - nx + h : c1 - nx + h;
+      if (c < 0 || c >= n) continue;
+      for (int m = 0;; ++m) {
+        const Word lo = TagLoad(zw + c);
+        if constexpr (sizeof(T) == 8) {
+          const Word hi = TagLoad(zw + n + c);
+          zs[h] = FromWords(lo, hi);
+          if (unsigned(lo >> 32) == tag && unsigned(hi >> 32) == tag) break;
+        } else {
+          zs[h] = __uint_as_float(unsigned(lo));
+          if (unsigned(lo >> 32) == tag) break;
+        }
+        if (m == kWholeSpin) return false;
+      }
+    }
+    return true;
+  };
+#pragma unroll
+  for (int i = 0; i < K; ++i) {
+    const int l = threadIdx.x + i * NT, c = c0 + l;
+    in[i] = l < C && c < c1;
+    const int cc = in[i] ? c : 0, ci = cc % nx, cj = cc / nx;
+    const int fw = ci + (nx + 1) * cj;
+    hw[i] = ci > 0;
+    he[i] = ci < nx - 1;
+    edge[i] = in[i] && (l < nx || c + nx >= c1);
+    kw[i] = kx[fw];
+    ke[i] = kx[fw + 1];
+    ks[i] = ky[cc];
+    kn[i] = ky[cc + nx];
+    d[i] = ((kw[i] + ke[i]) + ks[i]) + kn[i];
+    di[i] = dinv[cc];
+    r[i] = in[i] ? r0[cc] : T(0);
+    xv[i] = in[i] ? x[cc] : T(0);
+    zv[i] = r[i] * di[i];
+    if (in[i]) xsave[c] = xv[i];
+    PutZ(i);
+    dots[0] += double(r[i]) * double(zv[i]);
+    dots[1] += double(r[i]) * double(r[i]);
+  }
+  auto None = [](const auto&) { return 0.; };
+  if (!Exchange<2>(dots, quot, tag, words, &gave_up, None, Halo)) return;
+  int k = 0;
+  for (;; ++k) {
+    const double rz = dots[0], rr = dots[1];
+    if (!(rr > stop_rr) || k >= max_iter || !(rr == rr)) break;
+    const T b = T(quot);
+    // p on the rows before and after the range (0 outside the grid)
+    for (int h = threadIdx.x; h < 2 * nx; h += NT) {
+      const int l = h < nx ? h : c1 - c0 + h;
+      ps[l] = zs[h] + b * ps[l];
+    }
+    T p[K];
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+      const int l = nx + threadIdx.x + i * NT;
+      if (in[i]) {
+        p[i] = zv[i] + b * ps[l];
+        ps[l] = p[i];
+      }
+    }
+    __syncthreads();
+    double pq[1] = {0.};
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+      if (in[i]) {
+        const int l = nx + threadIdx.x + i * NT;
+        T v = d[i] * p[i];
+        v = hw[i] ? v - kw[i] * ps[l - 1] : v;
+        v = he[i] ? v - ke[i] * ps[l + 1] : v;
+        v = l + c0 >= 2 * nx ? v - ks[i] * ps[l - nx] : v;
+        v = l + c0 < n ? v - kn[i] * ps[l + nx] : v;
+        q[i] = v;
+        pq[0] += double(p[i]) * double(v);
+      }
+    }
+    ++tag;
+    if (!Exchange<1>(pq, quot, tag, words, &gave_up,
+                         [&](const auto& s) { return rz / s[0]; }, [] { return true; }))
+      return;
+    const T a = T(quot);
+    ++tag;
+    dots[0] = dots[1] = 0.;
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+      if (in[i]) {
+        xv[i] += a * p[i];
+        r[i] = r[i] - a * q[i];
+        zv[i] = r[i] * di[i];
+        PutZ(i);
+        dots[0] += double(r[i]) * double(zv[i]);
+        dots[1] += double(r[i]) * double(r[i]);
+      }
+    }
+    if (!Exchange<2>(dots, quot, tag, words, &gave_up,
+                         [&](const auto& s) { return s[0] / rz; }, Halo))
+      return;
+  }
+#pragma unroll
+  for (int i = 0; i < K; ++i)
+    if (in[i]) x[c0 + threadIdx.x + i * NT] = xv[i];
+  // the solve is done when every workgroup got here
+  if (threadIdx.x == 0 &&
+      __hip_atomic_fetch_add(words + kWholeDone, Word(1), __ATOMIC_RELAXED,
+                             __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1) {
+    words[kWholeDone] = 0;
+    words[kWholeEpoch] = tag;
+    sc->done = 1;
+    sc->iter = k;
+    sc->rr = dots[1];
+  }
+}
+
+// After a solve that gave up: no tag of it is used again.
+__global__ void KWholeReset(Word* words, unsigned tags) {
+  if (threadIdx.x == 0) {
+    words[kWholeDone] = 0;
+    words[kWholeEpoch] = Word(unsigned(words[kWholeEpoch]) + tags);
+  }
 }
 
 // ---- FCG(1) with an FP32 preconditioner output -----------------------------
@@ -714,6 +1008,10 @@ CgSolver::CgSolver(int nx, int ny, hipStream_t stream) : nx_(nx), ny_(ny), strea
   HG_CHECK(hipMemset(part_, 0, size_t(blocks_) * 10 * 8));
   A(&scal_, sizeof(CgScalars));
   HG_CHECK(hipMemset(scal_, 0, sizeof(CgScalars)));
+  // (the FP64 solve's z words, two per cell, where the grid is small enough)
+  const size_t words = kWholeWords + (n_ <= kWholeMaxCells ? 2 * size_t(n_) : 0);
+  A(&words_, words * 8);
+  HG_CHECK(hipMemset(words_, 0, words * 8));
   HG_CHECK(hipHostMalloc(&host_scal_, sizeof(CgScalars)));
   HG_CHECK(hipEventCreate(&ev0_));
   HG_CHECK(hipEventCreate(&ev1_));
@@ -723,7 +1021,7 @@ CgSolver::~CgSolver() {
   for (void* p : {(void*)kx_, (void*)ky_, (void*)dinv_, (void*)kx32_, (void*)ky32_,
                   (void*)dinv32_, (void*)r_, (void*)z_, (void*)pa_, (void*)pb_, (void*)q_,
                   (void*)b_, (void*)r32_, (void*)z32_, (void*)pa32_, (void*)pb32_,
-                  (void*)q32_, (void*)e32_, (void*)zprev32_, (void*)part_, scal_})
+                  (void*)q32_, (void*)e32_, (void*)zprev32_, (void*)part_, scal_, words_})
     if (p) (void)hipFree(p);
   if (host_scal_) (void)hipHostFree(host_scal_);
   if (dirx_) (void)hipFree(dirx_);
@@ -829,6 +1127,35 @@ void CgSolver::Prepare(const double* b, double* x, bool project, bool warm) {
   }
 }
 
+// The whole Jacobi-PCG solve in one launch (KPcgWhole), where the grid fits
+// and the workgroups ran together; else false, with x as it was.
+template <class T>
+bool CgSolver::WholePcg(const T* kx, const T* ky, const T* dinv, const T* r, T* x, T* xsave,
+                        int max_iters) {
+  if (n_ > kWholeMaxCells) return false;
+  // at most 16 workgroups where more cells per thread allow it: 32 cost 1.3 us
+  // more per iteration (65025 cells: 16 x 4096 4.6 us, 32 x 2048 5.0, 64 x 1024
+  // 5.8; 16384 cells: 16 x 1024 3.4, 8 x 2048 3.7, 4 x 4096 4.1)
+  const int n = int(n_), nt = kWholeThreads, k = n <= 16 * nt ? 1 : n <= 32 * nt ? 2 : 4;
+  int wgs = (n + k * nt - 1) / (k * nt);
+  const int c = ((n + wgs - 1) / wgs + 63) / 64 * 64;  // <= k nt
+  wgs = (n + c - 1) / c;
+  if (long(c) + 4L * nx_ > kWholeLds) return false;
+  Word* const words = (Word*)words_;
+  Word* const zw = words + kWholeWords;
+  CgScalars* const sc = (CgScalars*)scal_;
+  auto launch = [&](auto kernel) {
+    kernel<<<wgs, kWholeThreads, size_t(c + 4 * nx_) * sizeof(T), stream_>>>(
+        nx_, ny_, c, kx, ky, dinv, r, x, xsave, zw, words, sc);
+  };
+  launch(k == 1 ? KPcgWhole<T, 1> : k == 2 ? KPcgWhole<T, 2> : KPcgWhole<T, 4>);
+  ReadScalars();
+  if (((CgScalars*)host_scal_)->done) return true;
+  KWholeReset<<<1, 64, 0, stream_>>>(words, 2u * unsigned(max_iters) + 4u);
+  HG_CHECK(hipMemcpyAsync(x, xsave, size_t(n_) * sizeof(T), hipMemcpyDeviceToDevice, stream_));
+  return false;
+}
+
 // Jacobi-PCG on A x = b_ continuing from the current x and r_ (FP64).
 int CgSolver::JacobiPcg64(double* x, int max_iters) {
   int nb;
@@ -836,6 +1163,7 @@ int CgSolver::JacobiPcg64(double* x, int max_iters) {
   Parts pt = MakeParts(part_, nb);
   CgScalars* sc = (CgScalars*)scal_;
   CgScalars* hs = (CgScalars*)host_scal_;
+  if (WholePcg<double>(kx_, ky_, dinv_, r_, x, pb_, max_iters)) return hs->iter;
   KPcgStart<double><<<nb, kB, 0, stream_>>>(w, r_, dinv_, z_, pa_, pt);
   double* pold = pa_;
   double* pnew = pb_;
@@ -971,6 +1299,9 @@ int CgSolver::InnerFp32(double tol_inner, int max_iters, Precond*, bool*) {
   KSetup<<<1, 64, 0, stream_>>>(sc, tol_inner * tol_inner, max_iters);
   KPcgStart<float><<<nb, kB, 0, stream_>>>(w, r32_, dinv32_, z32_, pa32_, pt);
   KInnerBB<<<1, kB, 0, stream_>>>(pt, sc);
+  if (WholePcg<float>(kx32_, ky32_, dinv32_, r32_, e32_, pb32_, max_iters))
+    return hs->iter;
+  KPcgStart<float><<<nb, kB, 0, stream_>>>(w, r32_, dinv32_, z32_, pa32_, pt);
   float* pold = pa32_;
   float* pnew = pb32_;
   int k = 0;

@@ -99,3 +99,32 @@ def test_multigrid_any_side(gpu, nx, ny):
     res = np.linalg.norm(b - apply(kx, ky, p, nx, ny)) / np.linalg.norm(b)
     assert st.converged and res <= 1.05e-8
     assert st.iterations <= 100
+
+
+# grids around the one-launch solve's cells per thread and workgroup counts,
+# rows longer and shorter than a workgroup's range, the first sizes past it
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("nx,ny", [(2, 3), (64, 16), (2, 1030), (1500, 2), (129, 127), (128, 128),
+                                   (129, 128), (257, 128), (1000, 67), (1999, 9), (2100, 9),
+                                   (512, 512), (513, 512)])
+def test_jacobi_pcg_any_size(gpu, nx, ny, precision):
+    """cg against the oracle's Jacobi-PCG: the true residual meets the
+    tolerance, and in FP64 the iteration counts agree (the same recurrence;
+    sums in another order, so within two and one per cent)."""
+    rng = np.random.default_rng(nx + ny)
+    kx, ky = rng.uniform(0.5, 2.0, (ny, nx + 1)), rng.uniform(0.5, 2.0, (ny + 1, nx))
+    kx[:, 0] = kx[:, -1] = 0.0
+    ky[0] = ky[-1] = 0.0
+    kx, ky, rhs = kx.reshape(-1), ky.reshape(-1), rng.normal(size=nx * ny)
+    print(f"case: cg {nx}x{ny} precision {precision}", flush=True)
+    ps = Poisson(nx, ny, kx, ky)
+    b = rhs - rhs.mean()
+    for _ in range(2):  # a second solve on the same exchange words
+        p, st = ps.solve(rhs, solver="cg", tol=1e-6, precision=precision)
+        res = np.linalg.norm(b - apply(kx, ky, p, nx, ny)) / np.linalg.norm(b)
+        assert st.converged and res <= 1.05e-6, (res, st.iterations)
+        if precision == 0:
+            _, so = pyoracle.poisson_solve(nx, ny, kx, ky, rhs, tol=1e-6)
+            assert abs(st.iterations - so.iterations) <= 2 + 0.01 * so.iterations
+    q, sq = ps.solve(rhs, solver="cg", tol=0.0, max_iters=3, precision=0)
+    assert nx * ny < 7 or (sq.iterations == 3 and not sq.converged)
