@@ -109,6 +109,7 @@ class UNet {
   bool scale_free_ = false;
   double last_alpha_ = 0.;
   double* part_ = nullptr;
+  float* wpart_ = nullptr;  // partial weight gradients
   double* loss_h_ = nullptr;
   const float *mkx_ = nullptr, *mky_ = nullptr;
   bool linear_ = false, tied_ = false;

@@ -57,6 +57,19 @@ __device__ __forceinline__ uint4 Ld8(const bf* p) { return *reinterpret_cast<con
 __device__ __forceinline__ b8 LdOp(const bf* p) { return __builtin_bit_cast(b8, Ld8(p)); }
 __device__ __forceinline__ void St8(bf* p, uint4 v) { *reinterpret_cast<uint4*>(p) = v; }
 
+// Sum over the wave, in lane 63.
+__device__ __forceinline__ float WaveSumF(float v) {
+#define HG_DPP_ADD(ctrl, rows) \
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), ctrl, rows, 0xf, true))
+  HG_DPP_ADD(0x111, 0xf);  // row_shr:1, 2, 4, 8
+  HG_DPP_ADD(0x112, 0xf);
+  HG_DPP_ADD(0x114, 0xf);
+  HG_DPP_ADD(0x118, 0xf);
+  HG_DPP_ADD(0x142, 0xa);  // row_bcast:15, 31
+  HG_DPP_ADD(0x143, 0xc);
+#undef HG_DPP_ADD
+  return v;
+}
 
 // ---------------------------------------------------------------------------
 // 3x3 'same' convolution, CIN, COUT multiples of 16, as an implicit GEMM on
@@ -153,80 +166,142 @@ KConvMfma(int W, int H, const bf* __restrict__ in, const bf* __restrict__ wt,
 }
 
 // Weight gradient dW[tap][ci][co] += sum_p in[p + off(tap)][ci] g[p][co]:
-// per tap an implicit GEMM with M = 16 input channels, N = COUT, K = pixels,
-// 32 pixels per MFMA 16x16x32 BF16.  Grid: x = tap * (CIN/16) + channel
-// tile, y = row blocks of `rows` rows.  The block walks its rows in chunks of
-// kWgCols pixels: it stages the chunk's input pixels (shifted by the tap's
-// offset, zero outside the grid; 16 channels) and output gradients (COUT
-// channels) in LDS channel-major, from 16-byte global loads, so that each
-// lane's operand -- 8 consecutive pixels of one channel -- is one aligned
-// 16-byte LDS load; wave w takes the chunk's pixels 32 w .. 32 w + 31.
-constexpr int kWgCols = 128;                 // pixels per staged chunk (4 waves x 32)
-constexpr int kWgStride = kWgCols + 8;       // LDS row stride (16-byte multiple)
+// per tap an implicit GEMM with M = 16 input channels, N = 16 output channels,
+// K = pixels, 32 pixels per MFMA 16x16x32 BF16.  A block of 4 waves walks
+// tiles of 64 x TR pixels: it stages the input tile with its one-pixel halo and
+// the output gradients in LDS as they lie in memory (pixel by pixel, 16-byte
+// loads and stores), once for all nine taps.  An operand -- 8 consecutive
+// pixels of one channel per lane -- is two transposing LDS reads of 4 pixels x
+// 16 channels per 16 lanes (ds_read_b64_tr_b16: lane i reads channels 4 (i % 4)
+// .. of pixel i / 4, and gets channel i of the four pixels; checked on the
+// device), so that a tap is an address offset.  Wave w holds all taps and output
+// channels of input channels 16 (w % MW) .. and takes every KW-th 32 pixels.
+// Each (block, pixel share) writes its sums to `part`, which KSumParts adds in
+// order.
+//
+// What bounds it is latency: a tile's loads, a few hundred MFMAs per wave, and
+// the partial sums' way through memory.  One tap and 16 input channels per
+// block, with both operands transposed by 2-byte LDS stores, took (64 -> 64 at
+// 64 x 128 pixels, 32 -> 64 at 128 x 256, 16 -> 32 at 256 x 512) 188, 114 and
+// 75 us; this takes 14, 19 and 16, and KSumParts 5 more.
+constexpr int kWgX = 64;            // tile width
+constexpr int kWgHX = kWgX + 2;     // with halo
+constexpr long kWgPartFloats = 4L << 20;  // of one layer's partial sums
+template <int CIN, int COUT>
+struct WgShape {
+  static constexpr int MW = CIN / 16, KW = 4 / MW;
+  static constexpr int CP = CIN + 8, GP = COUT + 8;  // pixel strides in LDS (16-byte multiples)
+  static constexpr int Lds(int tr) { return (kWgHX * (tr + 2) * CP + kWgX * tr * GP) * 2; }
+  static constexpr int TR = Lds(4) <= 65536 ? 4 : 2;  // tile height
+  static_assert(CIN % 16 == 0 && COUT % 16 == 0 && 4 % MW == 0 && Lds(TR) <= 65536, "channels");
+  // blocks for a W x H layer: one per tile up to 256 and to kWgPartFloats
+  static int Blocks(int W, int H) {
+    const long tiles = long((W + kWgX - 1) / kWgX) * ((H + TR - 1) / TR);
+    return int(std::min({tiles, 256L, kWgPartFloats / (KW * 9L * CIN * COUT)}));
+  }
+};
+
 template <int CIN, int COUT>
 __global__ void __launch_bounds__(256)
-KConvWgrad(int W, int H, int rows, const bf* __restrict__ in, const bf* __restrict__ g,
-           float* __restrict__ dw) {
-  static_assert(CIN % 16 == 0 && COUT % 16 == 0, "channel counts");
-  __shared__ __attribute__((aligned(16))) bf sa[16 * kWgStride];
-  __shared__ __attribute__((aligned(16))) bf sb[COUT * kWgStride];
+KConvWgrad(int W, int H, int tiles_x, int tiles, const bf* __restrict__ in,
+           const bf* __restrict__ g, float* __restrict__ part) {
+  using S = WgShape<CIN, COUT>;
+  constexpr int TR = S::TR, CP = S::CP, GP = S::GP, NC = COUT / 16;
+  __shared__ __attribute__((aligned(16))) bf sin_[kWgHX * (TR + 2) * CP];
+  __shared__ __attribute__((aligned(16))) bf sg[kWgX * TR * GP];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int t = blockIdx.x / (CIN / 16), ct = blockIdx.x % (CIN / 16);
-  const int dy = t / 3 - 1, dx = t % 3 - 1;
-  const int kq = lane >> 4, pj = lane & 15;
-  f4 acc[COUT / 16];
+  const int mt = wave % S::MW, kw = wave / S::MW;
+  // this lane's pixel and channels of an operand's first transposing read
+  const int px = 8 * (lane >> 4) + ((lane & 15) >> 2), ch = 4 * (lane & 3);
+  auto Operand = [&](const bf* p, int stride) {
+    using L4 = __attribute__((address_space(3))) s4;
+    const s4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((L4*)p);
+    const s4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((L4*)(p + 4 * stride));
+    return __builtin_bit_cast(b8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+  };
+  f4 acc[9][NC];
 #pragma unroll
-  for (int n = 0; n < COUT / 16; ++n) acc[n] = f4{0.f, 0.f, 0.f, 0.f};
-  const int y0 = blockIdx.y * rows, y1 = min(H, y0 + rows);
-  for (int y = y0; y < y1; ++y) {
-    const int yy = y + dy;
-    for (int x0 = 0; x0 < W; x0 += kWgCols) {
-      // input: 16 channels = two 8-channel loads per pixel
-      for (int q = threadIdx.x; q < kWgCols * 2; q += 256) {
-        const int px = q >> 1, half = q & 1;
-        const int x = x0 + px, xx = x + dx;
-        uint4 v = uint4{0u, 0u, 0u, 0u};
-        if (x < W && xx >= 0 && xx < W && yy >= 0 && yy < H)
-          v = Ld8(in + (size_t(yy) * W + xx) * CIN + ct * 16 + half * 8);
-        float f[8];
-        Unpack8(v, f);
+  for (int t = 0; t < 9; ++t)
 #pragma unroll
-        for (int e = 0; e < 8; ++e) sa[(half * 8 + e) * kWgStride + px] = bf(__float_as_uint(f[e]) >> 16);
+    for (int n = 0; n < NC; ++n) acc[t][n] = f4{0.f, 0.f, 0.f, 0.f};
+  for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+    const int x0 = tile % tiles_x * kWgX, y0 = tile / tiles_x * TR;
+    constexpr int GI = CIN / 8, GO = COUT / 8;
+    for (int q = threadIdx.x; q < kWgHX * (TR + 2) * GI; q += 256) {
+      const int c8 = q % GI, p = q / GI;
+      const int xx = x0 + p % kWgHX - 1, yy = y0 + p / kWgHX - 1;
+      uint4 v = uint4{0u, 0u, 0u, 0u};
+      if (xx >= 0 && xx < W && yy >= 0 && yy < H) v = Ld8(in + (size_t(yy) * W + xx) * CIN + c8 * 8);
+      St8(sin_ + p * CP + c8 * 8, v);
+    }
+    for (int q = threadIdx.x; q < kWgX * TR * GO; q += 256) {
+      const int c8 = q % GO, p = q / GO;
+      const int xx = x0 + p % kWgX, yy = y0 + p / kWgX;
+      uint4 v = uint4{0u, 0u, 0u, 0u};
+      if (xx < W && yy < H) v = Ld8(g + (size_t(yy) * W + xx) * COUT + c8 * 8);
+      St8(sg + p * GP + c8 * 8, v);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 2 * TR / S::KW; ++k) {
+      const int ks = k * S::KW + kw;  // 32 pixels of row ks / 2
+      const int row = ks >> 1, col = (ks & 1) * 32 + px;
+      b8 bg[NC];
+#pragma unroll
+      for (int n = 0; n < NC; ++n) bg[n] = Operand(sg + (row * kWgX + col) * GP + n * 16 + ch, GP);
+#pragma unroll
+      for (int t = 0; t < 9; ++t) {
+        const b8 a =
+            Operand(sin_ + ((row + t / 3) * kWgHX + col + t % 3) * CP + mt * 16 + ch, CP);
+#pragma unroll
+        for (int n = 0; n < NC; ++n)
+          acc[t][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bg[n], acc[t][n], 0, 0, 0);
       }
-      // output gradient: COUT channels, 8 per load
-      for (int q = threadIdx.x; q < kWgCols * (COUT / 8); q += 256) {
-        const int px = q / (COUT / 8), grp = q % (COUT / 8);
-        const int x = x0 + px;
-        uint4 v = uint4{0u, 0u, 0u, 0u};
-        if (x < W) v = Ld8(g + (size_t(y) * W + x) * COUT + grp * 8);
-        float f[8];
-        Unpack8(v, f);
+    }
+    __syncthreads();  // the tile's LDS is restaged next
+  }
+  // D[i][j]: i = 4 (lane / 16) + v (input channel), j = lane % 16 (output channel)
+  float* const out = part + size_t(blockIdx.x * S::KW + kw) * (9 * CIN * COUT);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) sb[(grp * 8 + e) * kWgStride + px] = bf(__float_as_uint(f[e]) >> 16);
-      }
-      __syncthreads();
-      const int k0 = 32 * wave + 8 * kq;  // this lane's 8 pixels of the wave's 32
-      const b8 a = LdOp(sa + pj * kWgStride + k0);
+  for (int t = 0; t < 9; ++t)
 #pragma unroll
-      for (int n = 0; n < COUT / 16; ++n)
-        acc[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, LdOp(sb + (n * 16 + pj) * kWgStride + k0),
-                                                         acc[n], 0, 0, 0);
-      __syncthreads();  // the chunk's LDS is restaged next
+    for (int n = 0; n < NC; ++n)
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+        out[(t * CIN + mt * 16 + 4 * (lane >> 4) + v) * COUT + n * 16 + (lane & 15)] = acc[t][n][v];
+}
+
+// dw[i] += part[0][i] + part[1][i] + ... of np arrays of 4 n4 floats: a block
+// sums 64 weights, 16 shares of the arrays side by side, the shares in order.
+__global__ void __launch_bounds__(256)
+KSumParts(int n4, int np, const float4* __restrict__ part, float4* __restrict__ dw) {
+  __shared__ float4 red[16][16];
+  const int l = threadIdx.x & 15, share = threadIdx.x >> 4;
+  const int i = blockIdx.x * 16 + l;
+  float4 s = {0.f, 0.f, 0.f, 0.f};
+  if (i < n4) {
+#pragma unroll 8
+    for (int p = share; p < np; p += 16) {
+      const float4 v = part[size_t(p) * n4 + i];
+      s.x += v.x;
+      s.y += v.y;
+      s.z += v.z;
+      s.w += v.w;
     }
   }
-  // reduce the four waves in LDS, then one atomic add per weight
-  __shared__ float red[4][COUT / 16][4][64];
-#pragma unroll
-  for (int n = 0; n < COUT / 16; ++n)
-#pragma unroll
-    for (int v = 0; v < 4; ++v) red[wave][n][v][lane] = acc[n][v];
+  red[share][l] = s;
   __syncthreads();
-  for (int q = threadIdx.x; q < (COUT / 16) * 4 * 64; q += 256) {
-    const int n = q / 256, v = (q / 64) % 4, l = q % 64;
-    const float s = red[0][n][v][l] + red[1][n][v][l] + red[2][n][v][l] + red[3][n][v][l];
-    // D[i][j]: i = 4*(l/16) + v (input channel), j = l % 16 (output channel)
-    const int i = 4 * (l >> 4) + v, j = l & 15;
-    atomicAdd(&dw[(size_t(t) * CIN + ct * 16 + i) * COUT + n * 16 + j], s);
+  if (share == 0 && i < n4) {
+    float4 o = dw[i];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+      const float4 v = red[k][l];
+      o.x += v.x;
+      o.y += v.y;
+      o.z += v.z;
+      o.w += v.w;
+    }
+    dw[i] = o;
   }
 }
 
@@ -302,13 +377,18 @@ KConvD0Dgrad(int W, int H, const float* __restrict__ gy, const float* __restrict
   St8(gin + size_t(p) * 16 + 8, Pack8(acc + 8));
 }
 
-// Weight gradients of the 1-channel ends, reduced per block then atomics:
-// E0: dw[t][co] += x[p + off(t)] g[p][co];  D0: dw[t][ci] += in[p + off(t)][ci] gy[p].
+// Weight gradients of the 1-channel ends, with s the 1-channel and f the
+// 16-channel field:  E0: dw[t][co] += s[p + off(t)] f[p][co], f the gradient;
+// D0: dw[t][ci] += f[p][ci] s[p - off(t)], s the gradient.  Each thread sums its
+// pixels (f in two 16-byte loads), a wave its lanes, and each block writes its
+// sums for KSumParts.  (16 threads that added 256 rows of LDS per tap, behind
+// 16 two-byte loads per pixel, took 45 us at 512 x 1024; this takes 18.)
+constexpr int kEndBlocks = 256;
 template <bool E0>
 __global__ void __launch_bounds__(256)
-KEndWgrad(int W, int H, const float* __restrict__ xs, const bf* __restrict__ gb,
-          const bf* __restrict__ inb, const float* __restrict__ gys, float* __restrict__ dw) {
-  __shared__ float red[256][17];
+KEndWgrad(int W, int H, const float* __restrict__ s, const bf* __restrict__ f,
+          float* __restrict__ part) {
+  __shared__ float red[4][9 * 16];
   float acc[9][16];
 #pragma unroll
   for (int t = 0; t < 9; ++t)
@@ -316,31 +396,35 @@ KEndWgrad(int W, int H, const float* __restrict__ xs, const bf* __restrict__ gb,
     for (int c = 0; c < 16; ++c) acc[t][c] = 0.f;
   for (int p = blockIdx.x * 256 + threadIdx.x; p < W * H; p += gridDim.x * 256) {
     const int px = p % W, py = p / W;
+    float v[16];
+    Unpack8(Ld8(f + size_t(p) * 16), v);
+    Unpack8(Ld8(f + size_t(p) * 16 + 8), v + 8);
+    float a[9];
+    bool in[9];
 #pragma unroll
     for (int t = 0; t < 9; ++t) {
-      const int xx = px + t % 3 - 1, yy = py + t / 3 - 1;
-      if (xx < 0 || xx >= W || yy < 0 || yy >= H) continue;
-      if (E0) {
-        const float v = xs[yy * W + xx];
+      const int dx = t % 3 - 1, dy = t / 3 - 1;
+      const int xx = E0 ? px + dx : px - dx, yy = E0 ? py + dy : py - dy;
+      in[t] = xx >= 0 && xx < W && yy >= 0 && yy < H;
+      a[t] = s[in[t] ? yy * W + xx : p];
+    }
 #pragma unroll
-        for (int c = 0; c < 16; ++c) acc[t][c] += v * B2F(gb[size_t(p) * 16 + c]);
-      } else {
-        const float g = gys[p];
+    for (int t = 0; t < 9; ++t) {
+      if (!in[t]) continue;
 #pragma unroll
-        for (int c = 0; c < 16; ++c) acc[t][c] += B2F(inb[(size_t(yy) * W + xx) * 16 + c]) * g;
-      }
+      for (int c = 0; c < 16; ++c) acc[t][c] += a[t] * v[c];
     }
   }
-  for (int t = 0; t < 9; ++t) {
-    for (int c = 0; c < 16; ++c) red[threadIdx.x][c] = acc[t][c];
-    __syncthreads();
-    if (threadIdx.x < 16) {
-      float s = 0.f;
-      for (int q = 0; q < 256; ++q) s += red[q][threadIdx.x];
-      atomicAdd(&dw[t * 16 + threadIdx.x], s);
+#pragma unroll
+  for (int t = 0; t < 9; ++t)
+#pragma unroll
+    for (int c = 0; c < 16; ++c) {
+      const float w = WaveSumF(acc[t][c]);
+      if ((threadIdx.x & 63) == 63) red[threadIdx.x >> 6][t * 16 + c] = w;
     }
-    __syncthreads();
-  }
+  __syncthreads();
+  for (int q = threadIdx.x; q < 9 * 16; q += 256)
+    part[blockIdx.x * (9 * 16) + q] = ((red[0][q] + red[1][q]) + red[2][q]) + red[3][q];
 }
 
 // ---- elementwise ops on BF16 NHWC tensors ----------------------------------
@@ -627,19 +711,42 @@ void ConvFwd(int cin, int cout, bool relu, int W, int H, const bf* in, const bf*
   throw std::runtime_error("no MFMA conv for this channel pair");
 }
 
-void ConvWgrad(int cin, int cout, int W, int H, const bf* in, const bf* g, float* dw,
-               hipStream_t st) {
-  const int rows = std::max(1, std::min(H, 8192 / std::max(W, 1)));
-  dim3 grid(unsigned(9 * (cin / 16)), unsigned((H + rows - 1) / rows));
+// the channel pairs of the weight gradient
+#define HG_WG_PAIRS                                                                      \
+  HG_WG(16, 32) HG_WG(32, 64) HG_WG(64, 64) HG_WG(64, 32) HG_WG(32, 16)                  \
+  HG_WG(16, 16) HG_WG(32, 32) HG_WG(16, 64) HG_WG(64, 16)
+
+void SumParts(int n, int np, const float* part, float* dw, hipStream_t st) {
+  KSumParts<<<unsigned((n / 4 + 15) / 16), 256, 0, st>>>(
+      n / 4, np, reinterpret_cast<const float4*>(part), reinterpret_cast<float4*>(dw));
+}
+
+// dw += the weight gradient; part: WgradPartFloats(cin, cout, W, H) floats.
+void ConvWgrad(int cin, int cout, int W, int H, const bf* in, const bf* g, float* part,
+               float* dw, hipStream_t st) {
 #define HG_WG(CI, CO)                                                                     \
   if (cin == CI && cout == CO) {                                                          \
-    KConvWgrad<CI, CO><<<grid, 256, 0, st>>>(W, H, rows, in, g, dw);                      \
+    using S = WgShape<CI, CO>;                                                            \
+    const int tx = (W + kWgX - 1) / kWgX, tiles = tx * ((H + S::TR - 1) / S::TR);         \
+    const int nb = S::Blocks(W, H);                                                       \
+    KConvWgrad<CI, CO><<<unsigned(nb), 256, 0, st>>>(W, H, tx, tiles, in, g, part);       \
+    SumParts(9 * CI * CO, nb * S::KW, part, dw, st);                                      \
     return;                                                                               \
   }
-  HG_WG(16, 32) HG_WG(32, 64) HG_WG(64, 64) HG_WG(64, 32) HG_WG(32, 16)
-  HG_WG(16, 16) HG_WG(32, 32) HG_WG(16, 64) HG_WG(64, 16)
+  HG_WG_PAIRS
 #undef HG_WG
   throw std::runtime_error("no MFMA wgrad for this channel pair");
+}
+
+long WgradPartFloats(int cin, int cout, int W, int H) {
+#define HG_WG(CI, CO)                                                                     \
+  if (cin == CI && cout == CO) {                                                          \
+    using S = WgShape<CI, CO>;                                                            \
+    return long(S::Blocks(W, H)) * S::KW * 9 * CI * CO;                                   \
+  }
+  HG_WG_PAIRS
+#undef HG_WG
+  return 0;
 }
 
 }  // namespace
@@ -698,11 +805,15 @@ UNet::UNet(int nx, int ny) : nx_(nx), ny_(ny) {
   A((void**)&qt_, size_t(nx) * ny * 4);
   A((void**)&gy_, size_t(nx) * ny * 4);
   A((void**)&part_, 65536 * 8);
+  long np = kEndBlocks * 9 * 16;
+  for (const Layer& L : layer_)
+    np = std::max(np, WgradPartFloats(L.cin, L.cout, lw_[L.level], lh_[L.level]));
+  A((void**)&wpart_, size_t(np) * 4);
   HG_CHECK(hipHostMalloc((void**)&loss_h_, 65536 * 8));
 }
 
 UNet::~UNet() {
-  std::vector<void*> ps = {w_, g_, m_, v_, wf_, wb_, wd0_, gtie_, yb_, qu_, qt_, gy_, part_};
+  std::vector<void*> ps = {w_, g_, m_, v_, wf_, wb_, wd0_, gtie_, yb_, qu_, qt_, gy_, part_, wpart_};
   for (int l = 0; l < kLevels; ++l)
     for (void* p : {(void*)enc_[l], (void*)genc_[l], (void*)gin_[l], (void*)gpre_[l],
                     (void*)pin_[l], (void*)dout_[l], (void*)gtmp_[l], (void*)din_[l]})
@@ -796,10 +907,12 @@ void UNet::Backward(const float* x, const float* gy, hipStream_t st) {
   KConvD0Dgrad<<<Blk(n0), 256, 0, st>>>(W0, H0, gy, D0Weights(), gin_[0]);
   if (tied_) {
     HG_CHECK(hipMemsetAsync(gtie_, 0, 9 * 16 * 4, st));
-    KEndWgrad<false><<<256, 256, 0, st>>>(W0, H0, nullptr, nullptr, din_[0], gy, gtie_);
+    KEndWgrad<false><<<kEndBlocks, 256, 0, st>>>(W0, H0, gy, din_[0], wpart_);
+    SumParts(9 * 16, kEndBlocks, wpart_, gtie_, st);
     KFoldTied<<<1, 256, 0, st>>>(1, ch_[0], gtie_, g_ + layer_[0].off);
   } else {
-    KEndWgrad<false><<<256, 256, 0, st>>>(W0, H0, nullptr, nullptr, din_[0], gy, g_ + D0.off);
+    KEndWgrad<false><<<kEndBlocks, 256, 0, st>>>(W0, H0, gy, din_[0], wpart_);
+    SumParts(9 * 16, kEndBlocks, wpart_, g_ + D0.off, st);
   }
   // din0 = up(dout1) + enc0: grad to enc0 and (summed over children) to dout1
   HG_CHECK(hipMemcpyAsync(genc_[0], gin_[0], size_t(n0) * ch_[0] * 2, hipMemcpyDeviceToDevice, st));
@@ -819,11 +932,11 @@ void UNet::Backward(const float* x, const float* gy, hipStream_t st) {
     if (tied_) {
       const Layer& E = layer_[l];
       HG_CHECK(hipMemsetAsync(gtie_, 0, size_t(9) * E.cin * E.cout * 4, st));
-      ConvWgrad(L.cin, L.cout, W, H, src, gp, gtie_, st);
+      ConvWgrad(L.cin, L.cout, W, H, src, gp, wpart_, gtie_, st);
       KFoldTied<<<Blk(9L * E.cin * E.cout), 256, 0, st>>>(E.cin, E.cout, gtie_, g_ + E.off);
       ConvFwd(L.cout, L.cin, false, W, H, gp, wf_ + E.off, gin_[l], st, nullptr);
     } else {
-      ConvWgrad(L.cin, L.cout, W, H, src, gp, g_ + L.off, st);
+      ConvWgrad(L.cin, L.cout, W, H, src, gp, wpart_, g_ + L.off, st);
       ConvFwd(L.cout, L.cin, false, W, H, gp, wb_ + L.off, gin_[l], st, nullptr);
     }
     HG_CHECK(hipMemcpyAsync(genc_[l], gin_[l], size_t(np) * ch_[l] * 2, hipMemcpyDeviceToDevice,
@@ -842,7 +955,7 @@ void UNet::Backward(const float* x, const float* gy, hipStream_t st) {
       KMask<<<Blk(np * L.cout), 256, 0, st>>>(np * L.cout, genc_[l], enc_[l], gpre_[l]);
       gp = gpre_[l];
     }
-    ConvWgrad(L.cin, L.cout, W, H, pin_[l], gp, g_ + L.off, st);
+    ConvWgrad(L.cin, L.cout, W, H, pin_[l], gp, wpart_, g_ + L.off, st);
     ConvFwd(L.cout, L.cin, false, W, H, gp, wb_ + L.off, gin_[l], st, nullptr);
     KPoolBwdAdd<<<Blk(long(lw_[l - 1]) * lh_[l - 1] * ch_[l - 1]), 256, 0, st>>>(
         lw_[l - 1], lh_[l - 1], ch_[l - 1], gin_[l], genc_[l - 1]);
@@ -852,7 +965,8 @@ void UNet::Backward(const float* x, const float* gy, hipStream_t st) {
     KMask<<<Blk(n0 * ch_[0]), 256, 0, st>>>(n0 * ch_[0], genc_[0], enc_[0], gpre_[0]);
     gp0 = gpre_[0];
   }
-  KEndWgrad<true><<<256, 256, 0, st>>>(W0, H0, x, gp0, nullptr, nullptr, g_ + layer_[0].off);
+  KEndWgrad<true><<<kEndBlocks, 256, 0, st>>>(W0, H0, x, gp0, wpart_);
+  SumParts(9 * 16, kEndBlocks, wpart_, g_ + layer_[0].off, st);
 }
 
 void UNet::AdamStep(float lr, hipStream_t st) {

@@ -130,6 +130,30 @@ def test_gradient_matches_oracle(nets, weights, mode):
         off += k
 
 
+# tiles of 64 x 2 and 64 x 4 pixels on the levels: one, remainders in x and y,
+# more tiles than blocks.  The linear network and its bound (the number model's
+# own distance from FP64), which holds at any size: with ReLU the distance from
+# the model grows with the pixels at which a rounding flips the mask.
+@pytest.mark.parametrize("nx,ny", [(16, 16), (72, 24), (136, 40), (16, 264), (584, 272)])
+def test_gradient_any_size(gpu, weights, nx, ny):
+    rng = np.random.default_rng(nx)
+    x = rng.normal(size=(ny, nx))
+    gy = rng.normal(size=(ny, nx))
+    print(f"case: net gradient {nx}x{ny}", flush=True)
+    n = Net(nx, ny)
+    n.configure(linear=True)
+    n.set_weights(weights)
+    gw = n.gradient(x, gy).astype(np.float64)
+    n.close()
+    model, _ = pynet.backward(weights, x, gy, rnd=pynet.bf16, linear=True)
+    exact, _ = pynet.backward(weights, x, gy, linear=True)
+    off = 0
+    for name, ci, co, _ in pynet.layer_shapes():
+        sl = slice(off, off + 9 * ci * co)
+        assert rel(gw[sl], exact[sl]) < 1.5 * rel(model[sl], exact[sl]) + 1e-3, name
+        off += 9 * ci * co
+
+
 def test_tied_network_symmetric(nets):
     """(u, N v) = (N u, v) for the tied network, to BF16 rounding."""
     rng = np.random.default_rng(12)
