@@ -74,13 +74,13 @@ __device__ __forceinline__ float WaveSumF(float v) {
 // ---------------------------------------------------------------------------
 // 3x3 'same' convolution, CIN, COUT multiples of 16, as an implicit GEMM on
 // gfx950's MFMA 16x16x32 BF16 (FP32 accumulate).  A block of 4 waves
-// computes a 64 x 4 pixel tile (one row per wave) for all output channels.
+// computes a 16 SEG x 4 pixel tile (one row per wave) for all output channels.
 // The input tile with its one-pixel halo is staged once in LDS (16-byte
 // global loads and LDS stores; pixels padded to CIN + 8 channels, a 16-byte
 // multiple, so every operand read is one aligned 16-byte LDS load).  The
 // GEMM's K runs over (tap, input channel), k = tap * CIN + ci, 32 at a time:
 // per chunk a wave multiplies each weight block (M = 16 output channels,
-// read once and used kSeg times) by kSeg input blocks from LDS (N = 16
+// read once and used SEG times) by SEG input blocks from LDS (N = 16
 // pixels each); with CIN = 16 a chunk spans two taps, and the chunk past
 // the ninth tap is zero.  Operand lane layouts (checked on the device):
 // A[i][k] in lane i + 16*(k/8), element k%8 (8 consecutive channels of one
@@ -89,23 +89,42 @@ __device__ __forceinline__ float WaveSumF(float v) {
 // lane ends with 4 consecutive output channels of one pixel and stores them
 // as one 8-byte word.  Used for the forward pass and, with tap-flipped
 // weights, for dgrad.
-constexpr int kSeg = 4;           // 16-pixel blocks per wave: 64-pixel rows
-constexpr int kCTX = 16 * kSeg;   // tile width
+//
+// SEG input blocks per wave (a tile is 16 SEG pixels wide): four use a weight
+// block most often, but leave the coarse levels with fewer blocks than CUs;
+// there a wave's weight loads, from L2 or memory once per chunk, are what takes
+// the time, so they are issued kAhead chunks ahead and the tiles are narrower
+// (64 -> 64 at 64 x 128 pixels: 17.0 us with 32 blocks of 64 x 4, 12.1 with 128
+// of 16 x 4; 64 -> 32 at 128 x 256: 12.6 with 128, 10.1 with 256 of 32 x 4).
 constexpr int kCTY = 4;           // tile height (one row per wave)
+constexpr int kAhead = 4;
 
-template <int CIN, int COUT, bool RELU>
+template <int CIN, int COUT, bool RELU, int SEG>
 __global__ void __launch_bounds__(256)
 KConvMfma(int W, int H, const bf* __restrict__ in, const bf* __restrict__ wt,
           bf* __restrict__ out, const int* done) {
   if (Done(done)) return;
   static_assert(CIN % 16 == 0 && COUT % 16 == 0, "channel counts");
   constexpr int CP = CIN + 8;  // padded channel stride in LDS (16-byte multiple)
-  constexpr int HX = kCTX + 2, HY = kCTY + 2;
+  constexpr int kCTX = 16 * SEG, HX = kCTX + 2, HY = kCTY + 2;
   __shared__ __attribute__((aligned(16))) bf sin_[HY * HX * CP];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int tiles_x = (W + kCTX - 1) / kCTX;
   const int bx = blockIdx.x % tiles_x, by = blockIdx.x / tiles_x;
   const int x0 = bx * kCTX, y0 = by * kCTY;
+  const int pj = lane & 15, kq = lane >> 4;
+  constexpr int NQ = (9 * CIN + 31) / 32, NC = COUT / 16;  // K chunks, channel blocks
+  const b8 zero = __builtin_bit_cast(b8, uint4{0u, 0u, 0u, 0u});
+  // this lane's 8 values of chunk q: channels ci0..ci0+7 of tap t
+  b8 bw[kAhead][NC];
+  auto Weights = [&](int q) {
+    const int kk = 32 * q + 8 * kq, t = kk / CIN, ci0 = kk % CIN;
+#pragma unroll
+    for (int n = 0; n < NC; ++n)
+      bw[q % kAhead][n] = t < 9 ? LdOp(wt + size_t(t * COUT + n * 16 + pj) * CIN + ci0) : zero;
+  };
+#pragma unroll
+  for (int q = 0; q < kAhead - 1; ++q) Weights(q);
   // stage the input tile + halo: 8 channels (16 bytes) per load
   constexpr int G = CIN / 8;
   for (int q = threadIdx.x; q < HX * HY * G; q += 256) {
@@ -119,36 +138,30 @@ KConvMfma(int W, int H, const bf* __restrict__ in, const bf* __restrict__ wt,
   __syncthreads();
   const int ty = y0 + wave;
   if (ty >= H) return;
-  const int pj = lane & 15, kq = lane >> 4;
-  f4 acc[kSeg][COUT / 16];
+  f4 acc[SEG][NC];
 #pragma unroll
-  for (int s = 0; s < kSeg; ++s)
+  for (int s = 0; s < SEG; ++s)
 #pragma unroll
-    for (int n = 0; n < COUT / 16; ++n) acc[s][n] = f4{0.f, 0.f, 0.f, 0.f};
-  constexpr int NQ = (9 * CIN + 31) / 32;  // K chunks
-  const b8 zero = __builtin_bit_cast(b8, uint4{0u, 0u, 0u, 0u});
+    for (int n = 0; n < NC; ++n) acc[s][n] = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int q = 0; q < NQ; ++q) {
-    // this lane's 8 values of the chunk: channels ci0..ci0+7 of tap t
+    if (q + kAhead - 1 < NQ) Weights(q + kAhead - 1);
     const int kk = 32 * q + 8 * kq;
     const int t = kk / CIN, ci0 = kk % CIN;
     const bool live = t < 9;
     const int hy = wave + t / 3;
-    b8 bw[COUT / 16];
 #pragma unroll
-    for (int n = 0; n < COUT / 16; ++n)
-      bw[n] = live ? LdOp(wt + size_t(t * COUT + n * 16 + pj) * CIN + ci0) : zero;
-#pragma unroll
-    for (int s = 0; s < kSeg; ++s) {
+    for (int s = 0; s < SEG; ++s) {
       const int hx = 16 * s + pj + t % 3;
       const b8 xin = live ? LdOp(sin_ + (hy * HX + hx) * CP + ci0) : zero;
 #pragma unroll
-      for (int n = 0; n < COUT / 16; ++n)
-        acc[s][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bw[n], xin, acc[s][n], 0, 0, 0);
+      for (int n = 0; n < NC; ++n)
+        acc[s][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bw[q % kAhead][n], xin, acc[s][n], 0,
+                                                            0, 0);
     }
   }
 #pragma unroll
-  for (int s = 0; s < kSeg; ++s) {
+  for (int s = 0; s < SEG; ++s) {
     const int px = x0 + 16 * s + pj;
     if (px >= W) continue;
 #pragma unroll
@@ -696,13 +709,21 @@ inline unsigned Blk(long n) { return unsigned(std::min<long>((n + 255) / 256, 65
 // Dispatch of the MFMA conv for the (cin, cout) pairs of the network.
 void ConvFwd(int cin, int cout, bool relu, int W, int H, const bf* in, const bf* wt, bf* out,
              hipStream_t st, const int* done) {
-  const unsigned grid = unsigned(((W + kCTX - 1) / kCTX) * ((H + kCTY - 1) / kCTY));
+  auto blocks = [&](int seg) { return ((W + 16 * seg - 1) / (16 * seg)) * ((H + kCTY - 1) / kCTY); };
+  // at least a block per CU, if the grid has them (figures at KConvMfma)
+  const int seg = blocks(4) >= 256 ? 4 : blocks(2) >= 256 ? 2 : 1;
+  const unsigned grid = unsigned(blocks(seg));
+  auto launch = [&](auto k4, auto k2, auto k1) {
+    (seg == 4 ? k4 : seg == 2 ? k2 : k1)<<<grid, 256, 0, st>>>(W, H, in, wt, out, done);
+  };
 #define HG_CONV(CI, CO)                                                                  \
   if (cin == CI && cout == CO) {                                                         \
     if (relu)                                                                            \
-      KConvMfma<CI, CO, true><<<grid, 256, 0, st>>>(W, H, in, wt, out, done);            \
+      launch(KConvMfma<CI, CO, true, 4>, KConvMfma<CI, CO, true, 2>,                     \
+             KConvMfma<CI, CO, true, 1>);                                                \
     else                                                                                 \
-      KConvMfma<CI, CO, false><<<grid, 256, 0, st>>>(W, H, in, wt, out, done);           \
+      launch(KConvMfma<CI, CO, false, 4>, KConvMfma<CI, CO, false, 2>,                   \
+             KConvMfma<CI, CO, false, 1>);                                               \
     return;                                                                              \
   }
   HG_CONV(16, 32) HG_CONV(32, 64) HG_CONV(64, 64) HG_CONV(64, 32) HG_CONV(32, 16)

@@ -134,7 +134,8 @@ def test_gradient_matches_oracle(nets, weights, mode):
 # more tiles than blocks.  The linear network and its bound (the number model's
 # own distance from FP64), which holds at any size: with ReLU the distance from
 # the model grows with the pixels at which a rounding flips the mask.
-@pytest.mark.parametrize("nx,ny", [(16, 16), (72, 24), (136, 40), (16, 264), (584, 272)])
+@pytest.mark.parametrize("nx,ny", [(16, 16), (72, 24), (136, 40), (16, 264), (584, 272),
+                                   (1040, 520)])
 def test_gradient_any_size(gpu, weights, nx, ny):
     rng = np.random.default_rng(nx)
     x = rng.normal(size=(ny, nx))
