@@ -204,6 +204,8 @@ struct hg_ctx {
   // workspace of the gauss_seidel solves (a context with one of them)
   double* sor_ws = nullptr;
   long sor_doubles = 0;
+  double* lu_ws = nullptr;  // lu: LaunchLuWavefront's workspace
+  long lu_doubles = 0;
   hg::JacobiWork jw{};
   double* jdiff_host_dummy = nullptr;
   // pinned host mirrors
@@ -446,7 +448,7 @@ void HeatStep(hg_ctx* c) {
   switch (cfg.linear_solver_heat) {
     case HG_SOLVER_LU:
       hg::LaunchLuWavefront(c->st, nx, ny, rows, c->k0, nullptr, c->x0, nullptr, c->t_a,
-                            nullptr, c->t_b, nullptr);
+                            nullptr, c->t_b, nullptr, c->lu_ws, c->lu_doubles);
       break;
     case HG_SOLVER_LU_RB:
       // the red-black sweep takes two right-hand sides: the second is a copy
@@ -700,7 +702,7 @@ void SolveVelocity(hg_ctx* c, hg::Rows rows, hg_iter_stats* is) {
   switch (cfg.linear_solver_velocity) {
     case HG_SOLVER_LU:
       hg::LaunchLuWavefront(c->st, nx, ny, rows, c->k0, c->k1, c->x0, c->x1, c->u_ip[0],
-                            c->u_ip[1], c->u_ic[0], c->u_ic[1]);
+                            c->u_ip[1], c->u_ic[0], c->u_ic[1], c->lu_ws, c->lu_doubles);
       is->velocity_solve_iters[0] = is->velocity_solve_iters[1] = 0;
       break;
     case HG_SOLVER_LU_RB:
@@ -748,7 +750,7 @@ void SolvePressure(hg_ctx* c, hg_iter_stats* is) {
     }
     case HG_SOLVER_LU:
       hg::LaunchLuWavefront(c->st, nx, ny, rows, c->Pk, nullptr, c->pcorr, nullptr, nullptr,
-                            nullptr, nullptr, nullptr);
+                            nullptr, nullptr, nullptr, c->lu_ws, c->lu_doubles);
       is->pressure_solve_iters = 0;
       break;
     case HG_SOLVER_LU_RB:
@@ -1171,6 +1173,11 @@ hg_status hg_create(const hg_config* cfg_in, hg_ctx** out) {
         (cfg.heat_enable && cfg.linear_solver_heat == HG_SOLVER_GAUSS_SEIDEL)) {
       c->sor_doubles = hg::SorWorkspace(cfg.nx, cfg.ny);
       if (c->sor_doubles > 0) c->sor_ws = c->Alloc(c->sor_doubles);
+    }
+    if (cfg.linear_solver_pressure == HG_SOLVER_LU || cfg.linear_solver_velocity == HG_SOLVER_LU ||
+        (cfg.heat_enable && cfg.linear_solver_heat == HG_SOLVER_LU)) {
+      c->lu_doubles = hg::LuWorkspace(cfg.nx, cfg.ny);
+      if (c->lu_doubles > 0) c->lu_ws = c->Alloc(c->lu_doubles);
     }
     c->jw.xa = c->Alloc(nc);
     c->jw.xb = c->Alloc(nc);

@@ -171,9 +171,14 @@ using RowsF = RowsT<float>;
 // Exact-order symmetric Gauss-Seidel sweep from zero (linear.hpp:527-567) for
 // up to two right-hand sides sharing the coefficients, in one workgroup.
 // x_out[r] = base[r] + x[r] when base != nullptr (the delta-form update).
+// ws: a workspace of ws_doubles doubles for the rows of one step side by side
+// (LuWorkspace; 7 per cell are enough for one right-hand side).  Without it, or
+// where the shorter side exceeds 1024, the rows are read in place.
+long LuWorkspace(int nx, int ny);
 void LaunchLuWavefront(hipStream_t st, int nx, int ny, Rows a, const double* k0,
                        const double* k1, double* x0, double* x1, const double* base0,
-                       const double* base1, double* out0, double* out1);
+                       const double* base1, double* out0, double* out1, double* ws,
+                       long ws_doubles);
 // Exact-order lexicographic SOR from zero (linear.hpp:685-715), all sweeps in
 // one persistent workgroup.  info[0] = iterations (reference count),
 // info[1] = final max|corr| (as double bits).

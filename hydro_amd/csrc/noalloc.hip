@@ -118,7 +118,7 @@ hg_status hg_stencil_solve_noalloc(int32_t nx, int32_t ny, const double* s, cons
   switch (solver) {
     case HG_SOLVER_LU:
       hg::LaunchLuWavefront(st, nx, ny, rows, k, nullptr, x, nullptr, nullptr, nullptr, nullptr,
-                            nullptr);
+                            nullptr, a0, long((kScratchBytes - off_arr) / 8));
       break;
     case HG_SOLVER_LU_RB:
       // one right-hand side: the second lane solves it again into a3; the

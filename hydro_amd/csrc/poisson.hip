@@ -74,7 +74,7 @@ hg_status hg_stencil_solve(int32_t nx, int32_t ny, const double* s, const double
     std::unique_ptr<void, std::function<void(void*)>> guard(
         (void*)st, [](void* p) { (void)hipStreamDestroy((hipStream_t)p); });
     DevBuf ds(N), dw(N), dc(N), de(N), dn(N), dk(N), dx(N), dx2(N), dz(N), dout(N), dtmp(N);
-    std::unique_ptr<DevBuf> sor_ws;
+    std::unique_ptr<DevBuf> row_ws;
     DevBuf info(2), jdiff(size_t(std::max(opts->max_iters, 0)) + 2), jstate(2);
     const double* src[6] = {s, w, c, e, n, k};
     double* dst[6] = {ds.p, dw.p, dc.p, de.p, dn.p, dk.p};
@@ -90,21 +90,24 @@ hg_status hg_stencil_solve(int32_t nx, int32_t ny, const double* s, const double
     double diff = 0.;
     const double* result = dx.p;
     switch (opts->solver) {
-      case HG_SOLVER_LU:
+      case HG_SOLVER_LU: {
+        const long nws = hg::LuWorkspace(nx, ny);
+        row_ws.reset(new DevBuf(size_t(std::max(nws, 1L))));
         hg::LaunchLuWavefront(st, nx, ny, rows, dk.p, nullptr, dx.p, nullptr, nullptr, nullptr,
-                              nullptr, nullptr);
+                              nullptr, nullptr, row_ws->p, nws);
         break;
+      }
       case HG_SOLVER_LU_RB:
         hg::LaunchLuRb(st, nx, ny, rows, dk.p, dk.p, dx.p, dx2.p, dz.p, dz.p, dout.p, dtmp.p);
         result = dout.p;
         break;
       case HG_SOLVER_GAUSS_SEIDEL: {
         const long nws = hg::SorWorkspace(nx, ny);
-        sor_ws.reset(new DevBuf(size_t(nws)));
+        row_ws.reset(new DevBuf(size_t(nws)));
         unsigned long long h[2];
         for (bool retry : {false, true}) {
           hg::LaunchSor(st, nx, ny, rows, dk.p, dx.p, opts->tolerance, opts->max_iters,
-                        opts->relaxation_factor, (unsigned long long*)info.p, sor_ws->p, nws,
+                        opts->relaxation_factor, (unsigned long long*)info.p, row_ws->p, nws,
                         retry);
           HG_CHECK(hipMemcpyAsync(h, info.p, 16, hipMemcpyDeviceToHost, st));
           HG_CHECK(hipStreamSynchronize(st));

@@ -11,6 +11,7 @@
 // result equals the serial sweep bit for bit.  Compiled with
 // -ffp-contract=off.
 
+#include <algorithm>
 #include <type_traits>
 
 #include "kernels.h"
@@ -181,6 +182,228 @@ KLuWavefront(int nx, int ny, Rows a, const double* __restrict__ k0,
     double* oo[2] = {out0, out1};
     for (int r = t; r < nx * ny; r += T)
       for (int q = 0; q < NR; ++q) oo[q][r] = bb[q][r] + xx[q][r];
+  }
+}
+
+// ---- the symmetric sweep on skewed rows ----------------------------------------
+// The same sweep with the operands of one step contiguous.  Let a be the shorter
+// and b the longer side, t a cell's index along the short side and m along the
+// long one.  Cell (t, m) is computed at step t + m by thread t and lies in row
+// (t + m) mod b at column t (a b entries); KLuPack writes the coefficients so,
+// with 0 for neighbours outside the grid, and KLuUnpack takes the result back.
+// (Read in place the 64 lanes of a wave are on 64 rows and every load touches 64
+// cache lines.)
+//
+// A step is a chain: the value crosses to the next thread, two products, three
+// sums and a division.  Within a wave it crosses by a lane shift.  Between
+// waves it goes through LDS a group of kG steps at a time: wave w is w groups
+// behind the first, so there is one barrier per group.  Operands are loaded kG
+// steps ahead.  The backward half mirrors all of it.  Threads outside the grid
+// compute along and store nothing; a cell whose neighbour is outside takes +0
+// for it, as the sum of the in-place kernel, which starts at +0, does.
+//
+// Two right-hand sides, this and the in-place kernel: 64x64 45 | 108 us, 16x16
+// 13 | 30, 256x128 160 | 505; one, with the call around it: 333x217 241 | 592,
+// 500x300 412 | 1701.  KLuPack and KLuUnpack take 9 us of launches more.
+template <int NR>
+__global__ void __launch_bounds__(256)
+KLuPack(int nx, int ny, Rows r, const double* __restrict__ k0, const double* __restrict__ k1,
+        int tr, double2* __restrict__ sw, double2* __restrict__ en, double2* __restrict__ ck,
+        double* __restrict__ kb) {
+  const int a = tr ? ny : nx, b = tr ? nx : ny;
+  const int d = blockIdx.x * 256 + threadIdx.x;  // skewed index, so that stores coalesce
+  if (d >= a * b) return;
+  const int t = d % a, row = d / a;
+  const int m = row >= t ? row - t : row - t + b;  // t < a <= b
+  const int i = tr ? m : t, j = tr ? t : m;
+  const int c = i + nx * j;
+  sw[d] = double2{j > 0 ? r.s[c] : 0., i > 0 ? r.w[c] : 0.};
+  en[d] = double2{i < nx - 1 ? r.e[c] : 0., j < ny - 1 ? r.n[c] : 0.};
+  ck[d] = double2{r.c[c], k0[c]};
+  if (NR == 2) kb[d] = k1[c];
+}
+
+template <int NR>
+__global__ void __launch_bounds__(256)
+KLuUnpack(int nx, int ny, int tr, const double* __restrict__ v, double* __restrict__ x0,
+          double* __restrict__ x1, const double* __restrict__ base0,
+          const double* __restrict__ base1, double* __restrict__ out0,
+          double* __restrict__ out1) {
+  const int c = blockIdx.x * 256 + threadIdx.x;
+  if (c >= nx * ny) return;
+  const int a = tr ? ny : nx, b = tr ? nx : ny;
+  const int i = c % nx, j = c / nx;
+  const int t = tr ? j : i, m = tr ? i : j;
+  const int row = t + m >= b ? t + m - b : t + m;
+  const double* const p = v + (long(row) * a + t) * NR;
+  const double v0 = p[0], v1 = NR == 2 ? p[1] : 0.;
+  x0[c] = v0;
+  if (NR == 2) x1[c] = v1;
+  if (base0) {
+    out0[c] = base0[c] + v0;
+    if (NR == 2) out1[c] = base1[c] + v1;
+  }
+}
+
+// The value of the lane before (SHR) or after, `edge` in the first / last lane.
+template <bool SHR>
+__device__ __forceinline__ double LaneNext(double v, double edge) {
+  constexpr int kCtrl = SHR ? 0x138 : 0x130;  // wave_shr:1, wave_shl:1
+  return __hiloint2double(
+      __builtin_amdgcn_update_dpp(__double2hiint(edge), __double2hiint(v), kCtrl, 0xf, 0xf, false),
+      __builtin_amdgcn_update_dpp(__double2loint(edge), __double2loint(v), kCtrl, 0xf, 0xf,
+                                  false));
+}
+
+template <int NR, bool TR, int MAXT>
+__global__ void __launch_bounds__(MAXT)
+KLuSkew(int a, int b, const double2* __restrict__ sw, const double2* __restrict__ en,
+        const double2* __restrict__ ck, const double* __restrict__ kb, double* v) {
+  constexpr int kG = MAXT > 512 ? 4 : 8;  // steps per group (registers)
+  constexpr bool kOneWave = MAXT == 64;
+  __shared__ double edge[MAXT / 64][4 * kG][NR];  // values of a wave's border lane, by step
+  const int t = threadIdx.x, lane = t & 63, nw = kOneWave ? 1 : blockDim.x >> 6;
+  const int wave = kOneWave ? 0 : __builtin_amdgcn_readfirstlane(t >> 6);
+  const int tc = min(t, a - 1);
+  const int steps = a + b - 1, ng = (steps + kG - 1) / kG;
+  double val[NR], e[kG][NR], done[kG][NR];
+  // A group: the values of the group before are stored, the operands of the
+  // next loaded, and the steps run on registers, so that what a wait at the
+  // next group's start is for was issued a group ago.
+  auto Run = [&](auto& A, auto& B, auto&& group, int before, int after) {
+    if (!kOneWave)
+      for (int k = 0; k < before; ++k) LdsBarrier();
+    for (int g = 0; g < ng; g += 2) {
+      group(A, B, g);
+      if (!kOneWave) LdsBarrier();
+      if (g + 1 < ng) group(B, A, g + 1);
+      if (!kOneWave) LdsBarrier();
+    }
+    if (!kOneWave)
+      for (int k = 0; k < after; ++k) LdsBarrier();
+  };
+  auto Edges = [&](int other, int first) {  // steps first - 1 .. of wave `other`
+#pragma unroll
+    for (int i = 0; i < kG; ++i)
+#pragma unroll
+      for (int q = 0; q < NR; ++q)
+        e[i][q] = kOneWave || other < 0 || other >= nw
+                      ? 0.
+                      : edge[other][(first + i - 1) & (4 * kG - 1)][q];
+  };
+  auto PutEdges = [&](int border, int first) {
+    if (!kOneWave && lane == border)
+#pragma unroll
+      for (int i = 0; i < kG; ++i)
+#pragma unroll
+        for (int q = 0; q < NR; ++q) edge[wave][(first + i) & (4 * kG - 1)][q] = done[i][q];
+  };
+#pragma unroll
+  for (int q = 0; q < NR; ++q) val[q] = 0.;
+  // ---- forward: x = (-k - (s x_S + w x_W)) / c
+  {
+    struct Row {
+      double2 sw, ck;
+      double kb;
+    } A[kG], B[kG];
+    int next = 0, row = 0;  // rows of the next load and of the next store
+    auto Load = [&](Row (&o)[kG]) {
+#pragma unroll
+      for (int i = 0; i < kG; ++i) {
+        const long d = long(next) * a + tc;
+        o[i].sw = sw[d];
+        o[i].ck = ck[d];
+        if (NR == 2) o[i].kb = kb[d];
+        next = next + 1 == b ? 0 : next + 1;
+      }
+    };
+    auto Store = [&](int g) {
+#pragma unroll
+      for (int i = 0; i < kG; ++i) {
+        const int m = g * kG + i - t;
+        if (m >= 0 && m < b && t < a)
+#pragma unroll
+          for (int q = 0; q < NR; ++q) v[(long(row) * a + t) * NR + q] = done[i][q];
+        row = row + 1 == b ? 0 : row + 1;
+      }
+    };
+    auto Group = [&](Row (&o)[kG], Row (&o_next)[kG], int g) {
+      if (g > 0) Store(g - 1);
+      Load(o_next);
+      Edges(wave - 1, g * kG);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < kG; ++i) {
+        const int m = g * kG + i - t;
+#pragma unroll
+        for (int q = 0; q < NR; ++q) {
+          const double own = m == 0 ? 0. : val[q];
+          const double cross = LaneNext<true>(val[q], e[i][q]);
+          double sum = 0;
+          sum += o[i].sw.x * (TR ? cross : own);
+          sum += o[i].sw.y * (TR ? own : cross);
+          done[i][q] = val[q] = (-(q == 0 ? o[i].ck.y : o[i].kb) - sum) / o[i].ck.x;
+        }
+      }
+      PutEdges(63, g * kG);
+    };
+    Load(A);
+    Run(A, B, Group, wave, nw - 1 - wave);
+    Store(ng - 1);
+  }
+  __syncthreads();
+  // ---- backward: x -= (n x_N + e x_E) / c, from the last step to the first
+  {
+    struct Row {
+      double2 en;
+      double c, v[NR];
+    } A[kG], B[kG];
+    int next = a > 1 ? a - 2 : b - 1, row = next;  // (a + b - 2) mod b
+    auto Load = [&](Row (&o)[kG]) {
+#pragma unroll
+      for (int i = 0; i < kG; ++i) {
+        const long d = long(next) * a + tc;
+        o[i].en = en[d];
+        o[i].c = ck[d].x;
+#pragma unroll
+        for (int q = 0; q < NR; ++q) o[i].v[q] = v[d * NR + q];
+        next = next == 0 ? b - 1 : next - 1;
+      }
+    };
+    auto Store = [&](int g) {
+#pragma unroll
+      for (int i = 0; i < kG; ++i) {
+        const int m = steps - 1 - (g * kG + i) - t;
+        if (m >= 0 && m < b && t < a)
+#pragma unroll
+          for (int q = 0; q < NR; ++q) v[(long(row) * a + t) * NR + q] = done[i][q];
+        row = row == 0 ? b - 1 : row - 1;
+      }
+    };
+    auto Group = [&](Row (&o)[kG], Row (&o_next)[kG], int g) {
+      if (g > 0) Store(g - 1);
+      Load(o_next);
+      Edges(wave + 1, g * kG);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < kG; ++i) {
+        const int m = steps - 1 - (g * kG + i) - t;
+#pragma unroll
+        for (int q = 0; q < NR; ++q) {
+          const double own = m == b - 1 ? 0. : val[q];
+          const double next_lane = LaneNext<false>(val[q], e[i][q]);
+          const double cross = t == a - 1 ? 0. : next_lane;
+          double sum = 0;
+          sum += o[i].en.y * (TR ? cross : own);
+          sum += o[i].en.x * (TR ? own : cross);
+          done[i][q] = val[q] = o[i].v[q] - sum / o[i].c;
+        }
+      }
+      PutEdges(0, g * kG);
+    };
+    Load(A);
+    Run(A, B, Group, nw - 1 - wave, wave);
+    Store(ng - 1);
   }
 }
 
@@ -570,9 +793,42 @@ KLuRbRed(int nx, int ny, RowsT<T> a, const T* __restrict__ k0, const T* __restri
 
 }  // namespace
 
+long LuWorkspace(int nx, int ny) {
+  return std::min(nx, ny) <= kMaxThreads ? 9L * nx * ny : 0;
+}
+
 void LaunchLuWavefront(hipStream_t st, int nx, int ny, Rows a, const double* k0,
                        const double* k1, double* x0, double* x1, const double* base0,
-                       const double* base1, double* out0, double* out1) {
+                       const double* base1, double* out0, double* out1, double* ws,
+                       long ws_doubles) {
+  const int sa = std::min(nx, ny), sb = std::max(nx, ny);
+  const long n = long(nx) * ny;
+  if (sa <= kMaxThreads && ws && ws_doubles >= (k1 ? 9 : 7) * n) {
+    double2* sw = reinterpret_cast<double2*>(ws);
+    double2 *en = sw + n, *ck = en + n;
+    double* v = reinterpret_cast<double*>(ck + n);
+    double* kb = v + 2 * n;
+    const int tr = ny < nx ? 1 : 0;
+    const unsigned grid = unsigned((n + 255) / 256);
+    const int threads = (sa + 63) / 64 * 64;
+    auto run = [&](auto nr) {
+      constexpr int NR = decltype(nr)::value;
+      KLuPack<NR><<<grid, 256, 0, st>>>(nx, ny, a, k0, k1, tr, sw, en, ck, kb);
+      auto launch = [&](auto kernel) { kernel<<<1, threads, 0, st>>>(sa, sb, sw, en, ck, kb, v); };
+      if (threads <= 64)
+        launch(tr ? KLuSkew<NR, true, 64> : KLuSkew<NR, false, 64>);
+      else if (threads <= 512)
+        launch(tr ? KLuSkew<NR, true, 512> : KLuSkew<NR, false, 512>);
+      else
+        launch(tr ? KLuSkew<NR, true, 1024> : KLuSkew<NR, false, 1024>);
+      KLuUnpack<NR><<<grid, 256, 0, st>>>(nx, ny, tr, v, x0, x1, base0, base1, out0, out1);
+    };
+    if (k1)
+      run(std::integral_constant<int, 2>{});
+    else
+      run(std::integral_constant<int, 1>{});
+    return;
+  }
   int cw;
   int T = ThreadsFor(nx, &cw);
   auto launch = [&](auto nr, auto cwc) {
