@@ -88,7 +88,7 @@ template <int NQ>
 __device__ __forceinline__ void PutPartials(const double (&v)[NQ], double* part) {
   __shared__ double red[NQ][kB / 64];
   for (int q = 0; q < NQ; ++q) {
-    const double s = WaveSum(v[q]);
+    const double s = WaveTotal(v[q]);
     if ((threadIdx.x & 63) == 0) red[q][threadIdx.x >> 6] = s;
   }
   __syncthreads();
@@ -124,7 +124,7 @@ __device__ __forceinline__ double Fold(const double* part, int n) {
   __shared__ double red[kB / 64];
   __shared__ double tot;
   double s = StridedSum<8>(part, n, threadIdx.x, kB);
-  s = WaveSum(s);
+  s = WaveTotal(s);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
   __syncthreads();
   if (threadIdx.x == 0) {
@@ -149,7 +149,7 @@ __device__ __forceinline__ void FoldN(const double* const (&part)[NQ], const int
   for (int q = 0; q < NQ; ++q) s[q] = StridedSum<8>(part[q], n[q], threadIdx.x, kB);
 #pragma unroll
   for (int q = 0; q < NQ; ++q) {
-    const double v = WaveSum(s[q]);
+    const double v = WaveTotal(s[q]);
     if ((threadIdx.x & 63) == 0) red[q][threadIdx.x >> 6] = v;
   }
   __syncthreads();
@@ -329,33 +329,6 @@ __device__ __forceinline__ double FromWords(Word lo, Word hi) {
   return __hiloint2double(int(unsigned(hi)), int(unsigned(lo)));
 }
 
-// Sum over the lanes of each row of 16 in its last lane (R = 4 steps), over
-// the wave in lane 63 (R = 6), in a fixed order.
-template <int R>
-__device__ __forceinline__ double DppSum(double v) {
-  auto Step = [&](auto ctrl, auto rows) {
-    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), ctrl.value, rows.value, 0xf,
-                                               true);
-    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), ctrl.value, rows.value, 0xf,
-                                               true);
-    v += __hiloint2double(hi, lo);
-  };
-  using std::integral_constant;
-  Step(integral_constant<int, 0x111>{}, integral_constant<int, 0xf>{});  // row_shr:1
-  Step(integral_constant<int, 0x112>{}, integral_constant<int, 0xf>{});
-  Step(integral_constant<int, 0x114>{}, integral_constant<int, 0xf>{});
-  Step(integral_constant<int, 0x118>{}, integral_constant<int, 0xf>{});
-  if constexpr (R == 6) {
-    Step(integral_constant<int, 0x142>{}, integral_constant<int, 0xa>{});  // row_bcast:15
-    Step(integral_constant<int, 0x143>{}, integral_constant<int, 0xc>{});  // row_bcast:31
-  }
-  return v;
-}
-__device__ __forceinline__ double LaneOf(double v, int lane) {
-  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
-                          __builtin_amdgcn_readlane(__double2loint(v), lane));
-}
-
 // Sums v over all workgroups, in a fixed order; `extra` = post(sums), formed
 // in one wave.  Words of a parity are written again two exchanges later, when
 // every workgroup has read them.  `others` runs in the other waves while the
@@ -405,7 +378,7 @@ __device__ __forceinline__ bool Exchange(double (&v)[NV], double& extra, unsigne
       }
 #pragma unroll
       for (int q = 0; q < NV; ++q)
-        v[q] = LaneOf(DppSum<6>(lane < W ? FromWords(g[2 * q], g[2 * q + 1]) : 0.), 63);
+        v[q] = WaveTotal(lane < W ? FromWords(g[2 * q], g[2 * q + 1]) : 0.);
     }
     const double e = post(v);
     if (lane == 0) {
@@ -818,7 +791,7 @@ __device__ __forceinline__ bool WideFold(const double* const (&part)[NQ], const 
   if (stopped) return false;
 #pragma unroll
   for (int q = 0; q < NQ; ++q) {
-    s[q] = WaveSum(s[q]);
+    s[q] = WaveTotal(s[q]);
     if ((threadIdx.x & 63) == 0) red[q][threadIdx.x >> 6] = s[q];
   }
   __syncthreads();

@@ -122,6 +122,48 @@ __device__ __forceinline__ double WaveSum(double v) {
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
   return v;
 }
+
+// v shifted between lanes by the data-parallel move `kCtrl` into the rows of 16
+// lanes in the mask kRows, 0 elsewhere and where a lane has no source.
+template <int kCtrl, int kRows>
+__device__ __forceinline__ float DppMove(float v) {
+  return __int_as_float(
+      __builtin_amdgcn_update_dpp(0, __float_as_int(v), kCtrl, kRows, 0xf, true));
+}
+template <int kCtrl, int kRows>
+__device__ __forceinline__ double DppMove(double v) {
+  return __hiloint2double(
+      __builtin_amdgcn_update_dpp(0, __double2hiint(v), kCtrl, kRows, 0xf, true),
+      __builtin_amdgcn_update_dpp(0, __double2loint(v), kCtrl, kRows, 0xf, true));
+}
+// Sum over the lanes of each row of 16 in its last lane (R = 4 steps), over
+// the wave in lane 63 (R = 6), in a fixed order.  Lane shifts take a tenth of
+// the latency of WaveSum's shuffles through LDS.
+template <int R, class M>
+__device__ __forceinline__ M DppSum(M v) {
+  v += DppMove<0x111, 0xf>(v);  // row_shr:1, 2, 4, 8
+  v += DppMove<0x112, 0xf>(v);
+  v += DppMove<0x114, 0xf>(v);
+  v += DppMove<0x118, 0xf>(v);
+  if constexpr (R == 6) {
+    v += DppMove<0x142, 0xa>(v);  // row_bcast:15, 31
+    v += DppMove<0x143, 0xc>(v);
+  }
+  return v;
+}
+__device__ __forceinline__ float LaneOf(float v, int lane) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
+}
+__device__ __forceinline__ double LaneOf(double v, int lane) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                          __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+// Sum over a wave whose lanes are all active, the same in every lane.
+template <class M>
+__device__ __forceinline__ M WaveTotal(M v) {
+  return LaneOf(DppSum<6>(v), 63);
+}
+
 __device__ __forceinline__ double WaveMax(double v) {
   for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
   return v;

@@ -44,7 +44,7 @@ __device__ __forceinline__ void FcgStopTest(const FcgFusion& f) {
   __shared__ double red[4];
   double s = 0.;
   for (int b = threadIdx.x; b < f.nb; b += 256) s += f.rr_part[b];
-  s = WaveSum(s);
+  s = WaveTotal(s);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
   __syncthreads();
   if (threadIdx.x == 0) {

@@ -15,6 +15,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
 #include <vector>
 
 #include "learned.h"
@@ -23,7 +24,7 @@
 namespace hg {
 
 constexpr int kTallY = 16;  // tile height of the finest level's fused kernels
-constexpr int kMidY = 4;    // tile height of the coarser levels' fused kernels
+constexpr int kMidY = 4;    // of the coarser levels', and of a small finest level's
 
 // A level's arrays, in the level type M (float: the V-cycle of the mixed
 // path; double: the same cycle in FP64, for comparison).
@@ -33,7 +34,6 @@ struct MgLevelT {
   M lx, ly;       // distance ratio of the last inner face to the finer level's, in x and y
   TileGrid tg;    // 64 x 4 tiles
   TileGrid mid;   // 64 x kMidY tiles
-  TileGrid tall;  // 64 x kTallY tiles
   M *kx = nullptr, *ky = nullptr, *dinv = nullptr;
   M *r = nullptr, *xa = nullptr, *xb = nullptr;
 };
@@ -86,7 +86,7 @@ class MgPrecondT : public Precond {
   // and its direction dots in the finest level's last kernel.
   bool ApplyFcg(const double* r, float* z, hipStream_t st, const int* d_done,
                 const FcgFusion& f, int* ndir) override;
-  int FcgPartials() const override { return lv_.size() > 1 ? lv_[0].tall.blocks() : 0; }
+  int FcgPartials() const override { return lv_.size() > 1 ? fine_.blocks() : 0; }
   // level 1 runs a tiled down-leg (its first kernel takes the stop test)
   bool FusesUpdate() const override {
     return lv_.size() >= 3 && !(use_coarse_kernel && first_in_kernel_ == 1);
@@ -123,6 +123,15 @@ class MgPrecondT : public Precond {
  private:
   std::vector<MgLevelT<M>> lv_;
   int first_in_kernel_ = -1;
+  TileGrid fine_;  // the finest level's tiles: 64 x kTallY or 64 x kMidY
+  bool tall_;
+  template <class F>
+  void WithFineTile(F&& f) {  // f(the tile height as a constant)
+    if (tall_)
+      f(std::integral_constant<int, kTallY>{});
+    else
+      f(std::integral_constant<int, kMidY>{});
+  }
   // a device flag that stays 0: the stop flag of cycles run without one, so
   // that the kernels always read a flag (no null test ahead of their loads)
   int* never_done_ = nullptr;

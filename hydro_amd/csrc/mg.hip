@@ -20,7 +20,16 @@ namespace {
 
 constexpr int kTinyMax = 64;          // coarsest grid, solved by one wave
 constexpr int kCoarsestMax = kTinyMax;
-constexpr int kInKernelMax = 2048;    // levels handled by the one-workgroup cycle
+// levels handled by the one-workgroup cycle (4096 and 8192 cells, two or four
+// more launches saved, measured 1 and 2 us per cycle slower at 512 x 512: one
+// CU is then what takes the time)
+constexpr int kInKernelMax = 2048;
+// Tall tiles re-read less halo, but a thread has five cells to work through one
+// after another, which is what a grid of few tiles waits for.
+// Per flexible CG iteration, tall | low tiles: 64x64 42 | 38 us, 300x180 64 |
+// 58, 512x512 (256 tall tiles) 74 | 72, 512x1024 (512) 87 | 87, 1024x1024 106 |
+// 112, 1024x2048 142 | 155.
+constexpr int kTallBlocks = 512;
 // Jacobi-PCG iterations on the coarsest grid: a partial solve.  The V-cycle
 // is applied inside flexible CG, which tolerates the inexact coarse solve;
 // on the 4x8 coarsest grid of the 1024x2048 hierarchy 8 iterations leave the
@@ -296,7 +305,7 @@ __device__ __forceinline__ void FoldedUpdate(const FcgFusion& f, const SlotCell<
     }
   }
   __shared__ double red[kTileThreads / 64];
-  rr = WaveSum(rr);
+  rr = WaveTotal(rr);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = rr;
   __syncthreads();
   if (threadIdx.x == 0) {
@@ -519,8 +528,8 @@ KUp(int nx, int ny, TileGrid tg, const M* __restrict__ kx, const M* __restrict__
   }
   if (dots) {  // block partials of (z, q_old) and (r, z)
     __shared__ double red[2][kTileThreads / 64];
-    zq = WaveSum(zq);
-    rz = WaveSum(rz);
+    zq = WaveTotal(zq);
+    rz = WaveTotal(rz);
     if ((threadIdx.x & 63) == 0) {
       red[0][threadIdx.x >> 6] = zq;
       red[1][threadIdx.x >> 6] = rz;
@@ -580,12 +589,6 @@ KCoarsest(int nx, int ny, const M* __restrict__ kx, const M* __restrict__ ky,
   if (act) out[c] = xs[cur][c];
 }
 
-template <class M>
-__device__ __forceinline__ M WaveSumF(M v) {
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
-}
-
 __device__ __forceinline__ void BlockSync() {
   __threadfence_block();
   __syncthreads();
@@ -610,25 +613,25 @@ constexpr int CcLevels() {
   return l;
 }
 constexpr int kCcLevels = CcLevels();  // smoothed (non-coarsest) levels at most
-constexpr int kCcSlots = CcSlots(0);
-static_assert(kInKernelMax % kCcThreads == 0 || kInKernelMax < kCcThreads, "slots");
 
 template <class M>
 __global__ void __launch_bounds__(kCcThreads)
 KCoarseCycle(CoarseSetT<M> cs, SweepWeights w, const int* done) {
   const int stopped = *done;  // tested once the loads are in flight; never null
-  __shared__ M sxa[kLdsCells], sxb[kLdsCells], sr[kLdsCells];
+  constexpr int kCcSlots = CcSlots(0), kLevels = kCcLevels;
+  __shared__ M sxa[kLdsCells], sxb[kLdsCells];
   const int t = threadIdx.x;
   const int nlev = cs.count - 1;
   // per owned cell: faces w e s n, inverse diagonal, prolongation weights
-  M kw[kCcLevels][kCcSlots], ke[kCcLevels][kCcSlots], ks[kCcLevels][kCcSlots],
-      kn[kCcLevels][kCcSlots], di[kCcLevels][kCcSlots], wx[kCcLevels][kCcSlots],
-      wy[kCcLevels][kCcSlots];
+  M kw[kLevels][kCcSlots], ke[kLevels][kCcSlots], ks[kLevels][kCcSlots],
+      kn[kLevels][kCcSlots], di[kLevels][kCcSlots], wx[kLevels][kCcSlots],
+      wy[kLevels][kCcSlots];
   // and its position, i in the low and j in the high 16 bits (the phases
   // would otherwise divide by the level's width in every sweep)
-  int ij[kCcLevels][kCcSlots];
+  int ij[kLevels][kCcSlots];
+  M rv[kLevels][kCcSlots], rT = 0.f;  // right-hand sides; the coarsest level's
 #pragma unroll
-  for (int l = 0; l < kCcLevels; ++l) {
+  for (int l = 0; l < kLevels; ++l) {
 #pragma unroll
     for (int m = 0; m < CcSlots(l); ++m) {
       kw[l][m] = ke[l][m] = ks[l][m] = kn[l][m] = di[l][m] = wx[l][m] = wy[l][m] = 0.f;
@@ -676,9 +679,9 @@ KCoarseCycle(CoarseSetT<M> cs, SweepWeights w, const int* done) {
 #pragma unroll
   for (int m = 0; m < kCcSlots; ++m) {
     const int c = t + m * kCcThreads;
-    if (c < n0) sr[c] = cs.r[0][c];
+    rv[0][m] = c < n0 ? cs.r[0][c] : M(0);
   }
-  __syncthreads();
+  if (nlev == 0) rT = rv[0][0];
   // (A x) of owned cell (l, m) at (i, j) from LDS values x (level-local)
   auto Apply = [&](const M* x, int l, int m, int nx, int ny, int c, int i, int j) {
     M v = (((kw[l][m] + ke[l][m]) + ks[l][m]) + kn[l][m]) * x[c];
@@ -698,10 +701,9 @@ KCoarseCycle(CoarseSetT<M> cs, SweepWeights w, const int* done) {
   };
   // ---- down: kSweeps sweeps from zero, residual, restriction (sum of children)
 #pragma unroll
-  for (int l = 0; l < kCcLevels; ++l) {
+  for (int l = 0; l < kLevels; ++l) {
     if (l >= nlev) break;
     const int nx = cs.nx[l], ny = cs.ny[l], n = nx * ny;
-    const M* r = sr + cs.off[l];
     M *xa = sxa + cs.off[l], *xb = sxb + cs.off[l];
 #pragma unroll
     for (int k = 0; k < kSweeps; ++k) {
@@ -711,9 +713,9 @@ KCoarseCycle(CoarseSetT<M> cs, SweepWeights w, const int* done) {
       for (int m = 0; m < CcSlots(l); ++m) {
         const int c = t + m * kCcThreads;
         if (c >= n) continue;
-        dst[c] = k == 0 ? w.w[0] * di[l][m] * r[c]
+        dst[c] = k == 0 ? w.w[0] * di[l][m] * rv[l][m]
                         : src[c] + w.w[k] * di[l][m] *
-                                       (r[c] - Apply(src, l, m, nx, ny, c, ij[l][m] & 0xffff,
+                                       (rv[l][m] - Apply(src, l, m, nx, ny, c, ij[l][m] & 0xffff,
                                                      ij[l][m] >> 16));
       }
       __syncthreads();
@@ -722,12 +724,14 @@ KCoarseCycle(CoarseSetT<M> cs, SweepWeights w, const int* done) {
 #pragma unroll
     for (int m = 0; m < CcSlots(l); ++m) {
       const int c = t + m * kCcThreads;
-      if (c < n) xa[c] = r[c] - Apply(xb, l, m, nx, ny, c, ij[l][m] & 0xffff, ij[l][m] >> 16);
+      if (c < n) xa[c] = rv[l][m] - Apply(xb, l, m, nx, ny, c, ij[l][m] & 0xffff, ij[l][m] >> 16);
     }
     __syncthreads();
     const int nxc = cs.nx[l + 1], nc = nxc * cs.ny[l + 1];
-    M* rc = sr + cs.off[l + 1];
-    for (int C = t; C < nc; C += kCcThreads) {
+#pragma unroll
+    for (int m = 0; m < CcSlots(l + 1); ++m) {
+      const int C = t + m * kCcThreads;
+      if (C >= nc) continue;
       const int I = C % nxc, J = C / nxc;
       M sum = 0.f;
 #pragma unroll
@@ -735,21 +739,23 @@ KCoarseCycle(CoarseSetT<M> cs, SweepWeights w, const int* done) {
         const int i = 2 * I + (q & 1), j = 2 * J + (q >> 1);
         sum += (i < nx && j < ny) ? xa[i + nx * j] : M(0);
       }
-      rc[C] = sum;
+      if (l + 1 == nlev)
+        rT = sum;
+      else if (l + 1 < kLevels)
+        rv[l + 1 < kLevels ? l + 1 : 0][m] = sum;
     }
     __syncthreads();
   }
   // ---- coarsest: Jacobi-PCG in wave 0, result into sxa
   if (t < 64) {
-    const M* r = sr + cs.off[nlev];
-    M b = actT ? r[t] : 0.f;
+    M b = actT ? rT : 0.f;
     const M dg = ((tw + te) + ts) + tn;
     // the face-form operator has the constants as null space: solve with the
     // right-hand side projected to zero mean (consistent system)
-    b -= WaveSumF(b) / M(nT);
+    b -= WaveTotal(b) / M(nT);
     if (!actT) b = 0.f;
     M x = 0.f, rr = b, z = tdi * rr, p = z;
-    M rz = WaveSumF(rr * z);
+    M rz = WaveTotal(rr * z);
     const M rz0 = rz;
     for (int it = 0; it < kTinyIters && rz > 1e-12f * rz0; ++it) {
       const M pw = __shfl(p, (t + 63) & 63, 64), pe = __shfl(p, (t + 1) & 63, 64);
@@ -761,17 +767,17 @@ KCoarseCycle(CoarseSetT<M> cs, SweepWeights w, const int* done) {
       if (jT > 0) ap -= ts * ps;
       if (jT < nyT - 1) ap -= tn * pn;
       if (!actT) ap = 0.f;
-      const M pap = WaveSumF(p * ap);
+      const M pap = WaveTotal(p * ap);
       if (!(pap > 0.f)) break;
       const M alpha = rz / pap;
       x += alpha * p;
       rr -= alpha * ap;
       z = tdi * rr;
-      const M rzn = WaveSumF(rr * z);
+      const M rzn = WaveTotal(rr * z);
       p = z + (rzn / rz) * p;
       rz = rzn;
     }
-    x -= WaveSumF(actT ? x : 0.f) / M(nT);
+    x -= WaveTotal(actT ? x : M(0)) / M(nT);
     if (actT) sxa[cs.off[nlev] + t] = x;
   }
   __syncthreads();
@@ -779,10 +785,9 @@ KCoarseCycle(CoarseSetT<M> cs, SweepWeights w, const int* done) {
   // thread reading and writing only its own cells), kSweeps sweeps; the
   // level's result in xa
 #pragma unroll
-  for (int l = kCcLevels - 1; l >= 0; --l) {
+  for (int l = kLevels - 1; l >= 0; --l) {
     if (l >= nlev) continue;
     const int nx = cs.nx[l], ny = cs.ny[l], n = nx * ny, nxc = cs.nx[l + 1];
-    const M* r = sr + cs.off[l];
     const M* e = sxa + cs.off[l + 1];
     M *xa = sxa + cs.off[l], *xb = sxb + cs.off[l];
     M* yb = Buf(xa, xb, -1, false);
@@ -810,7 +815,7 @@ KCoarseCycle(CoarseSetT<M> cs, SweepWeights w, const int* done) {
         const int c = t + m * kCcThreads;
         if (c < n)
           dst[c] = src[c] + w.w[k] * di[l][m] *
-                                (r[c] - Apply(src, l, m, nx, ny, c, ij[l][m] & 0xffff,
+                                (rv[l][m] - Apply(src, l, m, nx, ny, c, ij[l][m] & 0xffff,
                                               ij[l][m] >> 16));
       }
       __syncthreads();
@@ -848,6 +853,9 @@ MgPrecondT<M>::MgPrecondT(int nx, int ny, M* kx0, M* ky0, M* dinv0) {
   if (std::is_same<M, double>::value &&
       ((nx & 1) || (ny & 1) || long(nx) * ny <= kTinyMax || nx < 4 || ny < 4))
     throw std::runtime_error("MgPrecond64: a grid with an odd or tiny side is not supported");
+  fine_ = MakeTileGrid(nx, ny, kTallY);
+  tall_ = fine_.blocks() >= kTallBlocks;
+  if (!tall_) fine_ = MakeTileGrid(nx, ny, kMidY);
   int cx = nx, cy = ny;
   double rx = 1., ry = 1., lx = 0.5, ly = 0.5;
   while (true) {
@@ -858,7 +866,6 @@ MgPrecondT<M>::MgPrecondT(int nx, int ny, M* kx0, M* ky0, M* dinv0) {
     L.ly = M(ly);
     L.tg = MakeTileGrid(cx, cy);
     L.mid = MakeTileGrid(cx, cy, kMidY);
-    L.tall = MakeTileGrid(cx, cy, kTallY);
     long n = long(cx) * cy;
     if (lv_.empty()) {
       L.kx = kx0;
@@ -1002,22 +1009,27 @@ void MgPrecondT<M>::Cycle(int l, const double* r64, float* z, M* out, hipStream_
     return;
   }
   MgLevelT<M>& C = lv_[l + 1];
-  // level 0 (FP64 residual) on 64 x kTallY tiles, the FP32 levels on 64 x kMidY;
+  // level 0 (FP64 residual) on its own tiles, the FP32 levels on 64 x kMidY;
   // with the FCG update folded into level 0 its stop test moves to level 1
   const bool up = fz.up_on != 0;
-  if (l == 0 && up)
-    KDown<M, double, kTallY, kFineSweeps, true><<<L.tall.blocks(), kTileThreads, 0, st>>>(
-        L.nx, L.ny, L.tall, L.kx, L.ky, L.dinv, r64, fine_sweeps, L.xb, C.nx, C.ny,
-        C.r, done, fz, 0);
-  else if (l == 0)
-    KDown<M, double, kTallY, kFineSweeps><<<L.tall.blocks(), kTileThreads, 0, st>>>(
-        L.nx, L.ny, L.tall, L.kx, L.ky, L.dinv, r64, fine_sweeps, L.xb, C.nx, C.ny,
-        C.r, done, fz, fused);
-  else
-    KDown<M, M, kMidY, kSweeps><<<L.mid.blocks(), kTileThreads, 0, st>>>(L.nx, L.ny, L.mid, L.kx, L.ky, L.dinv,
-                                                       L.r, sweeps, L.xb, C.nx,
-                                                       C.ny, C.r, done, fz,
-                                                       (l == 1 && up) ? 1 : 0);
+  if (l == 0) {
+    WithFineTile([&](auto ty) {
+      constexpr int TY = decltype(ty)::value;
+      auto launch = [&](auto kernel) {
+        kernel<<<fine_.blocks(), kTileThreads, 0, st>>>(L.nx, L.ny, fine_, L.kx, L.ky, L.dinv, r64,
+                                                        fine_sweeps, L.xb, C.nx, C.ny, C.r, done,
+                                                        fz, up ? 0 : fused);
+      };
+      if (up)
+        launch(KDown<M, double, TY, kFineSweeps, true>);
+      else
+        launch(KDown<M, double, TY, kFineSweeps>);
+    });
+  } else {
+    KDown<M, M, kMidY, kSweeps><<<L.mid.blocks(), kTileThreads, 0, st>>>(
+        L.nx, L.ny, L.mid, L.kx, L.ky, L.dinv, L.r, sweeps, L.xb, C.nx, C.ny, C.r, done, fz,
+        (l == 1 && up) ? 1 : 0);
+  }
   // the coarser level's correction goes to its xa: its xb holds the x2 that
   // its up-leg reads on tile halos while other workgroups write their output
   Cycle(l + 1, nullptr, nullptr, C.xa, st, done, (l == 0 && up) ? f : nullptr);
@@ -1033,10 +1045,13 @@ void MgPrecondT<M>::Cycle(int l, const double* r64, float* z, M* out, hipStream_
   if (l == 0) {
     // after the folded update the level's residual is the one it wrote
     const double* r0 = up ? fz.up_r : r64;
-    if (bilinear)
-      HG_UP(float, double, true, kTallY, kFineSweeps, fine_sweeps, L.tall, r0, z);
-    else
-      HG_UP(float, double, false, kTallY, kFineSweeps, fine_sweeps, L.tall, r0, z);
+    WithFineTile([&](auto ty) {
+      constexpr int TY = decltype(ty)::value;
+      if (bilinear)
+        HG_UP(float, double, true, TY, kFineSweeps, fine_sweeps, fine_, r0, z);
+      else
+        HG_UP(float, double, false, TY, kFineSweeps, fine_sweeps, fine_, r0, z);
+    });
   } else {
     if (bilinear)
       HG_UP(M, M, true, kMidY, kSweeps, sweeps, L.mid, L.r, out);
@@ -1056,7 +1071,7 @@ bool MgPrecondT<M>::ApplyFcg(const double* r, float* z, hipStream_t st, const in
                              const FcgFusion& f, int* ndir) {
   if (lv_.size() < 2) return false;  // no KDown / KUp pair on the finest level
   Cycle(0, r, z, nullptr, st, d_done, &f);
-  *ndir = lv_[0].tall.blocks();
+  *ndir = fine_.blocks();
   return true;
 }
 
@@ -1068,13 +1083,20 @@ double MgPrecondT<M>::TimeKernel(const char* name, int reps, const double* r, hi
   MgLevelT<M>& C = lv_[1];
   auto launch = [&]() {
     if (k == "KDown<double>") {
-      KDown<M, double, kTallY, kFineSweeps><<<L.tall.blocks(), kTileThreads, 0, st>>>(
-          L.nx, L.ny, L.tall, L.kx, L.ky, L.dinv, r, fine_sweeps, L.xb, C.nx, C.ny,
-          C.r, never_done_, FcgFusion{}, 0);
+      WithFineTile([&](auto ty) {
+        KDown<M, double, decltype(ty)::value, kFineSweeps>
+            <<<fine_.blocks(), kTileThreads, 0, st>>>(L.nx, L.ny, fine_, L.kx, L.ky, L.dinv, r,
+                                                      fine_sweeps, L.xb, C.nx, C.ny, C.r,
+                                                      never_done_, FcgFusion{}, 0);
+      });
     } else if (k == "KUp<double, true>") {
-      KUp<M, M, double, true, kTallY, kFineSweeps><<<L.tall.blocks(), kTileThreads, 0, st>>>(
-          L.nx, L.ny, L.tall, L.kx, L.ky, L.dinv, r, L.xb, C.xa, C.kx, C.ky, C.nx, C.ny,
-          fine_sweeps, L.xa, never_done_, FcgFusion{}, 0);
+      WithFineTile([&](auto ty) {
+        KUp<M, M, double, true, decltype(ty)::value, kFineSweeps>
+            <<<fine_.blocks(), kTileThreads, 0, st>>>(L.nx, L.ny, fine_, L.kx, L.ky, L.dinv, r,
+                                                      L.xb, C.xa, C.kx, C.ky, C.nx, C.ny,
+                                                      fine_sweeps, L.xa, never_done_, FcgFusion{},
+                                                      0);
+      });
     } else if (k == "KCoarseCycle" && first_in_kernel_ > 0) {
       Cycle(first_in_kernel_, nullptr, nullptr, lv_[first_in_kernel_].xa, st, nullptr);
     } else {

@@ -57,20 +57,6 @@ __device__ __forceinline__ uint4 Ld8(const bf* p) { return *reinterpret_cast<con
 __device__ __forceinline__ b8 LdOp(const bf* p) { return __builtin_bit_cast(b8, Ld8(p)); }
 __device__ __forceinline__ void St8(bf* p, uint4 v) { *reinterpret_cast<uint4*>(p) = v; }
 
-// Sum over the wave, in lane 63.
-__device__ __forceinline__ float WaveSumF(float v) {
-#define HG_DPP_ADD(ctrl, rows) \
-  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), ctrl, rows, 0xf, true))
-  HG_DPP_ADD(0x111, 0xf);  // row_shr:1, 2, 4, 8
-  HG_DPP_ADD(0x112, 0xf);
-  HG_DPP_ADD(0x114, 0xf);
-  HG_DPP_ADD(0x118, 0xf);
-  HG_DPP_ADD(0x142, 0xa);  // row_bcast:15, 31
-  HG_DPP_ADD(0x143, 0xc);
-#undef HG_DPP_ADD
-  return v;
-}
-
 // ---------------------------------------------------------------------------
 // 3x3 'same' convolution, CIN, COUT multiples of 16, as an implicit GEMM on
 // gfx950's MFMA 16x16x32 BF16 (FP32 accumulate).  A block of 4 waves
@@ -432,7 +418,7 @@ KEndWgrad(int W, int H, const float* __restrict__ s, const bf* __restrict__ f,
   for (int t = 0; t < 9; ++t)
 #pragma unroll
     for (int c = 0; c < 16; ++c) {
-      const float w = WaveSumF(acc[t][c]);
+      const float w = DppSum<6>(acc[t][c]);
       if ((threadIdx.x & 63) == 63) red[threadIdx.x >> 6][t * 16 + c] = w;
     }
   __syncthreads();
