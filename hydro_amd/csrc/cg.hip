@@ -33,6 +33,7 @@
 
 #include "cg.h"
 #include "device_common.h"
+#include "exchange.h"
 #include "learned.h"
 #include "tile.h"
 
@@ -302,101 +303,7 @@ KPcgStart(Walk w, const T* __restrict__ r, const T* __restrict__ dinv, T* __rest
 // after them saves about 1 us of that, sums by lane shifts instead of shuffles
 // through LDS 1.5 us, 1024 threads instead of 512 0.4 us.
 //
-// 64 workgroups: a quarter of the CUs, since kernels of four queues may run at
-// once and every workgroup waits for the others of its kernel (and one wave
-// reads all their partials).  The waits are bounded: a solve that waited too
-// long leaves sc->done 0 and the start's x in xsave.
-constexpr int kWholeMaxWg = 64;
-constexpr int kWholeThreads = 1024;
-constexpr long kWholeMaxCells = 4L * kWholeThreads * kWholeMaxWg;
-constexpr int kWholeLds = 8000;  // doubles
-constexpr int kWholeSpin = 1 << 17;
-// exchange words [2 parities][4][64], the count of finished workgroups, the
-// tags used so far
-constexpr int kWholeDone = 2 * 4 * kWholeMaxWg, kWholeEpoch = kWholeDone + 1;
-constexpr int kWholeWords = kWholeEpoch + 1;
-
-// A value travels as one (T = float) or two words that each hold 32 bits of it
-// under the exchange's number `tag`, so that it needs no flag behind it.
-using Word = unsigned long long;
-__device__ __forceinline__ Word TagLoad(const Word* p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void TagStore(Word* p, unsigned tag, unsigned v) {
-  __hip_atomic_store(p, Word(tag) << 32 | v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ double FromWords(Word lo, Word hi) {
-  return __hiloint2double(int(unsigned(hi)), int(unsigned(lo)));
-}
-
-// Sums v over all workgroups, in a fixed order; `extra` = post(sums), formed
-// in one wave.  Words of a parity are written again two exchanges later, when
-// every workgroup has read them.  `others` runs in the other waves while the
-// first waits for the sums.  False, in the whole workgroup: gave up.
-template <int NV, class Post, class Others>
-__device__ __forceinline__ bool Exchange(double (&v)[NV], double& extra, unsigned tag,
-                                         Word* words, int* gave_up, Post&& post,
-                                         Others&& others) {
-  constexpr int kWaves = kWholeThreads / 64;  // at most 16: one row of lanes
-  __shared__ double red[NV][kWaves];
-  __shared__ double tot[NV + 1];
-  const int lane = threadIdx.x & 63, W = gridDim.x;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-#pragma unroll
-  for (int q = 0; q < NV; ++q) {
-    const double s = DppSum<6>(v[q]);
-    if (lane == 63) red[q][wave] = s;
-  }
-  __syncthreads();
-  bool ok = true;
-  if (wave == 0) {
-#pragma unroll
-    for (int q = 0; q < NV; ++q)
-      v[q] = LaneOf(DppSum<4>(lane < kWaves ? red[q][lane] : 0.), 15);
-    if (W > 1) {
-      Word* const mine = words + (tag & 1) * 4 * kWholeMaxWg;
-      if (lane == 0) {
-#pragma unroll
-        for (int q = 0; q < NV; ++q) {
-          TagStore(mine + 2 * q * kWholeMaxWg + blockIdx.x, tag, unsigned(__double2loint(v[q])));
-          TagStore(mine + (2 * q + 1) * kWholeMaxWg + blockIdx.x, tag,
-                   unsigned(__double2hiint(v[q])));
-        }
-      }
-      Word g[2 * NV];
-      for (int n = 0;; ++n) {
-        bool all = true;
-#pragma unroll
-        for (int i = 0; i < 2 * NV; ++i) g[i] = TagLoad(mine + i * kWholeMaxWg + min(lane, W - 1));
-#pragma unroll
-        for (int i = 0; i < 2 * NV; ++i) all = all && unsigned(g[i] >> 32) == tag;
-        if (__all(all)) break;
-        if (n == kWholeSpin) {
-          ok = false;
-          break;
-        }
-      }
-#pragma unroll
-      for (int q = 0; q < NV; ++q)
-        v[q] = WaveTotal(lane < W ? FromWords(g[2 * q], g[2 * q + 1]) : 0.);
-    }
-    const double e = post(v);
-    if (lane == 0) {
-#pragma unroll
-      for (int q = 0; q < NV; ++q) tot[q] = v[q];
-      tot[NV] = e;
-    }
-  } else {
-    ok = others();
-  }
-  if (!ok) *gave_up = 1;
-  __syncthreads();
-#pragma unroll
-  for (int q = 0; q < NV; ++q) v[q] = tot[q];
-  extra = tot[NV];
-  return *gave_up == 0;
-}
-
+// A solve that waited too long leaves sc->done 0 and the start's x in xsave.
 template <class T, int K>
 __global__ void __launch_bounds__(kWholeThreads)
 KPcgWhole(int nx, int ny, int C, const T* __restrict__ kx, const T* __restrict__ ky,
@@ -473,7 +380,7 @@ KPcgWhole(int nx, int ny, int C, const T* __restrict__ kx, const T* __restrict__
     dots[1] += double(r[i]) * double(r[i]);
   }
   auto None = [](const auto&) { return 0.; };
-  if (!Exchange<2>(dots, quot, tag, words, &gave_up, None, Halo)) return;
+  if (!Exchange<SumFold>(dots, quot, tag, words, &gave_up, None, [] {}, Halo)) return;
   int k = 0;
   for (;; ++k) {
     const double rz = dots[0], rr = dots[1];
@@ -509,8 +416,8 @@ KPcgWhole(int nx, int ny, int C, const T* __restrict__ kx, const T* __restrict__
       }
     }
     ++tag;
-    if (!Exchange<1>(pq, quot, tag, words, &gave_up,
-                         [&](const auto& s) { return rz / s[0]; }, [] { return true; }))
+    if (!Exchange<SumFold>(pq, quot, tag, words, &gave_up,
+                         [&](const auto& s) { return rz / s[0]; }, [] {}, [] { return true; }))
       return;
     const T a = T(quot);
     ++tag;
@@ -526,30 +433,18 @@ KPcgWhole(int nx, int ny, int C, const T* __restrict__ kx, const T* __restrict__
         dots[1] += double(r[i]) * double(r[i]);
       }
     }
-    if (!Exchange<2>(dots, quot, tag, words, &gave_up,
-                         [&](const auto& s) { return s[0] / rz; }, Halo))
+    if (!Exchange<SumFold>(dots, quot, tag, words, &gave_up,
+                         [&](const auto& s) { return s[0] / rz; }, [] {}, Halo))
       return;
   }
 #pragma unroll
   for (int i = 0; i < K; ++i)
     if (in[i]) x[c0 + threadIdx.x + i * NT] = xv[i];
   // the solve is done when every workgroup got here
-  if (threadIdx.x == 0 &&
-      __hip_atomic_fetch_add(words + kWholeDone, Word(1), __ATOMIC_RELAXED,
-                             __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1) {
-    words[kWholeDone] = 0;
-    words[kWholeEpoch] = tag;
+  if (threadIdx.x == 0 && FinishWhole(words, tag)) {
     sc->done = 1;
     sc->iter = k;
     sc->rr = dots[1];
-  }
-}
-
-// After a solve that gave up: no tag of it is used again.
-__global__ void KWholeReset(Word* words, unsigned tags) {
-  if (threadIdx.x == 0) {
-    words[kWholeDone] = 0;
-    words[kWholeEpoch] = Word(unsigned(words[kWholeEpoch]) + tags);
   }
 }
 
@@ -1106,19 +1001,14 @@ template <class T>
 bool CgSolver::WholePcg(const T* kx, const T* ky, const T* dinv, const T* r, T* x, T* xsave,
                         int max_iters) {
   if (n_ > kWholeMaxCells) return false;
-  // at most 16 workgroups where more cells per thread allow it: 32 cost 1.3 us
-  // more per iteration (65025 cells: 16 x 4096 4.6 us, 32 x 2048 5.0, 64 x 1024
-  // 5.8; 16384 cells: 16 x 1024 3.4, 8 x 2048 3.7, 4 x 4096 4.1)
-  const int n = int(n_), nt = kWholeThreads, k = n <= 16 * nt ? 1 : n <= 32 * nt ? 2 : 4;
-  int wgs = (n + k * nt - 1) / (k * nt);
-  const int c = ((n + wgs - 1) / wgs + 63) / 64 * 64;  // <= k nt
-  wgs = (n + c - 1) / c;
+  const WholeSplit split = SplitWhole(int(n_));
+  const int k = split.k, c = split.cells;
   if (long(c) + 4L * nx_ > kWholeLds) return false;
   Word* const words = (Word*)words_;
   Word* const zw = words + kWholeWords;
   CgScalars* const sc = (CgScalars*)scal_;
   auto launch = [&](auto kernel) {
-    kernel<<<wgs, kWholeThreads, size_t(c + 4 * nx_) * sizeof(T), stream_>>>(
+    kernel<<<split.wgs, kWholeThreads, size_t(c + 4 * nx_) * sizeof(T), stream_>>>(
         nx_, ny_, c, kx, ky, dinv, r, x, xsave, zw, words, sc);
   };
   launch(k == 1 ? KPcgWhole<T, 1> : k == 2 ? KPcgWhole<T, 2> : KPcgWhole<T, 4>);

@@ -151,6 +151,19 @@ __device__ __forceinline__ M DppSum(M v) {
   }
   return v;
 }
+// The same for the maximum of non-negative values.
+template <int R>
+__device__ __forceinline__ double DppMax(double v) {
+  v = fmax(v, DppMove<0x111, 0xf>(v));
+  v = fmax(v, DppMove<0x112, 0xf>(v));
+  v = fmax(v, DppMove<0x114, 0xf>(v));
+  v = fmax(v, DppMove<0x118, 0xf>(v));
+  if constexpr (R == 6) {
+    v = fmax(v, DppMove<0x142, 0xa>(v));
+    v = fmax(v, DppMove<0x143, 0xc>(v));
+  }
+  return v;
+}
 __device__ __forceinline__ float LaneOf(float v, int lane) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
 }

@@ -30,6 +30,7 @@
 #include <vector>
 
 #include "../../include/hydro_gpu3d.h"
+#include "exchange.h"
 #include "mg3d.h"
 
 #define H3_CHECK(x)                                                                    \
@@ -41,6 +42,22 @@
 
 namespace hg3 {
 namespace {
+
+using hg::Exchange;
+using hg::FinishWhole;
+using hg::FromWords;
+using hg::kWholeEpoch;
+using hg::kWholeLds;
+using hg::kWholeSpin;
+using hg::kWholeThreads;
+using hg::kWholeWords;
+using hg::KWholeReset;
+using hg::MaxFold;
+using hg::SplitWhole;
+using hg::TagLoad;
+using hg::TagStore;
+using hg::WholeSplit;
+using hg::Word;
 
 constexpr int kB = 256;
 inline unsigned Grid(long n) { return unsigned((n + kB - 1) / kB); }
@@ -543,6 +560,143 @@ KJacobiSweep(G g, Rows A, const double* __restrict__ k, const double* __restrict
   }
   JacobiPut(m, JacRow(diff, s));
 }
+// The whole solve of a small grid in one launch (exchange.h): each workgroup a
+// contiguous range of cells, K per thread with their rows in registers, the
+// iterate of the range and of the planes before and after it in LDS.  A sweep
+// ends with one exchange of the maximum and of the new values of those planes;
+// its arithmetic and stop rule are KJacobiSweep's.  state[0] stays 0 when it
+// gave up.
+//
+// It is bound by that exchange, a round trip between XCDs, and by the planes'
+// values in it (at 48 x 40 x 36 every cell is in one of them).  Two steps of a
+// lid-driven cavity with SIMPLE loops of such solves, a launch per sweep | this:
+// 12x10x8 3.3 | 2.4 ms, 32^3 6.1 | 4.5, 40^3 7.2 | 5.6, 48x40x36 8.1 | 6.3, 50^3
+// 9.6 | 8.0; with four cells per thread and half the workgroups 48x40x36 takes
+// 7.4 (registers spill).
+constexpr long kJacWholeCells = 2L * kWholeThreads * hg::kWholeMaxWg;
+template <int K>
+__global__ void __launch_bounds__(kWholeThreads)
+KJacobiWhole(G g, int C, Rows A, const double* __restrict__ kc, double* __restrict__ x,
+             double omega, double tol, int limit, Word* words, int* state) {
+  extern __shared__ double xs[];  // x of the cells c0 - plane .., then a 0
+  __shared__ int gave_up;
+  constexpr int NT = kWholeThreads;
+  const int n = int(g.nc), plane = g.nx * g.ny;
+  const int c0 = blockIdx.x * C, c1 = min(c0 + C, n);
+  // the planes' values, by cell: low halves, high halves; two sets in turn, as
+  // a workgroup may write the next sweep's while another reads this sweep's
+  Word* const xw0 = words + kWholeWords;
+  const unsigned epoch = unsigned(TagLoad(words + kWholeEpoch));
+  unsigned tag = epoch;
+  const int off[7] = {-plane, -g.nx, -1, 0, 1, g.nx, plane};
+  double t[K][7], kv[K], xn[K];
+  bool in[K], edge[K];
+  unsigned at[K][3];  // the neighbours' places in xs, two to a word
+  if (threadIdx.x == 0) gave_up = 0;
+  const int zero = C + 2 * plane;
+  for (int h = threadIdx.x; h <= zero; h += NT) xs[h] = 0.;
+#pragma unroll
+  for (int i = 0; i < K; ++i) {
+    const int l = threadIdx.x + i * NT;
+    in[i] = l < C && c0 + l < c1;
+    edge[i] = in[i] && (l < plane || c0 + l + plane >= c1);
+    const JacCell o = JacAt(g, unsigned(in[i] ? c0 + l : 0));
+    // a missing neighbour is 0 times the 0 behind xs: it leaves the sum, which
+    // starts at +0 and so never is -0, as it is
+    unsigned p[6];
+#pragma unroll
+    for (int w = 0; w < 6; ++w) {
+      const int q = w < 3 ? w : w + 1;
+      const double tq = A.t[q][o.c];
+      t[i][w] = o.has[q] ? tq : 0.;
+      p[w] = unsigned(o.has[q] ? plane + l + off[q] : zero);
+    }
+    t[i][6] = A.t[3][o.c];  // the cell's own
+#pragma unroll
+    for (int q = 0; q < 3; ++q) at[i][q] = p[2 * q] | p[2 * q + 1] << 16;
+    kv[i] = kc[o.c];
+    xn[i] = 0.;
+  }
+  // the planes around the range, by all waves but the first, four at a time
+  auto Halo = [&]() {
+    const Word* const xw = xw0 + (tag & 1) * 2l * n;
+    for (int h0 = int(threadIdx.x) - 64; h0 < 2 * plane; h0 += 4 * (NT - 64)) {
+      for (int m = 0;; ++m) {
+        Word lo[4], hi[4];
+        bool ok = true;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int h = h0 + u * (NT - 64), c = h < plane ? c0 - plane + h : c1 - plane + h;
+          lo[u] = hi[u] = Word(tag) << 32;  // 0 outside the grid
+          if (h < 2 * plane && c >= 0 && c < n) {
+            lo[u] = TagLoad(xw + c);
+            hi[u] = TagLoad(xw + n + c);
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          ok = ok && unsigned(lo[u] >> 32) == tag && unsigned(hi[u] >> 32) == tag;
+        if (ok) {
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            const int h = h0 + u * (NT - 64);
+            if (h < 2 * plane) xs[h < plane ? h : c1 - c0 + h] = FromWords(lo[u], hi[u]);
+          }
+          break;
+        }
+        if (m == kWholeSpin) return false;
+      }
+    }
+    return true;
+  };
+  __syncthreads();
+  int s = 0, iters = 0;
+  for (;; ++s) {
+    ++tag;
+    double m[1] = {0.}, unused;
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+      if (!in[i]) continue;
+      double sum = 0.;
+#pragma unroll
+      for (int q = 0; q < 6; ++q)
+        sum += t[i][q] * xs[q & 1 ? at[i][q >> 1] >> 16 : at[i][q >> 1] & 0xffffu];
+      const double value = -(kv[i] + sum) / t[i][6];
+      const double corr = value - xn[i];
+      m[0] = fmax(m[0], fabs(corr));
+      xn[i] = xn[i] + corr * omega;
+      if (edge[i]) {
+        Word* const w = xw0 + (tag & 1) * 2l * n + c0 + threadIdx.x + i * NT;
+        TagStore(w, tag, unsigned(__double2loint(xn[i])));
+        TagStore(w + n, tag, unsigned(__double2hiint(xn[i])));
+      }
+    }
+    auto Put = [&]() {
+#pragma unroll
+      for (int i = 0; i < K; ++i)
+        if (in[i]) xs[plane + threadIdx.x + i * NT] = xn[i];
+    };
+    if (!Exchange<MaxFold>(m, unused, tag, words, &gave_up, [](const auto&) { return 0.; }, Put,
+                           Halo))
+      return;
+    if (!(m[0] > tol)) {
+      iters = s;
+      break;
+    }
+    if (!(s < limit)) {
+      iters = s + 1;
+      break;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < K; ++i)
+    if (in[i]) x[c0 + threadIdx.x + i * NT] = xn[i];
+  if (threadIdx.x == 0 && FinishWhole(words, tag)) {
+    state[0] = 1;
+    state[1] = iters;
+  }
+}
+
 // the stop rule after the last sweep s of a batch (one wave)
 __global__ void KJacobiCheck(unsigned long long* diff, int s, double tol, int limit, int* state) {
   if (state[0]) return;
@@ -1049,6 +1203,7 @@ struct hg3_ctx {
   double *part, *scal_d;
   unsigned long long* jdiff;
   int* jstate;
+  Word* jwords = nullptr;  // KJacobiWhole's words, where the grid is small enough
   int* flag;
   // cg
   double *cb, *cr, *cz, *cp, *cq, *cx;
@@ -1302,8 +1457,20 @@ int SolveJacobi(hg3_ctx* c, const Rows& R, const double* k, double* x) {
   const hg_config& cfg = c->cfg;
   const int limit = cfg.lu_relaxed_num_iters_limit;
   const double tol = cfg.lu_relaxed_tolerance, omega = cfg.lu_relaxed_relaxation_factor;
-  H3_CHECK(hipMemsetAsync(c->jdiff, 0, size_t(kJacSlots) * 8, c->st));
   H3_CHECK(hipMemsetAsync(c->jstate, 0, 4 * sizeof(int), c->st));
+  if (c->jwords) {
+    const WholeSplit w = SplitWhole(int(c->nc), 2);
+    auto launch = [&](auto kernel) {
+      kernel<<<w.wgs, kWholeThreads, size_t(w.cells + 2 * c->g.nx * c->g.ny + 1) * 8, c->st>>>(
+          c->g, w.cells, R, k, x, omega, tol, limit, c->jwords, c->jstate);
+    };
+    launch(w.k == 1 ? KJacobiWhole<1> : KJacobiWhole<2>);
+    H3_CHECK(hipMemcpyAsync(c->state_h, c->jstate, 4 * sizeof(int), hipMemcpyDeviceToHost, c->st));
+    c->Sync();
+    if (c->state_h[0]) return c->state_h[1];
+    KWholeReset<<<1, 64, 0, c->st>>>(c->jwords, unsigned(limit) + 2u);
+  }
+  H3_CHECK(hipMemsetAsync(c->jdiff, 0, size_t(kJacSlots) * 8, c->st));
   H3_CHECK(hipMemsetAsync(c->corr, 0, size_t(c->nc) * 8, c->st));
   double* buf[2] = {c->corr, c->corr2};
   int s = 0;
@@ -1721,6 +1888,11 @@ hg_status hg3_create(const hg3_config* cfg3, hg3_ctx** out) {
     // three components' parts of max |corr| and states (done, iters, buffer)
     c->jdiff = (unsigned long long*)c->Alloc(3L * kJacRows * kJacSlots);
     c->jstate = (int*)c->Alloc(6);
+    if (c->nc <= kJacWholeCells &&
+        SplitWhole(int(c->nc), 2).cells + 2L * cfg.nx * cfg.ny < kWholeLds) {
+      c->jwords = (Word*)c->Alloc(kWholeWords + 4 * c->nc);
+      H3_CHECK(hipMemsetAsync(c->jwords, 0, size_t(kWholeWords + 4 * c->nc) * 8, c->st));
+    }
     if (cfg.linear_solver_velocity == HG_SOLVER_JACOBI)
       for (int d = 0; d < 3; ++d)
         for (int b = 0; b < 2; ++b) c->jbuf[d][b] = c->Alloc(nc);

@@ -134,3 +134,21 @@ def test_gpu3d_iteration_cap_reports_not_converged(gpu, solver):
     with Hydro3(workloads.cavity3d(16, 16, 16, solver_p=solver)) as h:
         st = h.step()
         assert st.pressure_converged == 1
+
+
+# the one-launch Jacobi solve: one and two cells per thread, one and many
+# workgroups, planes larger and smaller than a workgroup's range, a plane its LDS
+# has no room for
+@pytest.mark.parametrize("nx,ny,nz", [(3, 2, 2), (16, 16, 4), (8, 8, 300), (40, 28, 17),
+                                      (50, 40, 4), (24, 30, 64), (100, 90, 3)])
+def test_gpu3d_jacobi_any_size_bitwise(gpu, nx, ny, nz):
+    print(f"case: jacobi {nx}x{ny}x{nz}", flush=True)
+    text = workloads.cavity3d(nx, ny, nz)
+    o = pyoracle.Oracle3(capi.parse_config3(text))
+    with Hydro3(text) as h:
+        for _ in range(2):
+            sg, so = h.step(), o.step()
+            assert sg.simple_iterations == so.simple_iterations
+        for fid in (capi.HG_FIELD_VELOCITY_X, capi.HG_FIELD_VELOCITY_Z, capi.HG_FIELD_PRESSURE):
+            np.testing.assert_array_equal(h.get(fid), o.get(fid))
+    o.close()
