@@ -8,8 +8,10 @@
 // handles row j = step - t at each step; the west value crosses threads
 // through LDS, the south value stays in registers, and one barrier separates
 // steps.  Each cell computes exactly the reference's expression, so the
-// result equals the serial sweep bit for bit.  Compiled with
-// -ffp-contract=off.
+// result equals the serial sweep bit for bit.  "lu" runs on rows packed by step
+// where it has a workspace (KLuSkew), and "gauss_seidel" with many sweeps in
+// flight (sor.hip); the in-place kernels here are for what those do not take.
+// Compiled with -ffp-contract=off.
 
 #include <algorithm>
 #include <type_traits>
