@@ -189,7 +189,7 @@ void LaunchGsWavefront(hipStream_t st, int nx, int ny, Rows a, const double* k, 
 // fewer sweeps in flight, and without room for two (or where the shorter side
 // exceeds 1024 or the longer is under 8) it runs LaunchGsWavefront.
 // info[0] == kSorRetry: the workgroups of a large grid did not run together
-// and the solve gave up; call again with `retry`.
+// and the solve gave up (or it ran for 2^30 steps); call again with `retry`.
 constexpr unsigned long long kSorRetry = ~0ull;
 long SorWorkspace(int nx, int ny);
 void LaunchSor(hipStream_t st, int nx, int ny, Rows a, const double* k, double* x, double tol,

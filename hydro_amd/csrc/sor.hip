@@ -40,99 +40,12 @@
 // workgroup 15.3) against 177 us; 333x217 13 (43) against 534 us.
 // For one workgroup 1024 threads beat 512 and 256 (256x128: 15.3, 19.7, 30.9
 // us); for each of several 512 (256x128: 3.7; 1024: 7.2, 256: 4.8 us).
-#include <algorithm>
-
 #include "kernels.h"
+#include "sor_plan.h"
 
 namespace hg {
 
 namespace {
-
-constexpr int kSorThreads = 1024;
-constexpr int kSorMaxQ = 32;
-constexpr int kSorHeader = 32;  // doubles before the arrays: [0] the result's ring slot
-
-// (several workgroups, below)
-constexpr int kLag = 20;
-constexpr int kSpin = 1 << 20;
-constexpr int kNever = 0x7fffffff;
-
-constexpr int kSorMaxG = 64, kSorMaxStages = 1024;
-constexpr long kChainMaxDoubles = 1L << 26;  // of the workspace
-// Workspace header, in doubles: the smallest sweep that ended the solve
-// (int `stop`), then a 64-byte line of progress per workgroup, then the max
-// |corr| of the sweep each stage last found to end it.
-constexpr int kChainProgress = 8, kChainRec = kChainProgress + 8 * kSorMaxG;
-constexpr int kChainHeader = kChainRec + kSorMaxStages;
-
-struct SorChain {
-  int a, b, ap;           // short and long side, line padded to waves
-  int Q, G, span, le;     // thread groups per workgroup, workgroups, log rows
-  int limit, tail;
-};
-
-struct SorPlan {
-  bool ok = false;
-  bool tr = false;   // threads along y (the short side), marching along x
-  int a = 0, b = 0;  // short and long side
-  int Q = 0, rounds = 0;
-  int G = 1, span = 0, le = 0;  // several workgroups (G > 1): see KSorChain
-  long doubles = 0;
-};
-
-// The ring holds `rounds` rounds of P = 2 Q sweeps: sweep s's buffer is
-// written again by sweep s + rounds P, which starts (rounds - 1) b steps after
-// the round that follows s begins, and s is decided a + b + 5 steps after its
-// own start at the latest.
-SorPlan PlanSor(int nx, int ny, int limit, long max_doubles) {
-  SorPlan p;
-  p.tr = ny < nx;
-  p.a = std::min(nx, ny);
-  p.b = std::max(nx, ny);
-  const long n = long(nx) * ny;
-  p.rounds = p.a + 7 <= p.b ? 2 : 3;
-  int q = std::min(std::min(kSorThreads / std::max(p.a, 1), (p.b - 4) / 4), kSorMaxQ);
-  q = std::min(q, limit / 2 + 1);  // sweeps 0 .. limit
-  for (; q >= 1; --q) {
-    p.doubles = kSorHeader + (6 + 2L * q * p.rounds) * n;
-    // (32-bit byte offsets in the kernel)
-    if (p.doubles <= max_doubles && p.doubles < (1L << 29)) {
-      p.Q = q;
-      p.ok = true;
-      break;
-    }
-  }
-  return p;
-}
-
-// The several-workgroup plan: 512 threads (1024 where a line needs them),
-// as many workgroups as keep kLag steps between them.  A log keeps what the
-// tail may read: a + b rows of a line, up to b + span steps after its end (a
-// workgroup is at most the sum of the lags, under b, ahead of another).
-SorPlan PlanChain(int nx, int ny, int limit, long max_doubles) {
-  SorPlan p;
-  p.tr = ny < nx;
-  p.a = std::min(nx, ny);
-  p.b = std::max(nx, ny);
-  const long n = long(nx) * ny;
-  const int ap = (p.a + 63) / 64 * 64;
-  if (ap > kSorThreads) return p;
-  p.Q = std::max(512 / ap, 1);
-  const int P = 2 * p.Q;
-  int g = std::min(std::min(p.b / (2 * P + kLag), kSorMaxG), kSorMaxStages / P);
-  g = std::min(g, limit / P + 1);
-  for (; g >= 2; --g) {
-    p.span = p.b / g;
-    p.le = p.a + 2 * p.b + p.span + 64;
-    p.doubles = kChainHeader + 7 * n + long(g) * p.le * p.a;
-    if (p.doubles <= std::min(max_doubles, kChainMaxDoubles)) {
-      p.G = g;
-      p.ok = true;
-      break;
-    }
-  }
-  return p;
-}
 
 // Barrier between steps.  It orders the LDS exchange and leaves the loads in
 // flight; of the global stores it waits for those of two steps before and
@@ -440,7 +353,9 @@ KSorChain(SorChain ch, const double2* __restrict__ oc, const double2* __restrict
   int from = wg == 0 ? b : -1;
   if (ch.tail) {
     const int s = *stop;
-    if (s < 0) {
+    // gave up, or ran out of step numbers before every sweep up to s was decided
+    // (kNever, the last number of 32 bits, is past them too: G P < b)
+    if (s < 0 || ChainDoneStep(s, P, G * P, span, a, b) + 4 > kChainMaxStep) {
       if (threadIdx.x == 0) info[0] = ~0ull;
       return;
     }
@@ -581,12 +496,9 @@ KSorChain(SorChain ch, const double2* __restrict__ oc, const double2* __restrict
         rec[s % ptot] = bits;
     }
   };
-  // virtual step by which sweep s is decided and every earlier one too
-  auto DoneStep = [&](int s) {
-    const int st = s % ptot;
-    return (st / P) * span + 2 * (st % P) + (s / ptot) * b + a + b;
-  };
-  const int end = DoneStep(limit) + 4;
+  // (steps are counted in 32 bits: a solve that gets to kChainMaxStep has not
+  // met the stop rule, and `stop` stays kNever)
+  const int end = int(min(ChainDoneStep(limit, P, ptot, span, a, b) + 4, long(kChainMaxStep)));
   int lrow = start % le, done_steps = start;
   for (int T = start;; T += 4) {
     // ---- the next group's input
@@ -680,7 +592,8 @@ KSorChain(SorChain ch, const double2* __restrict__ oc, const double2* __restrict
       for (int i = 0; i < 4; ++i) cur[i] = nxt[i];
     }
     const int s = lstop;
-    const int stop_at = s == kNever ? end : s < 0 ? 0 : min(end, DoneStep(s) + 4);
+    const int stop_at =
+        s == kNever ? end : s < 0 ? 0 : min(end, int(ChainDoneStep(s, P, ptot, span, a, b)) + 4);
     ChainBarrier();  // lstop is not written again before every thread read it
     if (T >= stop_at) break;
   }
@@ -694,20 +607,7 @@ KSorChain(SorChain ch, const double2* __restrict__ oc, const double2* __restrict
 
 }  // namespace
 
-// Several workgroups where they hold more sweeps than one does.  Measured per
-// sweep, one | several (stages held): 64x128 5.7 | 4.5 us (32 | 48), 64x256
-// 10.2 | 5.2 us (32 | 112), 256x128 at 700 sweeps 15.3 | 3.7 us (16 | 56),
-// 333x217 at 100 43.5 | 13.2 us (8 | 52); with fewer stages they lose: 32x128
-// 3.7 | 4.2 us (64 | 48), 16x256 4.0 | 5.2 us (128 | 112), as the lines are
-// padded to waves.
-static bool UseChain(const SorPlan& one, const SorPlan& many) {
-  return many.ok && (!one.ok || many.G * many.Q > one.Q);
-}
-
-long SorWorkspace(int nx, int ny) {
-  const SorPlan p = PlanSor(nx, ny, 1 << 30, 1L << 60), c = PlanChain(nx, ny, 1 << 30, 1L << 60);
-  return std::max(p.ok ? p.doubles : 0, c.ok ? c.doubles : 0);
-}
+long SorWorkspace(int nx, int ny) { return SorWorkspaceDoubles(nx, ny); }
 
 void LaunchSor(hipStream_t st, int nx, int ny, Rows a, const double* k, double* x, double tol,
                int limit, double omega, unsigned long long* info, double* ws, long ws_doubles,

@@ -42,3 +42,18 @@ def test_sor_bitwise(gpu, nx, ny, tol, limit):
     xo, so = pyoracle.stencil_solve(nx, ny, *r, capi.SOLVERS["gauss_seidel"], **args)
     assert st.iterations == so.iterations
     assert np.array_equal(x, xo)
+
+
+# a limit that only says "stop by the tolerance": its last step is past 32 bits
+# on the grids that run over several workgroups (here 4, 11 and 21 of them)
+@pytest.mark.parametrize("nx,ny", [(64, 256), (333, 217), (512, 512), (64, 64)])
+@pytest.mark.parametrize("limit", [10**9, 2**31 - 1])
+def test_sor_without_a_limit(gpu, nx, ny, limit):
+    print(f"case: SOR {nx}x{ny} limit {limit}", flush=True)
+    r = rows(nx, ny, 5)
+    args = dict(tol=3e-2, omega=1.7)
+    x, st = stencil_solve(nx, ny, *r, "gauss_seidel", max_iters=limit, **args)
+    xo, so = pyoracle.stencil_solve(nx, ny, *r, capi.SOLVERS["gauss_seidel"], max_iters=1000,
+                                    **args)
+    assert 2 < so.iterations < 1000 and st.iterations == so.iterations
+    assert np.array_equal(x, xo)

@@ -1,0 +1,55 @@
+"""The plan arithmetic of the pipelined SOR (hydro_amd/csrc/sor_plan.h) on the
+host, under UndefinedBehaviorSanitizer: limits up to 2^31 - 1 sweeps ("stop by
+the tolerance alone"), against the same formulas in Python's integers."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+KEYS = ("ok_one q_one rounds doubles_one chain q g span le doubles_many a b end").split()
+
+
+@pytest.fixture(scope="module")
+def plan(tmp_path_factory):
+    if not shutil.which("g++"):
+        pytest.skip("g++ not found")
+    exe = tmp_path_factory.mktemp("sor") / "sor_plan_driver"
+    r = subprocess.run(["g++", "-std=c++17", "-O1", "-fsanitize=undefined",
+                        "-fno-sanitize-recover=all", "-o", str(exe),
+                        os.path.join(ROOT, "tests", "sor_plan_driver.cpp")],
+                       capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stderr[-3000:]
+
+    def run(cases):
+        text = "".join("%d %d %d\n" % c for c in cases)
+        r = subprocess.run([str(exe)], input=text, capture_output=True, text=True, timeout=60)
+        assert r.returncode == 0, r.stderr[-3000:]
+        return [dict(zip(KEYS, map(int, line.split()))) for line in r.stdout.splitlines()]
+
+    return run
+
+
+GRIDS = [(64, 128), (128, 64), (128, 128), (64, 256), (256, 128), (333, 217), (512, 512),
+         (1024, 1024), (2048, 1024), (9, 1030), (3, 700), (1, 100000), (1024, 9000)]
+
+
+def test_last_step_of_any_limit(plan):
+    limits = [0, 7, 100, 10**6, 10**8, 10**9, 2**31 - 1]
+    cases = [(nx, ny, lim) for nx, ny in GRIDS for lim in limits]
+    chains = 0
+    for (nx, ny, lim), p in zip(cases, plan(cases)):
+        if not p["chain"]:
+            continue
+        chains += 1
+        stages = 2 * p["q"]
+        ptot = p["g"] * stages
+        st = lim % ptot
+        end = st // stages * p["span"] + 2 * (st % stages) + lim // ptot * p["b"] + p["a"] + p["b"]
+        assert p["end"] == end, (nx, ny, lim)
+        # a line is kept apart from its reader, and 32 bits hold every step the
+        # kernel can reach (2^30) with what it adds to one
+        assert p["g"] * p["span"] <= p["b"] and ptot < p["b"]
+        assert 2**30 + 2 * (p["le"] + p["b"] + p["span"] * p["g"]) < 2**31
+    assert chains > 40
