@@ -218,7 +218,7 @@ LIB_PATH = os.path.join(PKG_DIR, "libhydrogpu.so")
 # include/hydro_noalloc.h declare.
 EXPORTS = [
     "hg3_config_default", "hg3_config_parse", "hg3_create", "hg3_destroy", "hg3_last_error",
-    "hg3_step", "hg3_get_field", "hg3_set_field",
+    "hg3_step", "hg3_get_field", "hg3_set_field", "hg3_set_wait_polls", "hg3_wait_give_ups",
     "hg_get_config", "hg_get_progress", "hg_get_iteration_history",
     "hg_output_config_default", "hg_output_config_parse", "hg_output_open",
     "hg_output_write_results", "hg_output_close", "hg_output_last_error", "hg_vts_write",
@@ -228,6 +228,8 @@ EXPORTS = [
     "hg_fluid_start_step", "hg_fluid_iterate", "hg_fluid_is_converged",
     "hg_fluid_finish_step", "hg_advect_substep", "hg_update_properties",
     "hg_calc_stats", "hg_step", "hg_last_step_timing", "hg_time_kernel", "hg_batch_run",
+    "hg_set_wait_polls", "hg_wait_give_ups",
+    "hg_poisson_set_wait_polls", "hg_poisson_wait_give_ups",
     "hg_stencil_solve", "hg_stencil_solve_noalloc", "hg_poisson_create", "hg_poisson_destroy",
     "hg_poisson_solve", "hg_poisson_time_kernel",
     "hg_train_opts_default", "hg_poisson_train", "hg_train_pressure_net",
@@ -255,6 +257,9 @@ def _declare(lib):
         "hg3_step": (ctypes.c_int, [vp, _P(HgStepStats)]),
         "hg3_get_field": (ctypes.c_int, [vp, ctypes.c_int32, _dp, ctypes.c_size_t]),
         "hg3_set_field": (ctypes.c_int, [vp, ctypes.c_int32, _dp, ctypes.c_size_t]),
+        **{f"{p}_set_wait_polls": (ctypes.c_int, [vp, ctypes.c_int32])
+           for p in ("hg", "hg3", "hg_poisson")},
+        **{f"{p}_wait_give_ups": (ctypes.c_int64, [vp]) for p in ("hg", "hg3", "hg_poisson")},
         "hg_config_parse": (ctypes.c_int, [_P(HgConfig), ctypes.c_char_p,
                                            ctypes.c_char_p, ctypes.c_size_t]),
         "hg_solver_from_name": (ctypes.c_int32, [ctypes.c_char_p]),

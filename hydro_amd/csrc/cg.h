@@ -12,6 +12,8 @@
 
 #include <string>
 
+#include "wait_guard.h"
+
 namespace hg {
 
 class Precond;
@@ -67,6 +69,8 @@ class CgSolver {
   void Apply(const double* d_x, double* d_y);
   const double* kx() const { return kx_; }
   const double* ky() const { return ky_; }
+  WaitGuard& waits() { return waits_; }
+  const WaitGuard& waits() const { return waits_; }
   int nx() const { return nx_; }
   int ny() const { return ny_; }
   hipStream_t stream() const { return stream_; }
@@ -86,6 +90,7 @@ class CgSolver {
   double* part_ = nullptr;   // block partials
   void* scal_ = nullptr;     // device scalars (CgScalars)
   void* words_ = nullptr;    // exchange and z words of the one-launch Jacobi-PCG
+  WaitGuard waits_;          // of the one-launch solves
   void* host_scal_ = nullptr;  // pinned mirror
   int blocks_;
   int last_fcg_iters_ = 5;  // iterations of the last flexible solve

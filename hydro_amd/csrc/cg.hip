@@ -308,7 +308,7 @@ template <class T, int K>
 __global__ void __launch_bounds__(kWholeThreads)
 KPcgWhole(int nx, int ny, int C, const T* __restrict__ kx, const T* __restrict__ ky,
           const T* __restrict__ dinv, const T* __restrict__ r0, T* __restrict__ x,
-          T* __restrict__ xsave, Word* zw, Word* words, CgScalars* sc) {
+          T* __restrict__ xsave, Word* zw, Word* words, int spin, CgScalars* sc) {
   extern __shared__ double whole_lds[];
   __shared__ int gave_up;
   T* const ps = reinterpret_cast<T*>(whole_lds);  // p of the cells c0 - nx ..
@@ -351,7 +351,7 @@ KPcgWhole(int nx, int ny, int C, const T* __restrict__ kx, const T* __restrict__
           zs[h] = __uint_as_float(unsigned(lo));
           if (unsigned(lo >> 32) == tag) break;
         }
-        if (m == kWholeSpin) return false;
+        if (m == spin) return false;
       }
     }
     return true;
@@ -380,7 +380,7 @@ KPcgWhole(int nx, int ny, int C, const T* __restrict__ kx, const T* __restrict__
     dots[1] += double(r[i]) * double(r[i]);
   }
   auto None = [](const auto&) { return 0.; };
-  if (!Exchange<SumFold>(dots, quot, tag, words, &gave_up, None, [] {}, Halo)) return;
+  if (!Exchange<SumFold>(dots, quot, tag, words, spin, &gave_up, None, [] {}, Halo)) return;
   int k = 0;
   for (;; ++k) {
     const double rz = dots[0], rr = dots[1];
@@ -416,7 +416,7 @@ KPcgWhole(int nx, int ny, int C, const T* __restrict__ kx, const T* __restrict__
       }
     }
     ++tag;
-    if (!Exchange<SumFold>(pq, quot, tag, words, &gave_up,
+    if (!Exchange<SumFold>(pq, quot, tag, words, spin, &gave_up,
                          [&](const auto& s) { return rz / s[0]; }, [] {}, [] { return true; }))
       return;
     const T a = T(quot);
@@ -433,7 +433,7 @@ KPcgWhole(int nx, int ny, int C, const T* __restrict__ kx, const T* __restrict__
         dots[1] += double(r[i]) * double(r[i]);
       }
     }
-    if (!Exchange<SumFold>(dots, quot, tag, words, &gave_up,
+    if (!Exchange<SumFold>(dots, quot, tag, words, spin, &gave_up,
                          [&](const auto& s) { return s[0] / rz; }, [] {}, Halo))
       return;
   }
@@ -1003,17 +1003,21 @@ bool CgSolver::WholePcg(const T* kx, const T* ky, const T* dinv, const T* r, T* 
   if (n_ > kWholeMaxCells) return false;
   const WholeSplit split = SplitWhole(int(n_));
   const int k = split.k, c = split.cells;
-  if (long(c) + 4L * nx_ > kWholeLds) return false;
+  if (long(c) + 4L * nx_ > kWholeLds || !waits_.Try()) return false;
   Word* const words = (Word*)words_;
   Word* const zw = words + kWholeWords;
   CgScalars* const sc = (CgScalars*)scal_;
   auto launch = [&](auto kernel) {
     kernel<<<split.wgs, kWholeThreads, size_t(c + 4 * nx_) * sizeof(T), stream_>>>(
-        nx_, ny_, c, kx, ky, dinv, r, x, xsave, zw, words, sc);
+        nx_, ny_, c, kx, ky, dinv, r, x, xsave, zw, words, waits_.Polls(kWholeSpin), sc);
   };
   launch(k == 1 ? KPcgWhole<T, 1> : k == 2 ? KPcgWhole<T, 2> : KPcgWhole<T, 4>);
   ReadScalars();
-  if (((CgScalars*)host_scal_)->done) return true;
+  if (((CgScalars*)host_scal_)->done) {
+    waits_.Finished();
+    return true;
+  }
+  waits_.GaveUp();
   KWholeReset<<<1, 64, 0, stream_>>>(words, 2u * unsigned(max_iters) + 4u);
   HG_CHECK(hipMemcpyAsync(x, xsave, size_t(n_) * sizeof(T), hipMemcpyDeviceToDevice, stream_));
   return false;

@@ -27,6 +27,7 @@
 #include "kernels.h"
 #include "learned_net.h"
 #include "mg.h"
+#include "wait_guard.h"
 
 #define HG_CHECK(x)                                                                  \
   do {                                                                               \
@@ -204,6 +205,7 @@ struct hg_ctx {
   // workspace of the gauss_seidel solves (a context with one of them)
   double* sor_ws = nullptr;
   long sor_doubles = 0;
+  hg::WaitGuard sor_waits;
   double* lu_ws = nullptr;  // lu: LaunchLuWavefront's workspace
   long lu_doubles = 0;
   hg::JacobiWork jw{};
@@ -676,17 +678,22 @@ void SolveRowsIterative(hg_ctx* c, int32_t solver, hg::Rows rows, const double* 
     *iters = it;
     return;
   }
-  for (bool retry : {false, true}) {
+  for (bool may_wait : {solver == HG_SOLVER_GAUSS_SEIDEL && c->sor_waits.Try(), false}) {
+    bool waited = false;
     if (solver == HG_SOLVER_GAUSS_SEIDEL)
-      hg::LaunchSor(c->st, nx, ny, rows, k, x, tol, limit, omega, c->gs_info, c->sor_ws,
-                    c->sor_doubles, retry);
+      waited = hg::LaunchSor(c->st, nx, ny, rows, k, x, tol, limit, omega, c->gs_info, c->sor_ws,
+                             c->sor_doubles, may_wait, c->sor_waits.Polls(-1));
     else if (solver == HG_SOLVER_LU_RELAXED)
       hg::LaunchLuRelaxed(c->st, nx, ny, rows, k, x, w.xa, w.xb, tol, limit, omega, c->gs_info);
     else
       throw HgError(HG_ERR_UNSUPPORTED, "not an iterative row solver");
     HG_CHECK(hipMemcpyAsync(c->info_h, c->gs_info, 16, hipMemcpyDeviceToHost, c->st));
     c->Sync();
-    if (c->info_h[0] != hg::kSorRetry) break;
+    if (c->info_h[0] != hg::kSorRetry) {
+      if (waited) c->sor_waits.Finished();
+      break;
+    }
+    c->sor_waits.GaveUp();
   }
   *iters = int(c->info_h[0]);
   std::memcpy(diff, &c->info_h[1], 8);
@@ -1595,6 +1602,18 @@ hg_status hg_batch_run(hg_ctx* const* ctxs, int32_t n, int32_t steps, int32_t th
   for (int32_t i = 0; i < n; ++i)
     if (rc[i] != HG_OK) return rc[i];
   return HG_OK;
+}
+
+hg_status hg_set_wait_polls(hg_ctx* c, int32_t polls) {
+  if (!c) return HG_ERR_BAD_ARG;
+  c->sor_waits.SetPolls(polls);
+  if (c->cg) c->cg->waits().SetPolls(polls);
+  return HG_OK;
+}
+
+int64_t hg_wait_give_ups(const hg_ctx* c) {
+  if (!c) return 0;
+  return c->sor_waits.give_ups() + (c->cg ? c->cg->waits().give_ups() : 0);
 }
 
 hg_status hg_time_kernel(hg_ctx* c, const char* kernel, int32_t reps, double* avg_ms) {

@@ -3,8 +3,9 @@
 // For solves of small grids that run in one launch: at most kWholeMaxWg
 // workgroups, each waiting for all others once or more per iteration.  That is a
 // quarter of the CUs, since kernels of four queues may run at once and the waits
-// need a kernel's workgroups to run together; they are bounded (kWholeSpin), and
-// a solve that gave up is run again by kernels that do not wait.  16 workgroups
+// need a kernel's workgroups to run together; they are bounded (kWholeSpin polls,
+// see wait_guard.h), and a solve that gave up is run again by kernels that do
+// not wait.  16 workgroups
 // or fewer are faster where their threads can hold the grid: 32 cost 1.3 us more
 // per iteration of two exchanges.
 #pragma once
@@ -74,8 +75,8 @@ struct MaxFold {
 // workgroup: gave up.
 template <class Fold, int NV, class Post, class All, class Others>
 __device__ __forceinline__ bool Exchange(double (&v)[NV], double& extra, unsigned tag,
-                                         Word* words, int* gave_up, Post&& post, All&& all_waves,
-                                         Others&& others) {
+                                         Word* words, int spin, int* gave_up, Post&& post,
+                                         All&& all_waves, Others&& others) {
   constexpr int kWaves = kWholeThreads / 64;  // at most 16: one row of lanes
   __shared__ double red[NV][kWaves];
   __shared__ double tot[NV + 1];
@@ -111,7 +112,7 @@ __device__ __forceinline__ bool Exchange(double (&v)[NV], double& extra, unsigne
 #pragma unroll
         for (int i = 0; i < 2 * NV; ++i) all = all && unsigned(g[i] >> 32) == tag;
         if (__all(all)) break;
-        if (n == kWholeSpin) {
+        if (n == spin) {
           ok = false;
           break;
         }

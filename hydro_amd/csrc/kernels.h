@@ -188,13 +188,15 @@ void LaunchGsWavefront(hipStream_t st, int nx, int ny, Rows a, const double* k, 
 // of `ws_doubles` doubles; with fewer than SorWorkspace(nx, ny) it keeps
 // fewer sweeps in flight, and without room for two (or where the shorter side
 // exceeds 1024 or the longer is under 8) it runs LaunchGsWavefront.
-// info[0] == kSorRetry: the workgroups of a large grid did not run together
-// and the solve gave up (or it ran for 2^30 steps); call again with `retry`.
+// True: large grid, over several workgroups that wait for each other (if `wait`),
+// each wait for `polls` polls at most (negative: the kernel's own bound).  If
+// then info[0] == kSorRetry, they did not run together and the solve gave up (or
+// it ran for 2^30 steps): call again without `wait`.
 constexpr unsigned long long kSorRetry = ~0ull;
 long SorWorkspace(int nx, int ny);
-void LaunchSor(hipStream_t st, int nx, int ny, Rows a, const double* k, double* x, double tol,
+bool LaunchSor(hipStream_t st, int nx, int ny, Rows a, const double* k, double* x, double tol,
                int limit, double omega, unsigned long long* info, double* ws, long ws_doubles,
-               bool retry = false);
+               bool wait, int polls = -1);
 // LuDecompositionRelaxed (linear.hpp:578-651) from zero, every iteration in
 // one persistent workgroup: res receives the solution; corr and f are
 // scratch cell arrays; info as for LaunchGsWavefront.

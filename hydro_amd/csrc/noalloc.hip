@@ -130,9 +130,9 @@ hg_status hg_stencil_solve_noalloc(int32_t nx, int32_t ny, const double* s, cons
       // the solver's workspace: what the scratch array holds behind the header
       const long ws = long((kScratchBytes - off_arr) / 8);
       unsigned long long h[2] = {0, 0};
-      for (bool retry : {false, true}) {
+      for (bool wait : {true, false}) {
         hg::LaunchSor(st, nx, ny, rows, k, x, opts->tolerance, limit, opts->relaxation_factor,
-                      info, a0, ws, retry);
+                      info, a0, ws, wait);
         if (!check(hipMemcpyAsync(h, info, 16, hipMemcpyDeviceToHost, st)) ||
             !check(hipStreamSynchronize(st)))
           return Fail(HG_ERR_HIP, "iteration info readback failed");

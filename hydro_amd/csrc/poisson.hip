@@ -105,10 +105,10 @@ hg_status hg_stencil_solve(int32_t nx, int32_t ny, const double* s, const double
         const long nws = hg::SorWorkspace(nx, ny);
         row_ws.reset(new DevBuf(size_t(nws)));
         unsigned long long h[2];
-        for (bool retry : {false, true}) {
+        for (bool wait : {true, false}) {
           hg::LaunchSor(st, nx, ny, rows, dk.p, dx.p, opts->tolerance, opts->max_iters,
                         opts->relaxation_factor, (unsigned long long*)info.p, row_ws->p, nws,
-                        retry);
+                        wait);
           HG_CHECK(hipMemcpyAsync(h, info.p, 16, hipMemcpyDeviceToHost, st));
           HG_CHECK(hipStreamSynchronize(st));
           if (h[0] != hg::kSorRetry) break;
@@ -220,6 +220,16 @@ hg_status hg_poisson_create(int32_t nx, int32_t ny, const double* kx, const doub
 }
 
 void hg_poisson_destroy(hg_poisson* ps) { delete ps; }
+
+hg_status hg_poisson_set_wait_polls(hg_poisson* ps, int32_t polls) {
+  if (!ps) return HG_ERR_BAD_ARG;
+  ps->cg->waits().SetPolls(polls);
+  return HG_OK;
+}
+
+int64_t hg_poisson_wait_give_ups(const hg_poisson* ps) {
+  return ps ? ps->cg->waits().give_ups() : 0;
+}
 
 hg_status hg_poisson_solve(hg_poisson* ps, const double* rhs, double* p,
                            const hg_solve_opts* opts, hg_solve_stats* stats) {

@@ -452,7 +452,7 @@ KSorChain(SorChain ch, const double2* __restrict__ oc, const double2* __restrict
       seen = AgentLoad(progress + 16 * src);
       if (seen >= need) break;
       if (AgentLoad(stop) != kNever) return true;
-      if (k == kSpin) {
+      if (k == ch.spin) {
         __hip_atomic_fetch_min(stop, -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         return false;
       }
@@ -609,15 +609,15 @@ KSorChain(SorChain ch, const double2* __restrict__ oc, const double2* __restrict
 
 long SorWorkspace(int nx, int ny) { return SorWorkspaceDoubles(nx, ny); }
 
-void LaunchSor(hipStream_t st, int nx, int ny, Rows a, const double* k, double* x, double tol,
+bool LaunchSor(hipStream_t st, int nx, int ny, Rows a, const double* k, double* x, double tol,
                int limit, double omega, unsigned long long* info, double* ws, long ws_doubles,
-               bool retry) {
+               bool wait, int polls) {
   const SorPlan p = PlanSor(nx, ny, limit, ws ? ws_doubles : 0);
   const SorPlan c = PlanChain(nx, ny, limit, ws ? ws_doubles : 0);
-  const bool many = !retry && UseChain(p, c);
+  const bool many = wait && UseChain(p, c);
   if (!p.ok && !many) {
     LaunchGsWavefront(st, nx, ny, a, k, x, tol, limit, omega, info);
-    return;
+    return false;
   }
   const long n = long(nx) * ny;
   const int tr = p.tr ? 1 : 0;
@@ -627,7 +627,8 @@ void LaunchSor(hipStream_t st, int nx, int ny, Rows a, const double* k, double* 
   const unsigned grid = unsigned((n + 255) / 256);
   KSorPack<<<grid, 256, 0, st>>>(nx, ny, a, k, tr, oc, xn, ck, many ? ws : nullptr);
   if (many) {
-    SorChain ch{c.a, c.b, (c.a + 63) / 64 * 64, c.Q, c.G, c.span, c.le, limit, 0};
+    SorChain ch{c.a, c.b, (c.a + 63) / 64 * 64, c.Q, c.G, c.span, c.le, limit, 0,
+                polls < 0 ? kSpin : polls};
     const int threads = c.Q * ch.ap;
     const size_t lds = size_t(2) * c.Q * (c.a + 2) * sizeof(double2) + size_t(8) * c.Q * 8;
     double *out = ring, *logs = out + n;
@@ -643,7 +644,7 @@ void LaunchSor(hipStream_t st, int nx, int ny, Rows a, const double* k, double* 
         launch(tr ? KSorChain<true, 512> : KSorChain<false, 512>);
     }
     KSorUnpack<<<grid, 256, 0, st>>>(nx, ny, tr, out, nullptr, x);
-    return;
+    return true;
   }
   const int threads = (p.Q * p.a + 63) / 64 * 64;
   const size_t lds = size_t(2) * p.Q * (p.a + 2) * sizeof(double2) +
@@ -655,6 +656,7 @@ void LaunchSor(hipStream_t st, int nx, int ny, Rows a, const double* k, double* 
     KSorPipe<false><<<1, threads, lds, st>>>(p.a, p.b, p.Q, p.rounds, oc, xn, ck, ring, tol,
                                              limit, omega, ws, info);
   KSorUnpack<<<grid, 256, 0, st>>>(nx, ny, tr, ring, ws, x);
+  return false;
 }
 
 }  // namespace hg

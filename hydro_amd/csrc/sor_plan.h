@@ -33,6 +33,7 @@ struct SorChain {
   int a, b, ap;           // short and long side, line padded to waves
   int Q, G, span, le;     // thread groups per workgroup, workgroups, log rows
   int limit, tail;
+  int spin;               // bound on a wait's polls
 };
 
 struct SorPlan {

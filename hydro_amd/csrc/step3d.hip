@@ -32,6 +32,7 @@
 #include "../../include/hydro_gpu3d.h"
 #include "exchange.h"
 #include "mg3d.h"
+#include "wait_guard.h"
 
 #define H3_CHECK(x)                                                                    \
   do {                                                                                 \
@@ -577,7 +578,7 @@ constexpr long kJacWholeCells = 2L * kWholeThreads * hg::kWholeMaxWg;
 template <int K>
 __global__ void __launch_bounds__(kWholeThreads)
 KJacobiWhole(G g, int C, Rows A, const double* __restrict__ kc, double* __restrict__ x,
-             double omega, double tol, int limit, Word* words, int* state) {
+             double omega, double tol, int limit, Word* words, int spin, int* state) {
   extern __shared__ double xs[];  // x of the cells c0 - plane .., then a 0
   __shared__ int gave_up;
   constexpr int NT = kWholeThreads;
@@ -644,7 +645,7 @@ KJacobiWhole(G g, int C, Rows A, const double* __restrict__ kc, double* __restri
           }
           break;
         }
-        if (m == kWholeSpin) return false;
+        if (m == spin) return false;
       }
     }
     return true;
@@ -676,8 +677,8 @@ KJacobiWhole(G g, int C, Rows A, const double* __restrict__ kc, double* __restri
       for (int i = 0; i < K; ++i)
         if (in[i]) xs[plane + threadIdx.x + i * NT] = xn[i];
     };
-    if (!Exchange<MaxFold>(m, unused, tag, words, &gave_up, [](const auto&) { return 0.; }, Put,
-                           Halo))
+    if (!Exchange<MaxFold>(m, unused, tag, words, spin, &gave_up,
+                           [](const auto&) { return 0.; }, Put, Halo))
       return;
     if (!(m[0] > tol)) {
       iters = s;
@@ -1204,6 +1205,7 @@ struct hg3_ctx {
   unsigned long long* jdiff;
   int* jstate;
   Word* jwords = nullptr;  // KJacobiWhole's words, where the grid is small enough
+  hg::WaitGuard waits;
   int* flag;
   // cg
   double *cb, *cr, *cz, *cp, *cq, *cx;
@@ -1458,16 +1460,21 @@ int SolveJacobi(hg3_ctx* c, const Rows& R, const double* k, double* x) {
   const int limit = cfg.lu_relaxed_num_iters_limit;
   const double tol = cfg.lu_relaxed_tolerance, omega = cfg.lu_relaxed_relaxation_factor;
   H3_CHECK(hipMemsetAsync(c->jstate, 0, 4 * sizeof(int), c->st));
-  if (c->jwords) {
+  if (c->jwords && c->waits.Try()) {
     const WholeSplit w = SplitWhole(int(c->nc), 2);
     auto launch = [&](auto kernel) {
       kernel<<<w.wgs, kWholeThreads, size_t(w.cells + 2 * c->g.nx * c->g.ny + 1) * 8, c->st>>>(
-          c->g, w.cells, R, k, x, omega, tol, limit, c->jwords, c->jstate);
+          c->g, w.cells, R, k, x, omega, tol, limit, c->jwords, c->waits.Polls(kWholeSpin),
+          c->jstate);
     };
     launch(w.k == 1 ? KJacobiWhole<1> : KJacobiWhole<2>);
     H3_CHECK(hipMemcpyAsync(c->state_h, c->jstate, 4 * sizeof(int), hipMemcpyDeviceToHost, c->st));
     c->Sync();
-    if (c->state_h[0]) return c->state_h[1];
+    if (c->state_h[0]) {
+      c->waits.Finished();
+      return c->state_h[1];
+    }
+    c->waits.GaveUp();
     KWholeReset<<<1, 64, 0, c->st>>>(c->jwords, unsigned(limit) + 2u);
   }
   H3_CHECK(hipMemsetAsync(c->jdiff, 0, size_t(kJacSlots) * 8, c->st));
@@ -1977,6 +1984,14 @@ void hg3_destroy(hg3_ctx* c) { delete c; }
 const char* hg3_last_error(const hg3_ctx* c) {
   return c ? c->err.c_str() : g_create_error3.c_str();
 }
+
+hg_status hg3_set_wait_polls(hg3_ctx* c, int32_t polls) {
+  if (!c) return HG_ERR_BAD_ARG;
+  c->waits.SetPolls(polls);
+  return HG_OK;
+}
+
+int64_t hg3_wait_give_ups(const hg3_ctx* c) { return c ? c->waits.give_ups() : 0; }
 
 hg_status hg3_step(hg3_ctx* c, hg_step_stats* s) {
   if (!c) return HG_ERR_BAD_ARG;

@@ -172,6 +172,15 @@ class Hydro:
         _raise(self.lib, self.ctx, rc, "hg_time_kernel")
         return ms.value
 
+    def set_wait_polls(self, polls):
+        """Bounds the waits inside this object's one-launch solves (negative: the
+        default)."""
+        self.lib.hg_set_wait_polls(self.ctx, polls)
+
+    def wait_give_ups(self):
+        """Solves that gave up waiting and were run again by kernels that do not."""
+        return self.lib.hg_wait_give_ups(self.ctx)
+
     def timing(self):
         f, a, p = ctypes.c_double(), ctypes.c_double(), ctypes.c_double()
         self.lib.hg_last_step_timing(self.ctx, ctypes.byref(f), ctypes.byref(a), ctypes.byref(p))
@@ -275,6 +284,15 @@ class Poisson:
         rc = self.lib.hg_poisson_time_kernel(self.ps, kernel.encode(), reps, ctypes.byref(ms))
         _raise(self.lib, None, rc, "hg_poisson_time_kernel")
         return ms.value
+
+    def set_wait_polls(self, polls):
+        """Bounds the waits inside this object's one-launch solves (negative: the
+        default)."""
+        self.lib.hg_poisson_set_wait_polls(self.ps, polls)
+
+    def wait_give_ups(self):
+        """Solves that gave up waiting and were run again by kernels that do not."""
+        return self.lib.hg_poisson_wait_give_ups(self.ps)
 
     def train(self, rhs_count=None, mg_iters=None, steps=None, lr=None, seed=None, flags=None):
         """Trains the learned preconditioner on this operator; returns the
@@ -457,6 +475,15 @@ class Hydro3:
         v = np.ascontiguousarray(values, dtype=np.float64)
         _raise3(self.lib, self.ctx, self.lib.hg3_set_field(self.ctx, field, capi.dptr(v), v.size),
                 "hg3_set_field")
+
+    def set_wait_polls(self, polls):
+        """Bounds the waits inside this object's one-launch solves (negative: the
+        default)."""
+        self.lib.hg3_set_wait_polls(self.ctx, polls)
+
+    def wait_give_ups(self):
+        """Solves that gave up waiting and were run again by kernels that do not."""
+        return self.lib.hg3_wait_give_ups(self.ctx)
 
     def step(self):
         st = capi.HgStepStats()

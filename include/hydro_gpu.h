@@ -336,6 +336,17 @@ hg_status hg_last_step_timing(const hg_ctx* ctx, double* fluid_ms, double* advec
  * "KMomentum" (momentum rows of one SIMPLE iteration). */
 hg_status hg_time_kernel(hg_ctx* ctx, const char* kernel, int32_t reps, double* avg_ms);
 
+/* Solves that wait inside a kernel (no reference counterpart).  Some solves of
+ * this context (gauss_seidel on larger grids, cg on smaller ones) run in one
+ * launch whose workgroups wait for each other.  Where other processes keep some
+ * of them off the GPU, a wait ends after a bounded number of polls, the solve is
+ * run again by kernels that do not wait, with the same result, and the next
+ * ones do not try for a while.  hg_set_wait_polls sets the bound (negative: the
+ * default, 0.1 s and more; 0: give up at the first poll that would wait) and
+ * lets solves try again; hg_wait_give_ups counts the solves that gave up. */
+hg_status hg_set_wait_polls(hg_ctx* ctx, int32_t polls);
+int64_t hg_wait_give_ups(const hg_ctx* ctx);
+
 /* ---- many cases at once (replaces the console's experiment threads,
  * console.cpp:162-178 and :923, which run each experiment's step loop on its
  * own std::thread, at most max_threads_number at a time) ---------------------
@@ -389,6 +400,9 @@ typedef struct hg_poisson hg_poisson;
 hg_status hg_poisson_create(int32_t nx, int32_t ny, const double* kx, const double* ky,
                             hg_poisson** out);
 void hg_poisson_destroy(hg_poisson* ps);
+/* As hg_set_wait_polls and hg_wait_give_ups, for this object's cg solves. */
+hg_status hg_poisson_set_wait_polls(hg_poisson* ps, int32_t polls);
+int64_t hg_poisson_wait_give_ups(const hg_poisson* ps);
 /* Solves A p = rhs (rhs projected to zero mean) from p = 0 to the relative
  * residual opts->tolerance (true FP64 residual).  opts->solver is
  * HG_SOLVER_CG (Jacobi-PCG), HG_SOLVER_FCG_LEARNED or HG_SOLVER_FCG_MG.

@@ -64,6 +64,10 @@ void hg3_destroy(hg3_ctx* ctx);
 const char* hg3_last_error(const hg3_ctx* ctx);
 /* hydro::step (hydro2d.hpp:1531-1621). */
 hg_status hg3_step(hg3_ctx* ctx, hg_step_stats* stats);
+/* As hg_set_wait_polls and hg_wait_give_ups (hydro_gpu.h), for the jacobi
+ * pressure solves of smaller grids. */
+hg_status hg3_set_wait_polls(hg3_ctx* ctx, int32_t polls);
+int64_t hg3_wait_give_ups(const hg3_ctx* ctx);
 /* Fields of the time_curr layer, by HG_FIELD_* id; n must equal the field's
  * size (cells or faces).  set accepts velocity, pressure, flux and partial
  * densities and resets the previous time layer to the same values. */
