@@ -106,8 +106,7 @@ class CgSolver {
                          Precond* pc, bool warm);
   void Prepare(const double* b, double* x, bool project, bool warm);
   template <class T>
-  bool WholePcg(const T* kx, const T* ky, const T* dinv, const T* r, T* x, T* xsave,
-                int max_iters);
+  bool WholePcg(const T* kx, const T* ky, const T* dinv, const T* r, T* x, T* xsave);
   int JacobiPcg64(double* x, int max_iters);
   int InnerFp32(double tol_inner, int max_iters, Precond* pc, bool* pc_failed);
   double ResidualFp64(const double* b, const double* x, double* r);  // returns ||r||^2

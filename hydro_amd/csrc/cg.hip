@@ -998,8 +998,7 @@ void CgSolver::Prepare(const double* b, double* x, bool project, bool warm) {
 // The whole Jacobi-PCG solve in one launch (KPcgWhole), where the grid fits
 // and the workgroups ran together; else false, with x as it was.
 template <class T>
-bool CgSolver::WholePcg(const T* kx, const T* ky, const T* dinv, const T* r, T* x, T* xsave,
-                        int max_iters) {
+bool CgSolver::WholePcg(const T* kx, const T* ky, const T* dinv, const T* r, T* x, T* xsave) {
   if (n_ > kWholeMaxCells) return false;
   const WholeSplit split = SplitWhole(int(n_));
   const int k = split.k, c = split.cells;
@@ -1018,7 +1017,7 @@ bool CgSolver::WholePcg(const T* kx, const T* ky, const T* dinv, const T* r, T* 
     return true;
   }
   waits_.GaveUp();
-  KWholeReset<<<1, 64, 0, stream_>>>(words, 2u * unsigned(max_iters) + 4u);
+  WholeReset(words, kWholeWords + 2 * n_, stream_);
   HG_CHECK(hipMemcpyAsync(x, xsave, size_t(n_) * sizeof(T), hipMemcpyDeviceToDevice, stream_));
   return false;
 }
@@ -1030,7 +1029,7 @@ int CgSolver::JacobiPcg64(double* x, int max_iters) {
   Parts pt = MakeParts(part_, nb);
   CgScalars* sc = (CgScalars*)scal_;
   CgScalars* hs = (CgScalars*)host_scal_;
-  if (WholePcg<double>(kx_, ky_, dinv_, r_, x, pb_, max_iters)) return hs->iter;
+  if (WholePcg<double>(kx_, ky_, dinv_, r_, x, pb_)) return hs->iter;
   KPcgStart<double><<<nb, kB, 0, stream_>>>(w, r_, dinv_, z_, pa_, pt);
   double* pold = pa_;
   double* pnew = pb_;
@@ -1043,7 +1042,7 @@ int CgSolver::JacobiPcg64(double* x, int max_iters) {
       std::swap(pold, pnew);
     }
     ReadScalars();
-    if (hs->done || k >= max_iters + batch) break;
+    if (hs->done || k - batch >= max_iters) break;
   }
   return hs->iter;
 }
@@ -1135,7 +1134,7 @@ CgResult CgSolver::SolveFlexible(const double* b, double* x, double tol, int max
       std::swap(pold, pnew);
     }
     ReadScalars();
-    if (hs->done || k >= max_iters + batch) break;
+    if (hs->done || k - batch >= max_iters) break;
     batch = 2;
   }
   res.iterations = hs->iter;
@@ -1166,8 +1165,7 @@ int CgSolver::InnerFp32(double tol_inner, int max_iters, Precond*, bool*) {
   KSetup<<<1, 64, 0, stream_>>>(sc, tol_inner * tol_inner, max_iters);
   KPcgStart<float><<<nb, kB, 0, stream_>>>(w, r32_, dinv32_, z32_, pa32_, pt);
   KInnerBB<<<1, kB, 0, stream_>>>(pt, sc);
-  if (WholePcg<float>(kx32_, ky32_, dinv32_, r32_, e32_, pb32_, max_iters))
-    return hs->iter;
+  if (WholePcg<float>(kx32_, ky32_, dinv32_, r32_, e32_, pb32_)) return hs->iter;
   KPcgStart<float><<<nb, kB, 0, stream_>>>(w, r32_, dinv32_, z32_, pa32_, pt);
   float* pold = pa32_;
   float* pnew = pb32_;
@@ -1181,7 +1179,7 @@ int CgSolver::InnerFp32(double tol_inner, int max_iters, Precond*, bool*) {
       std::swap(pold, pnew);
     }
     ReadScalars();
-    if (hs->done || k >= max_iters + batch) break;
+    if (hs->done || k - batch >= max_iters) break;
   }
   return hs->iter;
 }

@@ -10,6 +10,8 @@
 // per iteration of two exchanges.
 #pragma once
 
+#include <algorithm>
+
 #include "device_common.h"
 
 namespace hg {
@@ -149,12 +151,16 @@ __device__ __forceinline__ bool FinishWhole(Word* words, unsigned tag) {
   return true;
 }
 
-// After a solve that gave up: no tag of it is used again.
-static __global__ void KWholeReset(Word* words, unsigned tags) {
-  if (threadIdx.x == 0) {
-    words[kWholeDone] = 0;
-    words[kWholeEpoch] = Word(unsigned(words[kWholeEpoch]) + tags);
-  }
+// After a solve that gave up: no word of it is taken for one of the next solve.
+// Its tags, from the epoch on, are used again, so every word goes back to the
+// epoch, which the next solve has behind it.
+static __global__ void __launch_bounds__(256) KWholeReset(Word* words, long n) {
+  const Word epoch = words[kWholeEpoch];
+  for (long i = blockIdx.x * 256l + threadIdx.x; i < n; i += gridDim.x * 256l)
+    if (i != kWholeEpoch) words[i] = i == kWholeDone ? Word(0) : epoch << 32;
+}
+inline void WholeReset(Word* words, long n, hipStream_t st) {
+  KWholeReset<<<unsigned(std::min((n + 255) / 256, 256l)), 256, 0, st>>>(words, n);
 }
 
 }  // namespace hg

@@ -860,7 +860,7 @@ Fcg3Result Mg3Fcg::Solve(double* const (&t)[7], const double* b, double* x, doub
     }
     M3_CHECK(hipMemcpyAsync(hs, sc, sizeof(Scal), hipMemcpyDeviceToHost, st));
     M3_CHECK(hipStreamSynchronize(st));
-    if (hs->done || k >= max_iters + batch) break;
+    if (hs->done || k - batch >= max_iters) break;
     batch = 2;
   }
   Fcg3Result res;

@@ -52,11 +52,11 @@ using hg::kWholeLds;
 using hg::kWholeSpin;
 using hg::kWholeThreads;
 using hg::kWholeWords;
-using hg::KWholeReset;
 using hg::MaxFold;
 using hg::SplitWhole;
 using hg::TagLoad;
 using hg::TagStore;
+using hg::WholeReset;
 using hg::WholeSplit;
 using hg::Word;
 
@@ -1475,7 +1475,7 @@ int SolveJacobi(hg3_ctx* c, const Rows& R, const double* k, double* x) {
       return c->state_h[1];
     }
     c->waits.GaveUp();
-    KWholeReset<<<1, 64, 0, c->st>>>(c->jwords, unsigned(limit) + 2u);
+    WholeReset(c->jwords, kWholeWords + 4 * c->nc, c->st);
   }
   H3_CHECK(hipMemsetAsync(c->jdiff, 0, size_t(kJacSlots) * 8, c->st));
   H3_CHECK(hipMemsetAsync(c->corr, 0, size_t(c->nc) * 8, c->st));

@@ -46,6 +46,25 @@ def test_cg_gives_up(gpu, nx, ny, precision):
     assert np.array_equal(p3, p0) and s3.iterations == s0.iterations
 
 
+@pytest.mark.parametrize("precision", [0, 1])
+def test_cg_gives_up_without_an_iteration_cap(gpu, precision):
+    """The cap of 2^31 - 1 iterations, where twice the cap and the cap plus a
+    batch are past 32 bits: the solve that gave up meets its tolerance, and so do
+    solves on the same words afterwards, with the bits of the first."""
+    print(f"case: cg 129x128 precision {precision}, no cap", flush=True)
+    ps, rhs = poisson(129, 128)
+    args = dict(solver="cg", tol=1e-6, precision=precision, max_iters=2**31 - 1)
+    p0, s0 = ps.solve(rhs, **args)
+    for _ in range(3):
+        ps.set_wait_polls(0)
+        p1, s1 = ps.solve(rhs, **args)
+        assert s1.converged and s1.iterations > 32
+        ps.set_wait_polls(-1)
+        p2, s2 = ps.solve(rhs, **args)
+        assert np.array_equal(p2, p0) and s2.iterations == s0.iterations
+    assert ps.wait_give_ups() == 3
+
+
 def test_give_ups_are_remembered(gpu):
     print("case: cg 64x64, give-ups in a row", flush=True)
     ps, rhs = poisson(64, 64)
