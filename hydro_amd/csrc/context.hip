@@ -277,6 +277,20 @@ struct hg_ctx {
     allocs.push_back(p);
     return (double*)p;
   }
+  // A workspace that the solvers can do without: *held doubles, 0 where there is
+  // no room for them.
+  double* TryAlloc(long n, long* held) {
+    void* p = nullptr;
+    *held = 0;
+    if (n < 1) return nullptr;
+    if (hipMalloc(&p, size_t(n) * sizeof(double)) != hipSuccess) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
+    allocs.push_back(p);
+    *held = n;
+    return (double*)p;
+  }
   float* AllocF(long n) {
     void* p = nullptr;
     HG_CHECK(hipMalloc(&p, size_t(std::max<long>(n, 1)) * sizeof(float)));
@@ -1175,17 +1189,6 @@ hg_status hg_create(const hg_config* cfg_in, hg_ctx** out) {
     c->rs_d = (unsigned long long*)c->Alloc(1);
     c->nan_d = (int*)c->Alloc(1);
     c->gs_info = (unsigned long long*)c->Alloc(2);
-    if (cfg.linear_solver_pressure == HG_SOLVER_GAUSS_SEIDEL ||
-        cfg.linear_solver_velocity == HG_SOLVER_GAUSS_SEIDEL ||
-        (cfg.heat_enable && cfg.linear_solver_heat == HG_SOLVER_GAUSS_SEIDEL)) {
-      c->sor_doubles = hg::SorWorkspace(cfg.nx, cfg.ny);
-      if (c->sor_doubles > 0) c->sor_ws = c->Alloc(c->sor_doubles);
-    }
-    if (cfg.linear_solver_pressure == HG_SOLVER_LU || cfg.linear_solver_velocity == HG_SOLVER_LU ||
-        (cfg.heat_enable && cfg.linear_solver_heat == HG_SOLVER_LU)) {
-      c->lu_doubles = hg::LuWorkspace(cfg.nx, cfg.ny);
-      if (c->lu_doubles > 0) c->lu_ws = c->Alloc(c->lu_doubles);
-    }
     c->jw.xa = c->Alloc(nc);
     c->jw.xb = c->Alloc(nc);
     c->jw.diff = (unsigned long long*)c->Alloc(cfg.lu_relaxed_num_iters_limit + 2);
@@ -1200,6 +1203,18 @@ hg_status hg_create(const hg_config* cfg_in, hg_ctx** out) {
     if (lsp == HG_SOLVER_FCG_LEARNED || lsp == HG_SOLVER_FCG_MG)
       c->mg.reset(new hg::MgPrecond(cfg.nx, cfg.ny, c->cg->kx32(), c->cg->ky32(),
                                     c->cg->dinv32()));
+    // the row solvers' workspaces, after everything the context cannot do without
+    auto uses = [&](int32_t solver) {
+      return lsp == solver || cfg.linear_solver_velocity == solver ||
+             (cfg.heat_enable && cfg.linear_solver_heat == solver);
+    };
+    if (uses(HG_SOLVER_GAUSS_SEIDEL))
+      c->sor_ws = c->TryAlloc(
+          hg::SorWorkspace(cfg.nx, cfg.ny, cfg.lu_relaxed_num_iters_limit), &c->sor_doubles);
+    if (uses(HG_SOLVER_LU))
+      c->lu_ws = c->TryAlloc(
+          hg::LuWorkspace(cfg.nx, cfg.ny, cfg.linear_solver_velocity == HG_SOLVER_LU ? 2 : 1),
+          &c->lu_doubles);
     Upload(c.get(), c->xn_d, c->mesh.xn);
     Upload(c.get(), c->yn_d, c->mesh.yn);
 

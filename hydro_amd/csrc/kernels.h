@@ -172,9 +172,9 @@ using RowsF = RowsT<float>;
 // up to two right-hand sides sharing the coefficients, in one workgroup.
 // x_out[r] = base[r] + x[r] when base != nullptr (the delta-form update).
 // ws: a workspace of ws_doubles doubles for the rows of one step side by side
-// (LuWorkspace; 7 per cell are enough for one right-hand side).  Without it, or
-// where the shorter side exceeds 1024, the rows are read in place.
-long LuWorkspace(int nx, int ny);
+// (LuWorkspace, for nrhs right-hand sides).  Without it, or where the shorter side
+// exceeds 1024, the rows are read in place.
+long LuWorkspace(int nx, int ny, int nrhs);
 void LaunchLuWavefront(hipStream_t st, int nx, int ny, Rows a, const double* k0,
                        const double* k1, double* x0, double* x1, const double* base0,
                        const double* base1, double* out0, double* out1, double* ws,
@@ -185,7 +185,7 @@ void LaunchLuWavefront(hipStream_t st, int nx, int ny, Rows a, const double* k0,
 void LaunchGsWavefront(hipStream_t st, int nx, int ny, Rows a, const double* k, double* x,
                        double tol, int limit, double omega, unsigned long long* info);
 // The same with many sweeps in flight (sor.hip), bit for bit, on a workspace
-// of `ws_doubles` doubles; with fewer than SorWorkspace(nx, ny) it keeps
+// of `ws_doubles` doubles; with fewer than SorWorkspace(nx, ny, limit) it keeps
 // fewer sweeps in flight, and without room for two (or where the shorter side
 // exceeds 1024 or the longer is under 8) it runs LaunchGsWavefront.
 // True: large grid, over several workgroups that wait for each other (if `wait`),
@@ -193,7 +193,7 @@ void LaunchGsWavefront(hipStream_t st, int nx, int ny, Rows a, const double* k, 
 // then info[0] == kSorRetry, they did not run together and the solve gave up (or
 // it ran for 2^30 steps): call again without `wait`.
 constexpr unsigned long long kSorRetry = ~0ull;
-long SorWorkspace(int nx, int ny);
+long SorWorkspace(int nx, int ny, int limit);
 bool LaunchSor(hipStream_t st, int nx, int ny, Rows a, const double* k, double* x, double tol,
                int limit, double omega, unsigned long long* info, double* ws, long ws_doubles,
                bool wait, int polls = -1);

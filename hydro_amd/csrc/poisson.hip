@@ -30,7 +30,15 @@ namespace {
 
 struct DevBuf {
   double* p = nullptr;
+  DevBuf() = default;
   explicit DevBuf(size_t n) { HG_CHECK(hipMalloc(&p, std::max<size_t>(n, 1) * 8)); }
+  // n doubles if there is room for them, else 0: how many it holds
+  long TryAlloc(long n) {
+    if (n > 0 && hipMalloc(&p, size_t(n) * 8) == hipSuccess) return n;
+    p = nullptr;
+    (void)hipGetLastError();
+    return 0;
+  }
   ~DevBuf() {
     if (p) (void)hipFree(p);
   }
@@ -74,7 +82,7 @@ hg_status hg_stencil_solve(int32_t nx, int32_t ny, const double* s, const double
     std::unique_ptr<void, std::function<void(void*)>> guard(
         (void*)st, [](void* p) { (void)hipStreamDestroy((hipStream_t)p); });
     DevBuf ds(N), dw(N), dc(N), de(N), dn(N), dk(N), dx(N), dx2(N), dz(N), dout(N), dtmp(N);
-    std::unique_ptr<DevBuf> row_ws;
+    DevBuf row_ws;  // a solver works without it, more slowly
     DevBuf info(2), jdiff(size_t(std::max(opts->max_iters, 0)) + 2), jstate(2);
     const double* src[6] = {s, w, c, e, n, k};
     double* dst[6] = {ds.p, dw.p, dc.p, de.p, dn.p, dk.p};
@@ -91,10 +99,9 @@ hg_status hg_stencil_solve(int32_t nx, int32_t ny, const double* s, const double
     const double* result = dx.p;
     switch (opts->solver) {
       case HG_SOLVER_LU: {
-        const long nws = hg::LuWorkspace(nx, ny);
-        row_ws.reset(new DevBuf(size_t(std::max(nws, 1L))));
+        const long nws = row_ws.TryAlloc(hg::LuWorkspace(nx, ny, 1));
         hg::LaunchLuWavefront(st, nx, ny, rows, dk.p, nullptr, dx.p, nullptr, nullptr, nullptr,
-                              nullptr, nullptr, row_ws->p, nws);
+                              nullptr, nullptr, row_ws.p, nws);
         break;
       }
       case HG_SOLVER_LU_RB:
@@ -102,12 +109,11 @@ hg_status hg_stencil_solve(int32_t nx, int32_t ny, const double* s, const double
         result = dout.p;
         break;
       case HG_SOLVER_GAUSS_SEIDEL: {
-        const long nws = hg::SorWorkspace(nx, ny);
-        row_ws.reset(new DevBuf(size_t(nws)));
+        const long nws = row_ws.TryAlloc(hg::SorWorkspace(nx, ny, opts->max_iters));
         unsigned long long h[2];
         for (bool wait : {true, false}) {
           hg::LaunchSor(st, nx, ny, rows, dk.p, dx.p, opts->tolerance, opts->max_iters,
-                        opts->relaxation_factor, (unsigned long long*)info.p, row_ws->p, nws,
+                        opts->relaxation_factor, (unsigned long long*)info.p, row_ws.p, nws,
                         wait);
           HG_CHECK(hipMemcpyAsync(h, info.p, 16, hipMemcpyDeviceToHost, st));
           HG_CHECK(hipStreamSynchronize(st));

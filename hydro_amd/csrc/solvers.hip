@@ -795,8 +795,8 @@ KLuRbRed(int nx, int ny, RowsT<T> a, const T* __restrict__ k0, const T* __restri
 
 }  // namespace
 
-long LuWorkspace(int nx, int ny) {
-  return std::min(nx, ny) <= kMaxThreads ? 9L * nx * ny : 0;
+long LuWorkspace(int nx, int ny, int nrhs) {
+  return std::min(nx, ny) <= kMaxThreads ? (nrhs == 2 ? 9L : 7L) * nx * ny : 0;
 }
 
 void LaunchLuWavefront(hipStream_t st, int nx, int ny, Rows a, const double* k0,
@@ -805,7 +805,7 @@ void LaunchLuWavefront(hipStream_t st, int nx, int ny, Rows a, const double* k0,
                        long ws_doubles) {
   const int sa = std::min(nx, ny), sb = std::max(nx, ny);
   const long n = long(nx) * ny;
-  if (sa <= kMaxThreads && ws && ws_doubles >= (k1 ? 9 : 7) * n) {
+  if (sa <= kMaxThreads && ws && ws_doubles >= LuWorkspace(nx, ny, k1 ? 2 : 1)) {
     double2* sw = reinterpret_cast<double2*>(ws);
     double2 *en = sw + n, *ck = en + n;
     double* v = reinterpret_cast<double*>(ck + n);

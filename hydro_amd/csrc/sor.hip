@@ -607,7 +607,7 @@ KSorChain(SorChain ch, const double2* __restrict__ oc, const double2* __restrict
 
 }  // namespace
 
-long SorWorkspace(int nx, int ny) { return SorWorkspaceDoubles(nx, ny); }
+long SorWorkspace(int nx, int ny, int limit) { return SorWorkspaceDoubles(nx, ny, limit); }
 
 bool LaunchSor(hipStream_t st, int nx, int ny, Rows a, const double* k, double* x, double tol,
                int limit, double omega, unsigned long long* info, double* ws, long ws_doubles,

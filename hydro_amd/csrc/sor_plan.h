@@ -22,7 +22,10 @@ constexpr int kSpin = 1 << 20;
 constexpr int kNever = 0x7fffffff;
 
 constexpr int kSorMaxG = 64, kSorMaxStages = 1024;
-constexpr long kChainMaxDoubles = 1L << 26;  // of the workspace
+// Bounds of the workspace, in doubles: 512 MB, or for a ring of two sweeps at any
+// size (about what a solve's own arrays take); 32 MB for the ring that only a
+// chain that gave up would use.
+constexpr long kSorMaxDoubles = 1L << 26, kRetryMaxDoubles = 1L << 22;
 // Workspace header, in doubles: the smallest sweep that ended the solve
 // (int `stop`), then a 64-byte line of progress per workgroup, then the max
 // |corr| of the sweep each stage last found to end it.
@@ -90,7 +93,7 @@ inline SorPlan PlanChain(int nx, int ny, int limit, long max_doubles) {
     p.span = p.b / g;
     p.le = p.a + 2 * p.b + p.span + 64;
     p.doubles = kChainHeader + 7 * n + long(g) * p.le * p.a;
-    if (p.doubles <= std::min(max_doubles, kChainMaxDoubles)) {
+    if (p.doubles <= std::min(max_doubles, kSorMaxDoubles)) {
       p.G = g;
       p.ok = true;
       break;
@@ -120,9 +123,16 @@ inline bool UseChain(const SorPlan& one, const SorPlan& many) {
   return many.ok && (!one.ok || many.G * many.Q > one.Q);
 }
 
-inline long SorWorkspaceDoubles(int nx, int ny) {
-  const SorPlan p = PlanSor(nx, ny, 1 << 30, 1L << 60), c = PlanChain(nx, ny, 1 << 30, 1L << 60);
-  return std::max(p.ok ? p.doubles : 0, c.ok ? c.doubles : 0);
+// The workspace of a solve of at most limit + 1 sweeps.
+inline long SorWorkspaceDoubles(int nx, int ny, int limit) {
+  auto ring = [&](long cap) {
+    SorPlan p = PlanSor(nx, ny, limit, cap);
+    return p.ok ? p : PlanSor(nx, ny, std::min(limit, 0), 1L << 60);
+  };
+  const SorPlan p = ring(kSorMaxDoubles), c = PlanChain(nx, ny, limit, kSorMaxDoubles);
+  if (!UseChain(p, c)) return p.ok ? p.doubles : 0;
+  const SorPlan retry = ring(std::max(c.doubles, kRetryMaxDoubles));
+  return std::max(c.doubles, retry.ok ? retry.doubles : 0);
 }
 
 }  // namespace hg

@@ -1,7 +1,7 @@
 // sor_plan_driver.cpp -- prints the plans of hydro_amd/csrc/sor_plan.h for grids
 // and iteration limits (built by tests/test_sor_plan.py with g++
 // -fsanitize=undefined): for each "nx ny limit" on the input one line
-//   ok_one Q rounds doubles_one | use_chain Q G span le doubles_many a b end
+//   ok_one Q rounds doubles_one | use_chain Q G span le doubles_many a b end workspace
 #include <cstdio>
 
 #include "../hydro_amd/csrc/sor_plan.h"
@@ -14,9 +14,9 @@ int main() {
     const bool many = hg::UseChain(p, c);
     const int P = 2 * c.Q;
     const long end = many ? hg::ChainDoneStep(limit, P, c.G * P, c.span, c.a, c.b) : 0;
-    std::printf("%d %d %d %ld %d %d %d %d %d %ld %d %d %ld\n", int(p.ok), p.Q, p.rounds,
+    std::printf("%d %d %d %ld %d %d %d %d %d %ld %d %d %ld %ld\n", int(p.ok), p.Q, p.rounds,
                 p.ok ? p.doubles : 0, int(many), c.Q, c.G, c.span, c.le, c.ok ? c.doubles : 0, c.a,
-                c.b, end);
+                c.b, end, hg::SorWorkspaceDoubles(nx, ny, limit));
   }
   return 0;
 }
