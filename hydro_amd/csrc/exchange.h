@@ -106,18 +106,18 @@ __device__ __forceinline__ bool Exchange(double (&v)[NV], double& extra, unsigne
                    unsigned(__double2hiint(v[q])));
         }
       }
-      Word g[2 * NV];
+      Word g[2 * NV] = {};
       for (int n = 0;; ++n) {
+        if (n == spin) {
+          ok = false;
+          break;
+        }
         bool all = true;
 #pragma unroll
         for (int i = 0; i < 2 * NV; ++i) g[i] = TagLoad(mine + i * kWholeMaxWg + min(lane, W - 1));
 #pragma unroll
         for (int i = 0; i < 2 * NV; ++i) all = all && unsigned(g[i] >> 32) == tag;
         if (__all(all)) break;
-        if (n == spin) {
-          ok = false;
-          break;
-        }
       }
 #pragma unroll
       for (int q = 0; q < NV; ++q)

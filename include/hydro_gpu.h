@@ -342,7 +342,7 @@ hg_status hg_time_kernel(hg_ctx* ctx, const char* kernel, int32_t reps, double* 
  * of them off the GPU, a wait ends after a bounded number of polls, the solve is
  * run again by kernels that do not wait, with the same result, and the next
  * ones do not try for a while.  hg_set_wait_polls sets the bound (negative: the
- * default, 0.1 s and more; 0: give up at the first poll that would wait) and
+ * default, 0.1 s and more; 0: give up without a poll) and
  * lets solves try again; hg_wait_give_ups counts the solves that gave up. */
 hg_status hg_set_wait_polls(hg_ctx* ctx, int32_t polls);
 int64_t hg_wait_give_ups(const hg_ctx* ctx);

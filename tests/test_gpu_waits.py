@@ -1,6 +1,5 @@
 """Solves whose workgroups wait for each other inside one launch, made to give up
-from the host: with a bound of 0 polls every wait that is not met at once ends the
-kernel, and the solve is run again by kernels that do not wait.  The result is
+from the host: with a bound of 0 polls the first wait ends the kernel, and the solve is run again by kernels that do not wait.  The result is
 that of those kernels bit for bit, from the start values the solve had (a warm
 start among them), the next solves do not try, and with the default bound the
 object goes back to one launch, on words that hold what the failed solve left."""
