@@ -171,6 +171,16 @@ __device__ __forceinline__ double LaneOf(double v, int lane) {
   return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
                           __builtin_amdgcn_readlane(__double2loint(v), lane));
 }
+// The value of the lane before (SHR) or after, `edge` in the first / last lane.
+template <bool SHR>
+__device__ __forceinline__ double LaneNext(double v, double edge) {
+  constexpr int kCtrl = SHR ? 0x138 : 0x130;  // wave_shr:1, wave_shl:1
+  return __hiloint2double(
+      __builtin_amdgcn_update_dpp(__double2hiint(edge), __double2hiint(v), kCtrl, 0xf, 0xf, false),
+      __builtin_amdgcn_update_dpp(__double2loint(edge), __double2loint(v), kCtrl, 0xf, 0xf,
+                                  false));
+}
+
 // Sum over a wave whose lanes are all active, the same in every lane.
 template <class M>
 __device__ __forceinline__ M WaveTotal(M v) {

@@ -247,16 +247,6 @@ KLuUnpack(int nx, int ny, int tr, const double* __restrict__ v, double* __restri
   }
 }
 
-// The value of the lane before (SHR) or after, `edge` in the first / last lane.
-template <bool SHR>
-__device__ __forceinline__ double LaneNext(double v, double edge) {
-  constexpr int kCtrl = SHR ? 0x138 : 0x130;  // wave_shr:1, wave_shl:1
-  return __hiloint2double(
-      __builtin_amdgcn_update_dpp(__double2hiint(edge), __double2hiint(v), kCtrl, 0xf, 0xf, false),
-      __builtin_amdgcn_update_dpp(__double2loint(edge), __double2loint(v), kCtrl, 0xf, 0xf,
-                                  false));
-}
-
 template <int NR, bool TR, int MAXT>
 __global__ void __launch_bounds__(MAXT)
 KLuSkew(int a, int b, const double2* __restrict__ sw, const double2* __restrict__ en,

@@ -40,6 +40,7 @@
 // workgroup 15.3) against 177 us; 333x217 13 (43) against 534 us.
 // For one workgroup 1024 threads beat 512 and 256 (256x128: 15.3, 19.7, 30.9
 // us); for each of several 512 (256x128: 3.7; 1024: 7.2, 256: 4.8 us).
+#include "device_common.h"
 #include "kernels.h"
 #include "sor_plan.h"
 
@@ -49,7 +50,7 @@ namespace {
 
 // Barrier between steps.  It orders the LDS exchange and leaves the loads in
 // flight; of the global stores it waits for those of two steps before and
-// earlier (a step issues at most 3 + 2 loads and 2 stores per wave, vector
+// earlier (a step issues at least 3 loads and 2 stores per wave, vector
 // memory operations complete in order on vmcnt, and at most 10 may be
 // outstanding here), which the first stage reads four steps after they were
 // issued at the earliest.  The workgroup's waves share one L1.
@@ -78,10 +79,11 @@ struct SorRow {
 // Rows into the skewed order, zero where the neighbour is outside the grid.
 __global__ void __launch_bounds__(256)
 KSorPack(int nx, int ny, Rows r, const double* __restrict__ k, int tr, double2* __restrict__ oc,
-         double2* __restrict__ xn, double2* __restrict__ ck, double* head) {
-  if (blockIdx.x == 0 && head) {  // no sweep has ended, no steps done
+         double2* __restrict__ xn, double2* __restrict__ ck, double* __restrict__ xf,
+         double* head, int head_doubles) {
+  if (blockIdx.x == 0) {  // no sweep has ended, no steps done
     int* const h = reinterpret_cast<int*>(head);
-    for (int z = threadIdx.x; z < 2 * kChainRec; z += 256) h[z] = z == 0 ? kNever : 0;
+    for (int z = threadIdx.x; z < 2 * head_doubles; z += 256) h[z] = z == 0 ? kNever : 0;
   }
   const int a = tr ? ny : nx, b = tr ? nx : ny;
   const int d = blockIdx.x * 256 + threadIdx.x;  // skewed index, so that stores coalesce
@@ -98,26 +100,156 @@ KSorPack(int nx, int ny, Rows r, const double* __restrict__ k, int tr, double2* 
   // -0 where the reference's, which starts at +0, is +0; k + sum is then the
   // same)
   ck[d] = double2{r.c[c], k[c] + 0.};
+  xf[d] = 0.;
 }
 
 __global__ void __launch_bounds__(256)
 KSorUnpack(int nx, int ny, int tr, const double* __restrict__ ring,
-           const double* __restrict__ head, double* __restrict__ x) {
+           const double* __restrict__ head, double* __restrict__ x) {  // head[1]: the ring slot
   const int c = blockIdx.x * 256 + threadIdx.x;
   if (c >= nx * ny) return;
   const int a = tr ? ny : nx, b = tr ? nx : ny;
   const int i = c % nx, j = c / nx;
   const int t = tr ? j : i, m = tr ? i : j;
   const int row = t + m >= b ? t + m - b : t + m;
-  const long slot = head ? reinterpret_cast<const long long*>(head)[0] : 0;
+  const long slot = reinterpret_cast<const long long*>(head)[1];
   x[c] = ring[slot * nx * ny + long(row) * a + t];
+}
+
+__device__ __forceinline__ double AgentLoad(const double* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ int AgentLoad(const int* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+template <bool TR>
+__device__ __forceinline__ double SorCell(const SorRow& r, double own, double cross, double xold,
+                                          double nold, double old, double omega, double& dmax) {
+  const double po = r.oc.x * own, pc = r.oc.y * cross;  // new: south and west
+  const double px = r.xn.x * xold, pn = r.xn.y * nold;  // old: east and north
+  double sum = po + pc;
+  sum += TR ? pn : px;  // east
+  sum += TR ? px : pn;  // north
+  const double value = -(r.ck.y + sum) / r.ck.x;
+  const double corr = value - old;
+  dmax = fmax(dmax, fabs(corr));
+  return old + corr * omega;
+}
+
+// ---- the first sweeps, one after another --------------------------------------
+// A pipeline takes longer over its first sweep than a workgroup with nothing else
+// to do, and a solve often ends there (a start that is nearly the solution).  So
+// one more workgroup of the same launch runs the first kFirstSweeps sweeps one
+// after another in xf; if the stop rule is met within them it ends the solve:
+// info, the result's slot, `word` lowered to kEndedFirst.  The pipeline leaves
+// when it sees that.  Where both end the solve they do at the same sweep, with
+// the same values.
+//
+// Device time in us of a solve that ends in its first and second sweep (launches
+// and the read back of info, about 40, in all of them): a sweep at a time in place,
+// the pipeline alone, with this: 16x16 46, 60 | 56, 57 | 51, 58; 64x64 102, 135 |
+// 162, 165 | 74, 96; 128x128 249, 338 | 411, 418 | 103, 160; 512x512 3490, 5690 |
+// 1776, 1808 | 478, 890.  A third sweep would end after the pipeline could (512x512:
+// two take 840 us, the pipeline's first decision 900) and gain little elsewhere.
+//
+// Thread t takes line t, one row per step.  The value before it on its line stays
+// in a register, that of line t - 1 comes by a lane shift, between waves through
+// LDS: wave w is w groups of kG steps behind the first, one barrier per group.
+// All operands are loaded kG steps ahead; an old value is loaded before the step
+// that writes its cell, by the same wave or by one a group behind.
+template <bool TR, int kG>
+__device__ __forceinline__ void FirstSweeps(int a, int b, const double2* __restrict__ oc,
+                                            const double2* __restrict__ xn,
+                                            const double2* __restrict__ ck, double* xf, double tol,
+                                            int limit, double omega, long long slot, int* word,
+                                            double* head, unsigned long long* __restrict__ info) {
+  constexpr int kRing = 16;
+  __shared__ double edge[kSorThreads / 64][kRing];  // values of a wave's last lane, by step
+  __shared__ double red[kSorThreads / 64];
+  const int t = threadIdx.x, nw = (a + 63) >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  if (wave >= nw) return;
+  const unsigned tc = unsigned(min(t, a - 1)), tx = t < a - 1 ? tc + 1 : tc;
+  const int ng = (a + b - 2 + kG) / kG;  // groups of the a + b - 1 steps
+  for (int s = 0;; ++s) {
+    struct Step {
+      SorRow r;
+      double next, cross;  // old values: the next cell of the line, the line after's
+    } o[kG];
+    int lrow = 0, srow = 0;  // rows of the next load and of the next store
+    auto Load = [&](Step& q) {
+      const int nrow = lrow + 1 == b ? 0 : lrow + 1;
+      const size_t d = size_t(unsigned(lrow)) * unsigned(a);
+      const size_t e = size_t(unsigned(nrow)) * unsigned(a);
+      q.r.oc = (oc + d)[tc];
+      q.r.xn = (xn + d)[tc];
+      q.r.ck = (ck + d)[tc];
+      q.next = (xf + e)[tc];
+      q.cross = (xf + e)[tx];
+      lrow = nrow;
+    };
+    double val = 0., old = xf[tc], dmax = 0., out[kG], e[kG];
+#pragma unroll
+    for (int i = 0; i < kG; ++i) Load(o[i]);
+    for (int k = 0; k < wave; ++k) ChainBarrier();
+    for (int g = 0; g < ng; ++g) {
+#pragma unroll
+      for (int i = 0; i < kG; ++i)
+        e[i] = wave == 0 ? 0. : edge[wave - 1][(g * kG + i - 1) & (kRing - 1)];
+#pragma unroll
+      for (int i = 0; i < kG; ++i) {
+        const int m = g * kG + i - t;
+        const Step& q = o[i];
+        const double cross = LaneNext<true>(val, e[i]);
+        double d = 0.;
+        val = SorCell<TR>(q.r, m == 0 ? 0. : val, cross, t < a - 1 ? q.cross : 0.,
+                          m < b - 1 ? q.next : 0., old, omega, d);
+        if (m >= 0 && m < b && t < a) {
+          (xf + size_t(unsigned(srow)) * unsigned(a))[tc] = val;
+          dmax = fmax(dmax, d);
+        }
+        old = q.next;
+        out[i] = val;
+        srow = srow + 1 == b ? 0 : srow + 1;
+        __builtin_amdgcn_sched_barrier(0);
+        Load(o[i]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (nw > 1) {
+        if ((t & 63) == 63)
+#pragma unroll
+          for (int i = 0; i < kG; ++i) edge[wave][(g * kG + i) & (kRing - 1)] = out[i];
+        ChainBarrier();
+      }
+    }
+    for (int k = wave + 1; k < nw; ++k) ChainBarrier();
+    const double md = LaneOf(DppMax<6>(dmax), 63);
+    if ((t & 63) == 0) red[wave] = md;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the next sweep reads this one's values
+    __syncthreads();
+    double diff = red[0];
+    for (int w = 1; w < nw; ++w) diff = fmax(diff, red[w]);
+    const bool met = !(diff > tol);
+    if (met || s == limit) {
+      if (t == 0) {
+        info[0] = (unsigned long long)(met ? s : s + 1);
+        info[1] = (unsigned long long)__double_as_longlong(diff);
+        reinterpret_cast<long long*>(head)[1] = slot;
+        __hip_atomic_fetch_min(word, kEndedFirst, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      return;
+    }
+    if (s + 1 == kFirstSweeps) return;
+  }
 }
 
 template <bool TR>
 __global__ void __launch_bounds__(kSorThreads)
 KSorPipe(int a, int b, int Q, int rounds, const double2* __restrict__ oc,
-         const double2* __restrict__ xn, const double2* __restrict__ ck, double* ring, double tol,
-         int limit, double omega, double* head, unsigned long long* __restrict__ info) {
+         const double2* __restrict__ xn, const double2* __restrict__ ck, double* ring, double* xf,
+         double tol, int limit, double omega, double* head,
+         unsigned long long* __restrict__ info) {
   // [2 step parities][Q][a + 2] values (first, second stage) with a zero
   // pad either side, then the sweeps' maxima
   extern __shared__ double2 lds2[];
@@ -126,6 +258,11 @@ KSorPipe(int a, int b, int Q, int rounds, const double2* __restrict__ oc,
   double2* const val = lds2;
   unsigned long long* const sd = reinterpret_cast<unsigned long long*>(lds2 + 2 * Q * W);
   const int P = 2 * Q, R = rounds * P;
+  int* const word = reinterpret_cast<int*>(head);  // kNever until FirstSweeps ends the solve
+  if (blockIdx.x == 1) {
+    FirstSweeps<TR, 4>(a, b, oc, xn, ck, xf, tol, limit, omega, R, word, head, info);
+    return;
+  }
   const int tid = threadIdx.x;
   for (int z = tid; z < 2 * Q * W; z += blockDim.x) val[z] = double2{0., 0.};
   for (int z = tid; z < R; z += blockDim.x) sd[z] = 0ull;
@@ -193,7 +330,7 @@ KSorPipe(int a, int b, int Q, int rounds, const double2* __restrict__ oc,
   LoadPrev(g[0], m, slot, RowOn(off));
   double2* const mine = val + q * W + t;
   double ownA = 0., ownB = 0., oldA = 0., h1 = 0., h2 = 0., dA = 0., dB = 0.;
-  int group = 0;
+  int group = 0, ended = kNever;
   // sweep s (in ring slot `idx`) has just finished: the stop rule,
   // do { sweep } while (diff > tol && iter++ < limit), sweeps in order
   auto Decide = [&](int s, int idx) {
@@ -205,23 +342,15 @@ KSorPipe(int a, int b, int Q, int rounds, const double2* __restrict__ oc,
     if (met || !(s < limit)) {
       info[0] = (unsigned long long)(met ? s : s + 1);
       info[1] = bits;
-      reinterpret_cast<long long*>(head)[0] = idx;
+      reinterpret_cast<long long*>(head)[1] = idx;
       flag = group + 1;
     }
   };
-  auto Cell = [&](const SorRow& r, double own, double cross, double xold, double nold, double old,
-                  double& dmax) {
-    const double po = r.oc.x * own, pc = r.oc.y * cross;  // new: south and west
-    const double px = r.xn.x * xold, pn = r.xn.y * nold;  // old: east and north
-    double sum = po + pc;
-    sum += TR ? pn : px;  // east
-    sum += TR ? px : pn;  // north
-    const double value = -(r.ck.y + sum) / r.ck.x;
-    const double corr = value - old;
-    dmax = fmax(dmax, fabs(corr));
-    return old + corr * omega;
-  };
   for (;; ++group) {
+    if (tid == 0) {  // (as the group before found it: no wait)
+      if (ended != kNever && !flag) flag = group + 1;
+      ended = AgentLoad(word);
+    }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       // the loads of step T + 1, then step T
@@ -258,9 +387,10 @@ KSorPipe(int a, int b, int Q, int rounds, const double2* __restrict__ oc,
           const int st = 2 * q + (m >> 1);
           Decide(st + P * (rd - 1), st + P * (rm == 0 ? rounds - 1 : rm - 1));
         }
-        const double xA = Cell(ca, m != 0 ? ownA : 0., west.x, crossA, m1 != 0 ? nextA : 0., oldA,
-                               dA);
-        const double xB = Cell(cb, m != 2 ? ownB : 0., west.y, eastA, m != 1 ? h1 : 0., h2, dB);
+        const double xA = SorCell<TR>(ca, m != 0 ? ownA : 0., west.x, crossA, m1 != 0 ? nextA : 0.,
+                                      oldA, omega, dA);
+        const double xB = SorCell<TR>(cb, m != 2 ? ownB : 0., west.y, eastA, m != 1 ? h1 : 0., h2,
+                                      omega, dB);
         mine[(i & 1) * Q * W + 1] = double2{xA, xB};
         const unsigned pos = slot + off;
         *reinterpret_cast<double*>(reinterpret_cast<char*>(ring) + pos) = xA;
@@ -325,18 +455,11 @@ KSorPipe(int a, int b, int Q, int rounds, const double2* __restrict__ oc,
 // found by a second launch (tail) of one workgroup, which repeats the sweeps
 // from the last logged one before the stop to the stop -- unless the solve
 // ran to its last sweep, which is written as it is computed.
-__device__ __forceinline__ double AgentLoad(const double* p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ int AgentLoad(const int* p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
 template <bool TR, int MAXT>
 __global__ void __launch_bounds__(MAXT)
 KSorChain(SorChain ch, const double2* __restrict__ oc, const double2* __restrict__ xn,
-          const double2* __restrict__ ck, double* head, double* logs, double* out, double tol,
-          double omega, unsigned long long* __restrict__ info) {
+          const double2* __restrict__ ck, double* head, double* logs, double* out, double* xf,
+          double tol, double omega, unsigned long long* __restrict__ info) {
   extern __shared__ double2 lds2[];  // as KSorPipe's; maxima [stage][4 rounds]
   __shared__ int lstop;
   int* const stop = reinterpret_cast<int*>(head);
@@ -345,6 +468,10 @@ KSorChain(SorChain ch, const double2* __restrict__ oc, const double2* __restrict
   const int a = ch.a, b = ch.b, Q = ch.Q, P = 2 * Q, W = a + 2, le = ch.le, span = ch.span;
   const long log_n = long(le) * a;
   int G = ch.G, wg = blockIdx.x, limit = ch.limit;
+  if (wg == G) {
+    FirstSweeps<TR, MAXT <= 512 ? 4 : 3>(a, b, oc, xn, ck, xf, tol, limit, omega, 1, stop, head, info);
+    return;
+  }
   // where the first stage's input comes from: the log of workgroup `src`, the
   // values for this workgroup's step T in row T + shift; the zero start where
   // T - t < from
@@ -353,6 +480,7 @@ KSorChain(SorChain ch, const double2* __restrict__ oc, const double2* __restrict
   int from = wg == 0 ? b : -1;
   if (ch.tail) {
     const int s = *stop;
+    if (s == kEndedFirst) return;
     // gave up, or ran out of step numbers before every sweep up to s was decided
     // (kNever, the last number of 32 bits, is past them too: G P < b)
     if (s < 0 || ChainDoneStep(s, P, G * P, span, a, b) + 4 > kChainMaxStep) {
@@ -449,13 +577,13 @@ KSorChain(SorChain ch, const double2* __restrict__ oc, const double2* __restrict
     if (!wait) return true;
     seen = max(seen, ahead);
     for (int k = 0; seen < need; ++k) {
-      seen = AgentLoad(progress + 16 * src);
-      if (seen >= need) break;
-      if (AgentLoad(stop) != kNever) return true;
       if (k == ch.spin) {
         __hip_atomic_fetch_min(stop, -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         return false;
       }
+      seen = AgentLoad(progress + 16 * src);
+      if (seen >= need) break;
+      if (AgentLoad(stop) != kNever) return true;
     }
     return true;
   };
@@ -474,18 +602,6 @@ KSorChain(SorChain ch, const double2* __restrict__ oc, const double2* __restrict
     }
   }
   double2* const mine = val + q * W + t;
-  auto Cell = [&](const SorRow& r, double own, double cross, double xold, double nold, double old,
-                  double& dmax) {
-    const double po = r.oc.x * own, pc = r.oc.y * cross;
-    const double px = r.xn.x * xold, pn = r.xn.y * nold;
-    double sum = po + pc;
-    sum += TR ? pn : px;
-    sum += TR ? px : pn;
-    const double value = -(r.ck.y + sum) / r.ck.x;
-    const double corr = value - old;
-    dmax = fmax(dmax, fabs(corr));
-    return old + corr * omega;
-  };
   auto Decide = [&](int stage, int r) {
     const int slot = 4 * stage + (r & 3), s = wg * P + stage + ptot * r;
     const unsigned long long bits = sd[slot];
@@ -537,8 +653,10 @@ KSorChain(SorChain ch, const double2* __restrict__ oc, const double2* __restrict
         const bool m0 = tm == ez, mend = tm1 == ez;
         const int tb1 = tm >= 1 ? tm - 1 : tm - 1 + b, tb2 = tm >= 2 ? tm - 2 : tm - 2 + b;
         const bool mb1 = tb1 == ez, mb2 = tb2 == ez;
-        const double xA = Cell(ca, m0 ? 0. : ownA, west.x, crossA, mend ? 0. : nextA, oldA, dA);
-        const double xB = Cell(cb, mb2 ? 0. : ownB, west.y, eastA, mb1 ? 0. : h1, h2, dB);
+        const double xA = SorCell<TR>(ca, m0 ? 0. : ownA, west.x, crossA, mend ? 0. : nextA, oldA,
+                                      omega, dA);
+        const double xB = SorCell<TR>(cb, mb2 ? 0. : ownB, west.y, eastA, mb1 ? 0. : h1, h2, omega,
+                                      dB);
         mine[(i & 1) * Q * W + 1] = double2{xA, xB};
         if (last && wait) {  // (the tail reads the logs)
           int r = lrow + i;
@@ -625,35 +743,38 @@ bool LaunchSor(hipStream_t st, int nx, int ny, Rows a, const double* k, double* 
   double2 *xn = oc + n, *ck = xn + n;
   double* ring = reinterpret_cast<double*>(ck + n);
   const unsigned grid = unsigned((n + 255) / 256);
-  KSorPack<<<grid, 256, 0, st>>>(nx, ny, a, k, tr, oc, xn, ck, many ? ws : nullptr);
+  // the first sweeps' values: behind the ring, or the chain's result
+  double* const xf = ring + (many ? 1 : 2 * p.Q * p.rounds) * n;
+  KSorPack<<<grid, 256, 0, st>>>(nx, ny, a, k, tr, oc, xn, ck, xf, ws,
+                                 many ? kChainRec : kSorHeader);
   if (many) {
     SorChain ch{c.a, c.b, (c.a + 63) / 64 * 64, c.Q, c.G, c.span, c.le, limit, 0,
                 polls < 0 ? kSpin : polls};
     const int threads = c.Q * ch.ap;
     const size_t lds = size_t(2) * c.Q * (c.a + 2) * sizeof(double2) + size_t(8) * c.Q * 8;
-    double *out = ring, *logs = out + n;
+    double *out = ring, *logs = xf + n;
     for (int tail = 0; tail < 2; ++tail) {
       ch.tail = tail;
-      const unsigned g = tail ? 1u : unsigned(c.G);
+      const unsigned g = tail ? 1u : unsigned(c.G) + 1u;
       auto launch = [&](auto kernel) {
-        kernel<<<g, threads, lds, st>>>(ch, oc, xn, ck, ws, logs, out, tol, omega, info);
+        kernel<<<g, threads, lds, st>>>(ch, oc, xn, ck, ws, logs, out, xf, tol, omega, info);
       };
       if (threads > 512)
         launch(tr ? KSorChain<true, 1024> : KSorChain<false, 1024>);
       else
         launch(tr ? KSorChain<true, 512> : KSorChain<false, 512>);
     }
-    KSorUnpack<<<grid, 256, 0, st>>>(nx, ny, tr, out, nullptr, x);
+    KSorUnpack<<<grid, 256, 0, st>>>(nx, ny, tr, out, ws, x);
     return true;
   }
   const int threads = (p.Q * p.a + 63) / 64 * 64;
   const size_t lds = size_t(2) * p.Q * (p.a + 2) * sizeof(double2) +
                      size_t(p.rounds) * 2 * p.Q * 8 + 16;
   if (p.tr)
-    KSorPipe<true><<<1, threads, lds, st>>>(p.a, p.b, p.Q, p.rounds, oc, xn, ck, ring, tol, limit,
-                                            omega, ws, info);
+    KSorPipe<true><<<2, threads, lds, st>>>(p.a, p.b, p.Q, p.rounds, oc, xn, ck, ring, xf, tol,
+                                            limit, omega, ws, info);
   else
-    KSorPipe<false><<<1, threads, lds, st>>>(p.a, p.b, p.Q, p.rounds, oc, xn, ck, ring, tol,
+    KSorPipe<false><<<2, threads, lds, st>>>(p.a, p.b, p.Q, p.rounds, oc, xn, ck, ring, xf, tol,
                                              limit, omega, ws, info);
   KSorUnpack<<<grid, 256, 0, st>>>(nx, ny, tr, ring, ws, x);
   return false;

@@ -14,7 +14,9 @@ namespace hg {
 
 constexpr int kSorThreads = 1024;
 constexpr int kSorMaxQ = 32;
-constexpr int kSorHeader = 32;  // doubles before the arrays: [0] the result's ring slot
+constexpr int kSorHeader = 32;  // doubles before the arrays: [0] kNever, [1] the result's slot
+constexpr int kFirstSweeps = 2;  // of FirstSweeps
+constexpr int kEndedFirst = -2;
 
 // (several workgroups, below)
 constexpr int kLag = 20;
@@ -27,7 +29,8 @@ constexpr int kSorMaxG = 64, kSorMaxStages = 1024;
 // chain that gave up would use.
 constexpr long kSorMaxDoubles = 1L << 26, kRetryMaxDoubles = 1L << 22;
 // Workspace header, in doubles: the smallest sweep that ended the solve
-// (int `stop`), then a 64-byte line of progress per workgroup, then the max
+// (int `stop`; -1: gave up, kEndedFirst), the result's slot (0 the chain's, 1 the
+// first sweeps'), then a 64-byte line of progress per workgroup, then the max
 // |corr| of the sweep each stage last found to end it.
 constexpr int kChainProgress = 8, kChainRec = kChainProgress + 8 * kSorMaxG;
 constexpr int kChainHeader = kChainRec + kSorMaxStages;
@@ -62,7 +65,7 @@ inline SorPlan PlanSor(int nx, int ny, int limit, long max_doubles) {
   int q = std::min(std::min(kSorThreads / std::max(p.a, 1), (p.b - 4) / 4), kSorMaxQ);
   q = std::min(q, limit / 2 + 1);  // sweeps 0 .. limit
   for (; q >= 1; --q) {
-    p.doubles = kSorHeader + (6 + 2L * q * p.rounds) * n;
+    p.doubles = kSorHeader + (7 + 2L * q * p.rounds) * n;
     // (32-bit byte offsets in the kernel)
     if (p.doubles <= max_doubles && p.doubles < (1L << 29)) {
       p.Q = q;
@@ -92,7 +95,7 @@ inline SorPlan PlanChain(int nx, int ny, int limit, long max_doubles) {
   for (; g >= 2; --g) {
     p.span = p.b / g;
     p.le = p.a + 2 * p.b + p.span + 64;
-    p.doubles = kChainHeader + 7 * n + long(g) * p.le * p.a;
+    p.doubles = kChainHeader + 8 * n + long(g) * p.le * p.a;
     if (p.doubles <= std::min(max_doubles, kSorMaxDoubles)) {
       p.G = g;
       p.ok = true;
@@ -119,8 +122,13 @@ constexpr int kChainMaxStep = 1 << 30;
 // 333x217 at 100 43.5 | 13.2 us (8 | 52); with fewer stages they lose: 32x128
 // 3.7 | 4.2 us (64 | 48), 16x256 4.0 | 5.2 us (128 | 112), as the lines are
 // padded to waves.
+// Nor on lines of under 16 cells, of which one workgroup holds 64 sweeps: solves
+// of few sweeps, which take a chain twice as long (it repeats them), then lose
+// against a sweep at a time.  3x700 at 9 | 101 sweeps 468 | 800 us by one, 1353 |
+// 1257 by several, 9x1030 721 | 1419 and 1442 | 1359, 16x600 430 | 830 and 875 |
+// 833; a sweep at a time 9x1030 takes 4 sweeps in 1230 us, 16x600 in 1050.
 inline bool UseChain(const SorPlan& one, const SorPlan& many) {
-  return many.ok && (!one.ok || many.G * many.Q > one.Q);
+  return many.ok && (!one.ok || (many.G * many.Q > one.Q && many.a >= 16));
 }
 
 // The workspace of a solve of at most limit + 1 sweeps.

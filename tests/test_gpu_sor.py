@@ -57,3 +57,40 @@ def test_sor_without_a_limit(gpu, nx, ny, limit):
                                     **args)
     assert 2 < so.iterations < 1000 and st.iterations == so.iterations
     assert np.array_equal(x, xo)
+
+
+# stops within and just past the sweeps that one workgroup runs ahead of the
+# pipeline: one and several waves, part of a wave, lines much longer than wide
+@pytest.mark.parametrize("nx,ny", [(1, 8), (8, 8), (9, 8), (31, 33), (64, 64), (65, 64), (40, 333),
+                                   (9, 1030), (128, 128), (217, 333), (513, 600), (1024, 12)])
+@pytest.mark.parametrize("sweep", [0, 1, 2, 3, 4])
+def test_sor_stops_in_its_first_sweeps(gpu, nx, ny, sweep):
+    print(f"case: SOR {nx}x{ny} stops in sweep {sweep}", flush=True)
+    r = rows(nx, ny, nx)
+    sid = capi.SOLVERS["gauss_seidel"]
+    args = dict(omega=1.2)
+    tol = pyoracle.stencil_solve(nx, ny, *r, sid, tol=0.0, max_iters=sweep, **args)[1].final_diff
+    x, st = stencil_solve(nx, ny, *r, sid, tol=tol, max_iters=1000, **args)
+    xo, so = pyoracle.stencil_solve(nx, ny, *r, sid, tol=tol, max_iters=1000, **args)
+    assert st.iterations == so.iterations <= sweep and st.final_diff == so.final_diff
+    assert np.array_equal(x, xo)
+
+
+# values that are not finite spread as in the serial sweeps, and constants of -0
+# (the signs of zeros included); stops at once, after two and after nine sweeps
+@pytest.mark.parametrize("nx,ny", [(9, 8), (64, 65), (217, 333), (3, 7)])
+@pytest.mark.parametrize("value", [np.nan, np.inf, -0.0])
+@pytest.mark.parametrize("limit", [0, 1, 8])
+def test_sor_special_values(gpu, nx, ny, value, limit):
+    print(f"case: SOR {nx}x{ny} {value} limit {limit}", flush=True)
+    s, w, c, e, n, k = rows(nx, ny, 11)
+    if value == 0:
+        k = np.full(nx * ny, value)
+    else:
+        k[nx * ny // 2] = value
+    args = dict(tol=0.0, max_iters=limit, omega=1.3)
+    x, st = stencil_solve(nx, ny, s, w, c, e, n, k, "gauss_seidel", **args)
+    xo, so = pyoracle.stencil_solve(nx, ny, s, w, c, e, n, k, capi.SOLVERS["gauss_seidel"], **args)
+    assert st.iterations == so.iterations
+    assert np.array_equal(x, xo, equal_nan=True)
+    assert np.array_equal(np.signbit(x[~np.isnan(x)]), np.signbit(xo[~np.isnan(xo)]))

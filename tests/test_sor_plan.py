@@ -52,21 +52,21 @@ def test_last_step_of_any_limit(plan):
         # kernel can reach (2^30) with what it adds to one
         assert p["g"] * p["span"] <= p["b"] and ptot < p["b"]
         assert 2**30 + 2 * (p["le"] + p["b"] + p["span"] * p["g"]) < 2**31
-    assert chains > 40
+    assert chains > 30
 
 
 def test_workspace_is_bounded(plan):
-    """512 MB, or two sweeps' ring where that is more (10 or 12 doubles per cell);
+    """512 MB, or two sweeps' ring where that is more (11 or 13 doubles per cell);
     a solve of few sweeps asks for less; a chain's holds a ring for the retry."""
     grids = GRIDS + [(64, 65536), (32, 120000), (512, 1024), (1024, 20000), (2, 4000000)]
     cases = [(nx, ny, lim) for nx, ny in grids for lim in (-3, 0, 5, 1000, 2**31 - 1)]
     for (nx, ny, lim), p in zip(cases, plan(cases)):
         n = nx * ny
-        ring = 32 + (6 + 2 * p["rounds"]) * n
+        ring = 32 + (7 + 2 * p["rounds"]) * n
         assert p["workspace"] <= max(2**26, ring), (nx, ny, lim)
         if min(nx, ny) <= 1024 and lim >= 0 and ring < 2**29:
             assert p["workspace"] >= ring
         if lim == 0:
             assert p["workspace"] <= ring
         if lim == 5:  # three pairs of sweeps
-            assert p["workspace"] <= 32 + (6 + 6 * p["rounds"]) * n
+            assert p["workspace"] <= 32 + (7 + 6 * p["rounds"]) * n
