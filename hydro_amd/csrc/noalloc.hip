@@ -9,9 +9,11 @@
 // lives in one file-scope device array, `scratch`, of kScratchBytes.  Each
 // GPU holds its own copy of that array until the process ends; its address
 // on the current device is looked up once per device with
-// hipGetSymbolAddress and kept.  Calls on one device share the array, so
-// calls that overlap on one device race; every array that must start at
-// zero is cleared by a fill kernel at the start of each call.
+// hipGetSymbolAddress and kept.  Calls on one device share the array: a call
+// holds the device's lock until its kernels are done, so calls of several
+// threads run one after another, except lu, which does without the array
+// while another call has it.  Every array that must start at zero is cleared
+// by a fill kernel at the start of each call.
 
 #include <cstdio>
 #include <cstring>
@@ -34,6 +36,7 @@ __device__ __align__(256) unsigned char scratch[kScratchBytes];
 void* g_scratch_ptr[kMaxDevices] = {};
 std::once_flag g_scratch_once[kMaxDevices];
 hipError_t g_scratch_err[kMaxDevices] = {};
+std::mutex g_scratch_lock[kMaxDevices];
 
 hg_status Fail(hg_status rc, const std::string& msg) {
   hg::SetThreadError("hg_stencil_solve_noalloc: " + msg);
@@ -107,6 +110,12 @@ hg_status hg_stencil_solve_noalloc(int32_t nx, int32_t ny, const double* s, cons
   double* a2 = reinterpret_cast<double*>(base + off_arr + 2 * arr);
   double* a3 = reinterpret_cast<double*>(base + off_arr + 3 * arr);
 
+  std::unique_lock<std::mutex> lock(g_scratch_lock[dev], std::defer_lock);
+  if (solver == HG_SOLVER_LU)
+    (void)lock.try_lock();
+  else
+    lock.lock();
+
   hipStream_t st = static_cast<hipStream_t>(stream);
   // the last-error record may hold an earlier call's error on this thread:
   // clear it, so the check after the launches sees only this call's
@@ -118,7 +127,8 @@ hg_status hg_stencil_solve_noalloc(int32_t nx, int32_t ny, const double* s, cons
   switch (solver) {
     case HG_SOLVER_LU:
       hg::LaunchLuWavefront(st, nx, ny, rows, k, nullptr, x, nullptr, nullptr, nullptr, nullptr,
-                            nullptr, a0, long((kScratchBytes - off_arr) / 8));
+                            nullptr, a0,
+                            lock.owns_lock() ? long((kScratchBytes - off_arr) / 8) : 0);
       break;
     case HG_SOLVER_LU_RB:
       // one right-hand side: the second lane solves it again into a3; the

@@ -32,8 +32,9 @@ extern "C" {
  * and nx <= 4096, else HG_ERR_BAD_ARG (hg_last_error(NULL) says why).
  * stream: the hipStream_t to run on (NULL: the null stream); the call waits
  * for it before it returns.  Every call on one GPU shares that GPU's scratch
- * array and leaves the last call's contents there: calls that overlap on one
- * GPU race.  stats: iterations, final_diff and converged as in
+ * array and leaves the last call's contents there: calls of several threads of
+ * a process wait for each other (lu runs without the array instead, more
+ * slowly).  stats: iterations, final_diff and converged as in
  * hg_stencil_solve; rel_residual is -1 (not computed) and ms 0. */
 hg_status hg_stencil_solve_noalloc(int32_t nx, int32_t ny, const double* s, const double* w,
                                    const double* c, const double* e, const double* n,

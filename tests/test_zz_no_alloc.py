@@ -115,3 +115,48 @@ def test_noalloc_refuses_sizes_beyond_its_scratch(gpu):
         assert b"scratch" in lib.hg_last_error(None)
     finally:
         hip.free()
+
+
+def test_noalloc_from_several_threads(gpu):
+    """Threads that call at the same time, each on its own stream with its own
+    rows: every result is that of a call alone."""
+    import threading
+    lib = capi.load()
+    fn = _noalloc(lib)
+    hip = _Hip()
+    hip.lib.hipStreamCreate.argtypes = [ctypes.POINTER(ctypes.c_void_p)]
+    hip.lib.hipStreamDestroy.argtypes = [ctypes.c_void_p]
+    jobs = []
+    for q, solver in enumerate(("lu", "lu", "lu_rb", "lu", "gauss_seidel", "jacobi", "lu_relaxed")):
+        nx, ny = 200 - 16 * q, 90 + 10 * q
+        rows = _system(nx, ny, q)
+        sid = capi.SOLVERS[solver]
+        omega = {"jacobi": 0.8, "lu_relaxed": 0.5}.get(solver, 1.5)
+        x_ref, _ = stencil_solve(nx, ny, *rows, sid, tol=1e-3, max_iters=20, omega=omega)
+        stream = ctypes.c_void_p()
+        assert hip.lib.hipStreamCreate(ctypes.byref(stream)) == 0
+        jobs.append((nx, ny, [hip.upload(a) for a in rows], hip.upload(np.zeros(nx * ny)),
+                     capi.HgSolveOpts(solver=sid, tolerance=1e-3, max_iters=20,
+                                      relaxation_factor=omega, precision=0), stream, x_ref))
+    rcs = [[] for _ in jobs]
+
+    def work(q):
+        nx, ny, dev, dx, opts, stream, _ = jobs[q]
+        st = capi.HgSolveStats()
+        for _ in range(40):
+            rcs[q].append(fn(nx, ny, *dev, dx, ctypes.byref(opts), ctypes.byref(st), stream))
+
+    print("case: noalloc, 7 threads x 40 calls", flush=True)
+    try:
+        threads = [threading.Thread(target=work, args=(q,)) for q in range(len(jobs))]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        for q, (nx, ny, _, dx, _, _, x_ref) in enumerate(jobs):
+            assert rcs[q] == [capi.HG_OK] * 40
+            assert np.array_equal(hip.download(dx, nx * ny), x_ref), q
+    finally:
+        for job in jobs:
+            hip.lib.hipStreamDestroy(job[5])
+        hip.free()
