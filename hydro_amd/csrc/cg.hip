@@ -298,8 +298,8 @@ KPcgStart(Walk w, const T* __restrict__ r, const T* __restrict__ dinv, T* __rest
 // It is bound by the two exchanges, each a round trip between XCDs behind two
 // sums over the workgroup, against two launches per iteration of which each
 // begins with a fold over all partials.  Time per iteration, FP64, before and
-// after: 64x64 10.0 and 3.0 us, 128x128 9.9 and 3.4, 255x255 10.2 and 4.6,
-// 255x511 11.5 and 6.0, 512x512 15.2 and 7.4.  z sent with the dots instead of
+// after: 64x64 10.8 and 3.1 us, 128x128 9.9 and 3.4, 255x255 10.2 and 4.6,
+// 255x511 11.7 and 5.7, 512x512 15.2 and 7.3.  z sent with the dots instead of
 // after them saves about 1 us of that, sums by lane shifts instead of shuffles
 // through LDS 1.5 us, 1024 threads instead of 512 0.4 us.
 //

@@ -5,9 +5,9 @@
 // quarter of the CUs, since kernels of four queues may run at once and the waits
 // need a kernel's workgroups to run together; they are bounded (kWholeSpin polls,
 // see wait_guard.h), and a solve that gave up is run again by kernels that do
-// not wait.  16 workgroups
-// or fewer are faster where their threads can hold the grid: 32 cost 1.3 us more
-// per iteration of two exchanges.
+// not wait.  A thread holds one cell while 16 workgroups hold the grid, then two,
+// then four: 32 or 64 workgroups cost more per exchange than fewer cells per thread
+// save, fewer than 16 less (figures at SplitWhole).
 #pragma once
 
 #include <algorithm>

@@ -89,7 +89,7 @@ class MgPrecondT : public Precond {
   int FcgPartials() const override { return lv_.size() > 1 ? fine_.blocks() : 0; }
   // level 1 runs a tiled down-leg (its first kernel takes the stop test)
   bool FusesUpdate() const override {
-    return lv_.size() >= 3 && !(use_coarse_kernel && first_in_kernel_ == 1);
+    return lv_.size() >= 3 && first_in_kernel_ != 1;
   }
   int levels() const { return int(lv_.size()); }
   // Average device time (ms) of one launch of a V-cycle kernel ("KDown<double>",
@@ -98,7 +98,7 @@ class MgPrecondT : public Precond {
   // finest level) and the level buffers.  Throws on an unknown name.
   double TimeKernel(const char* name, int reps, const double* r, hipStream_t st);
   const MgLevelT<M>& level(int l) const { return lv_[l]; }
-  float omega = 0.8f;  // damping of the plain Jacobi sweeps (coarsest-level fallbacks)
+  float omega = 0.8f;  // damping of the plain Jacobi sweeps (a single-level hierarchy)
   // Chebyshev smoothing (pre and post): damping 1/r_k at the roots r_k of
   // the Chebyshev polynomial of the sweep count on an interval [a, 2] of the
   // spectrum of D^-1 A (which is in [0, 2] by Gershgorin), applied in that
@@ -114,14 +114,12 @@ class MgPrecondT : public Precond {
   // flexible CG from 7.35 to about 6.2 iterations per solve to 1e-8, where
   // a third sweep on the finest level too adds nothing more.
   SweepWeights sweeps{{0.532078f, 0.909091f, 3.119374f}};
-  int coarse_sweeps = 40;
   bool bilinear = true;  // prolongation: bilinear (true) or injection
-  // levels of <= 2048 cells down to a coarsest grid of <= 64 cells run in
-  // one workgroup (one launch) instead of one launch per sweep
-  bool use_coarse_kernel = true;
 
  private:
   std::vector<MgLevelT<M>> lv_;
+  // levels of <= 2048 cells down to the coarsest of <= 64 run in one workgroup
+  // (one launch), from this one on
   int first_in_kernel_ = -1;
   TileGrid fine_;  // the finest level's tiles: 64 x kTallY or 64 x kMidY
   bool tall_;

@@ -19,7 +19,6 @@ namespace hg {
 namespace {
 
 constexpr int kTinyMax = 64;          // coarsest grid, solved by one wave
-constexpr int kCoarsestMax = kTinyMax;
 // levels handled by the one-workgroup cycle (4096 and 8192 cells, two or four
 // more launches saved, measured 1 and 2 us per cycle slower at 512 x 512: one
 // CU is then what takes the time)
@@ -547,53 +546,6 @@ KUp(int nx, int ny, TileGrid tg, const M* __restrict__ kx, const M* __restrict__
   }
 }
 
-// Coarsest level: Jacobi sweeps in one workgroup, x and r in LDS.
-template <class M>
-__global__ void __launch_bounds__(kCoarsestMax)
-KCoarsest(int nx, int ny, const M* __restrict__ kx, const M* __restrict__ ky,
-          const M* __restrict__ dinv, const M* __restrict__ r, M omega, int sweeps,
-          M* __restrict__ out, const int* done) {
-  if (Done(done)) return;
-  __shared__ M xs[2][kCoarsestMax];
-  const int n = nx * ny;
-  const int c = threadIdx.x;
-  const bool act = c < n;
-  M kw = 0, ke = 0, ks = 0, kn = 0, di = 0, rc = 0;
-  int i = 0, j = 0;
-  if (act) {
-    i = c % nx;
-    j = c / nx;
-    kw = kx[i + (nx + 1) * j];
-    ke = kx[i + 1 + (nx + 1) * j];
-    ks = ky[i + nx * j];
-    kn = ky[i + nx * (j + 1)];
-    di = dinv[c];
-    rc = r[c];
-    xs[0][c] = omega * di * rc;
-  }
-  __syncthreads();
-  int cur = 0;
-  for (int s = 1; s < sweeps; ++s) {
-    if (act) {
-      const M* x = xs[cur];
-      M v = (((kw + ke) + ks) + kn) * x[c];
-      if (i > 0) v -= kw * x[c - 1];
-      if (i < nx - 1) v -= ke * x[c + 1];
-      if (j > 0) v -= ks * x[c - nx];
-      if (j < ny - 1) v -= kn * x[c + nx];
-      xs[cur ^ 1][c] = x[c] + omega * di * (rc - v);
-    }
-    __syncthreads();
-    cur ^= 1;
-  }
-  if (act) out[c] = xs[cur][c];
-}
-
-__device__ __forceinline__ void BlockSync() {
-  __threadfence_block();
-  __syncthreads();
-}
-
 // The coarse end of the V-cycle in one workgroup of kCcThreads threads:
 // levels first..last of the hierarchy (the first <= kInKernelMax cells, each
 // next one a quarter of it), the same smoothing / restriction / bilinear
@@ -907,6 +859,8 @@ MgPrecondT<M>::MgPrecondT(int nx, int ny, M* kx0, M* ky0, M* dinv0) {
       break;
     }
   }
+  if (lv_.size() > 1 && first_in_kernel_ < 0)  // (the last level always fits)
+    throw std::logic_error("MgPrecond: no level for the one-workgroup cycle");
 }
 
 template <class M>
@@ -959,7 +913,7 @@ void MgPrecondT<M>::Cycle(int l, const double* r64, float* z, M* out, hipStream_
   const FcgFusion fz = f ? *f : FcgFusion{};
   const int fused = (f && l == 0) ? 1 : 0;
   MgLevelT<M>& L = lv_[l];
-  if (l > 0 && l == first_in_kernel_ && use_coarse_kernel) {
+  if (l > 0 && l == first_in_kernel_) {
     CoarseSetT<M> cs{};
     cs.count = int(lv_.size()) - l;
     cs.bilinear = bilinear ? 1 : 0;
@@ -981,14 +935,7 @@ void MgPrecondT<M>::Cycle(int l, const double* r64, float* z, M* out, hipStream_
     KCoarseCycle<M><<<1, 1024, 0, st>>>(cs, sweeps, done);
     return;
   }
-  const bool coarsest = (l == int(lv_.size()) - 1);
-  if (coarsest && l > 0) {
-    // (a chain the one-workgroup cycle does not take: a long thin grid)
-    KCoarsest<M><<<1, kCoarsestMax, 0, st>>>(L.nx, L.ny, L.kx, L.ky, L.dinv, L.r, omega,
-                                              coarse_sweeps, out, done);
-    return;
-  }
-  if (coarsest) {
+  if (lv_.size() == 1) {
     // a single level (at most kTinyMax cells): eight Jacobi sweeps into z
     // (FP32), ping-ponging between xa and xb
     if constexpr (std::is_same<M, float>::value) {
