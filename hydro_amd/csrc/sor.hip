@@ -36,8 +36,8 @@
 // where the long side has room for several workgroups (KSorChain, below) the
 // b / (G P) steps of a sweep, plus once per solve the a + b to fill the
 // pipeline.  Per sweep, against the sweep-at-a-time kernel (101 sweeps unless
-// noted): 64x64 3.6 against 34.6 us; 256x128 at 701 sweeps 3.7 (one
-// workgroup 15.3) against 177 us; 333x217 13 (43) against 534 us.
+// noted): 64x64 3.7 against 34 us; 256x128 at 701 sweeps 3.7 (one workgroup 15.3)
+// against 177 us; 333x217 9.8 (44) against 440 us.
 // For one workgroup 1024 threads beat 512 and 256 (256x128: 15.3, 19.7, 30.9
 // us); for each of several 512 (256x128: 3.7; 1024: 7.2, 256: 4.8 us).
 #include "device_common.h"
@@ -100,7 +100,7 @@ KSorPack(int nx, int ny, Rows r, const double* __restrict__ k, int tr, double2* 
   // -0 where the reference's, which starts at +0, is +0; k + sum is then the
   // same)
   ck[d] = double2{r.c[c], k[c] + 0.};
-  xf[d] = 0.;
+  if (xf) xf[d] = 0.;
 }
 
 __global__ void __launch_bounds__(256)
@@ -743,8 +743,10 @@ bool LaunchSor(hipStream_t st, int nx, int ny, Rows a, const double* k, double* 
   double2 *xn = oc + n, *ck = xn + n;
   double* ring = reinterpret_cast<double*>(ck + n);
   const unsigned grid = unsigned((n + 255) / 256);
-  // the first sweeps' values: behind the ring, or the chain's result
-  double* const xf = ring + (many ? 1 : 2 * p.Q * p.rounds) * n;
+  // the first sweeps' values, if there is room: behind the ring, or the chain's
+  // result
+  const bool first = many ? c.first : p.first;
+  double* const xf = first ? ring + (many ? 1 : 2 * p.Q * p.rounds) * n : nullptr;
   KSorPack<<<grid, 256, 0, st>>>(nx, ny, a, k, tr, oc, xn, ck, xf, ws,
                                  many ? kChainRec : kSorHeader);
   if (many) {
@@ -752,10 +754,10 @@ bool LaunchSor(hipStream_t st, int nx, int ny, Rows a, const double* k, double* 
                 polls < 0 ? kSpin : polls};
     const int threads = c.Q * ch.ap;
     const size_t lds = size_t(2) * c.Q * (c.a + 2) * sizeof(double2) + size_t(8) * c.Q * 8;
-    double *out = ring, *logs = xf + n;
+    double *out = ring, *logs = out + (first ? 2 : 1) * n;
     for (int tail = 0; tail < 2; ++tail) {
       ch.tail = tail;
-      const unsigned g = tail ? 1u : unsigned(c.G) + 1u;
+      const unsigned g = tail ? 1u : unsigned(c.G + first);
       auto launch = [&](auto kernel) {
         kernel<<<g, threads, lds, st>>>(ch, oc, xn, ck, ws, logs, out, xf, tol, omega, info);
       };
@@ -771,10 +773,10 @@ bool LaunchSor(hipStream_t st, int nx, int ny, Rows a, const double* k, double* 
   const size_t lds = size_t(2) * p.Q * (p.a + 2) * sizeof(double2) +
                      size_t(p.rounds) * 2 * p.Q * 8 + 16;
   if (p.tr)
-    KSorPipe<true><<<2, threads, lds, st>>>(p.a, p.b, p.Q, p.rounds, oc, xn, ck, ring, xf, tol,
+    KSorPipe<true><<<1 + first, threads, lds, st>>>(p.a, p.b, p.Q, p.rounds, oc, xn, ck, ring, xf, tol,
                                             limit, omega, ws, info);
   else
-    KSorPipe<false><<<2, threads, lds, st>>>(p.a, p.b, p.Q, p.rounds, oc, xn, ck, ring, xf, tol,
+    KSorPipe<false><<<1 + first, threads, lds, st>>>(p.a, p.b, p.Q, p.rounds, oc, xn, ck, ring, xf, tol,
                                              limit, omega, ws, info);
   KSorUnpack<<<grid, 256, 0, st>>>(nx, ny, tr, ring, ws, x);
   return false;

@@ -48,6 +48,7 @@ struct SorPlan {
   int a = 0, b = 0;  // short and long side
   int Q = 0, rounds = 0;
   int G = 1, span = 0, le = 0;  // several workgroups (G > 1): see KSorChain
+  bool first = false;  // room for FirstSweeps, too (not at the cost of sweeps in flight)
   long doubles = 0;
 };
 
@@ -65,9 +66,11 @@ inline SorPlan PlanSor(int nx, int ny, int limit, long max_doubles) {
   int q = std::min(std::min(kSorThreads / std::max(p.a, 1), (p.b - 4) / 4), kSorMaxQ);
   q = std::min(q, limit / 2 + 1);  // sweeps 0 .. limit
   for (; q >= 1; --q) {
-    p.doubles = kSorHeader + (7 + 2L * q * p.rounds) * n;
+    p.doubles = kSorHeader + (6 + 2L * q * p.rounds) * n;
     // (32-bit byte offsets in the kernel)
     if (p.doubles <= max_doubles && p.doubles < (1L << 29)) {
+      p.first = p.doubles + n <= max_doubles;
+      p.doubles += p.first ? n : 0;
       p.Q = q;
       p.ok = true;
       break;
@@ -95,8 +98,10 @@ inline SorPlan PlanChain(int nx, int ny, int limit, long max_doubles) {
   for (; g >= 2; --g) {
     p.span = p.b / g;
     p.le = p.a + 2 * p.b + p.span + 64;
-    p.doubles = kChainHeader + 8 * n + long(g) * p.le * p.a;
+    p.doubles = kChainHeader + 7 * n + long(g) * p.le * p.a;
     if (p.doubles <= std::min(max_doubles, kSorMaxDoubles)) {
+      p.first = p.doubles + n <= max_doubles;
+      p.doubles += p.first ? n : 0;
       p.G = g;
       p.ok = true;
       break;
@@ -117,11 +122,11 @@ HG_HOST_DEVICE inline long ChainDoneStep(int s, int P, int ptot, int span, int a
 constexpr int kChainMaxStep = 1 << 30;
 
 // Several workgroups where they hold more sweeps than one does.  Measured per
-// sweep, one | several (stages held): 64x128 5.7 | 4.5 us (32 | 48), 64x256
-// 10.2 | 5.2 us (32 | 112), 256x128 at 700 sweeps 15.3 | 3.7 us (16 | 56),
-// 333x217 at 100 43.5 | 13.2 us (8 | 52); with fewer stages they lose: 32x128
-// 3.7 | 4.2 us (64 | 48), 16x256 4.0 | 5.2 us (128 | 112), as the lines are
-// padded to waves.
+// sweep at 701 sweeps, one | several (stages held): 64x256 7.6 | 3.2 us (32 | 64),
+// 256x128 15.3 | 3.7 (16 | 56), 333x217 40 | 6.1 (8 | 44), 512x512 130 | 11.4
+// (4 | 42), 30x700 10.1 | 3.1 (64 | 208); where they do not: 16x256 2.6 | 3.4 us
+// (64 | 64), 32x128 2.2 | 3.0 (62 | 32), 64x128 4.0 | 3.1 (32 | 32), as the lines
+// are padded to waves.
 // Nor on lines of under 16 cells, of which one workgroup holds 64 sweeps: solves
 // of few sweeps, which take a chain twice as long (it repeats them), then lose
 // against a sweep at a time.  3x700 at 9 | 101 sweeps 468 | 800 us by one, 1353 |
@@ -133,11 +138,15 @@ inline bool UseChain(const SorPlan& one, const SorPlan& many) {
 
 // The workspace of a solve of at most limit + 1 sweeps.
 inline long SorWorkspaceDoubles(int nx, int ny, int limit) {
-  auto ring = [&](long cap) {
-    SorPlan p = PlanSor(nx, ny, limit, cap);
-    return p.ok ? p : PlanSor(nx, ny, std::min(limit, 0), 1L << 60);
+  auto first = [&](SorPlan p) {
+    if (p.ok && !p.first) p.doubles += long(nx) * ny;
+    return p;
   };
-  const SorPlan p = ring(kSorMaxDoubles), c = PlanChain(nx, ny, limit, kSorMaxDoubles);
+  auto ring = [&](long cap) {
+    const SorPlan p = PlanSor(nx, ny, limit, cap);
+    return first(p.ok ? p : PlanSor(nx, ny, std::min(limit, 0), 1L << 60));
+  };
+  const SorPlan p = ring(kSorMaxDoubles), c = first(PlanChain(nx, ny, limit, kSorMaxDoubles));
   if (!UseChain(p, c)) return p.ok ? p.doubles : 0;
   const SorPlan retry = ring(std::max(c.doubles, kRetryMaxDoubles));
   return std::max(c.doubles, retry.ok ? retry.doubles : 0);

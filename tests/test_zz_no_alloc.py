@@ -160,3 +160,29 @@ def test_noalloc_from_several_threads(gpu):
         for job in jobs:
             hip.lib.hipStreamDestroy(job[5])
         hip.free()
+
+
+# at the scratch array's limits: no room for the first sweeps' values beside two
+# pairs and one pair of sweeps, a chain of fewer workgroups than its own workspace
+# would hold, no room for two sweeps
+@pytest.mark.parametrize("nx,ny", [(340, 435), (700, 290), (333, 217), (700, 320)])
+@pytest.mark.parametrize("tol", [0.0, 1e9])
+def test_noalloc_sor_at_the_scratch_limits(gpu, nx, ny, tol):
+    lib = capi.load()
+    hip = _Hip()
+    print(f"case: noalloc gauss_seidel {nx}x{ny} tol {tol}", flush=True)
+    rows = _system(nx, ny, 5)
+    sid = capi.SOLVERS["gauss_seidel"]
+    x_ref, st_ref = stencil_solve(nx, ny, *rows, sid, tol=tol, max_iters=30, omega=1.5)
+    try:
+        dev = [hip.upload(a) for a in rows]
+        dx = hip.upload(np.full(nx * ny, np.nan))
+        opts = capi.HgSolveOpts(solver=sid, tolerance=tol, max_iters=30, relaxation_factor=1.5,
+                                precision=0)
+        st = capi.HgSolveStats()
+        assert _noalloc(lib)(nx, ny, *dev, dx, ctypes.byref(opts), ctypes.byref(st),
+                             None) == capi.HG_OK
+        assert np.array_equal(hip.download(dx, nx * ny), x_ref)
+        assert st.iterations == st_ref.iterations
+    finally:
+        hip.free()
