@@ -56,7 +56,7 @@ def test_last_step_of_any_limit(plan):
 
 
 def test_workspace_is_bounded(plan):
-    """512 MB, or two sweeps' ring where that is more (11 or 13 doubles per cell);
+    """512 MB and a double per cell, or two sweeps' ring where that is more;
     a solve of few sweeps asks for less; a chain's holds a ring for the retry."""
     grids = GRIDS + [(64, 65536), (32, 120000), (512, 1024), (1024, 20000), (2, 4000000)]
     cases = [(nx, ny, lim) for nx, ny in grids for lim in (-3, 0, 5, 1000, 2**31 - 1)]
