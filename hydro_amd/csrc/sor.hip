@@ -116,6 +116,19 @@ KSorUnpack(int nx, int ny, int tr, const double* __restrict__ ring,
   x[c] = ring[slot * nx * ny + long(row) * a + t];
 }
 
+// The same by `threads` threads of a workgroup that has formed the values, for grids
+// so small (kCopyOutCells) that a launch of its own costs more: 101 sweeps of 24x24
+// 197 us with the launch, 193 this way, 64x64 376 and 373.
+template <bool TR>
+__device__ __forceinline__ void CopyOut(int a, int b, const double* from, double* __restrict__ x,
+                                        int t, int threads) {
+  for (int d = t; d < a * b; d += threads) {
+    const int row = d / a, l = d - row * a;
+    const int m = row >= l ? row - l : row - l + b;
+    x[TR ? m + b * l : l + a * m] = from[d];
+  }
+}
+
 __device__ __forceinline__ double AgentLoad(const double* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -148,14 +161,15 @@ __device__ __forceinline__ double SorCell(const SorRow& r, double own, double cr
 //
 // Device time in us of a solve that ends in its first and second sweep (launches
 // and the read back of info, about 40, in all of them): a sweep at a time in place,
-// the pipeline alone, with this: 16x16 46, 60 | 56, 57 | 51, 58; 64x64 102, 135 |
-// 162, 165 | 74, 96; 128x128 249, 338 | 411, 418 | 103, 160; 512x512 3490, 5690 |
+// the pipeline alone, with this: 16x16 48, 62 | 55, 57 | 52, 58; 64x64 102, 135 |
+// 162, 165 | 79, 102; 128x128 249, 338 | 411, 418 | 103, 160; 512x512 3490, 5690 |
 // 1776, 1808 | 478, 890.  A third sweep would end after the pipeline could (512x512:
 // two take 840 us, the pipeline's first decision 900) and gain little elsewhere.
 //
 // Thread t takes line t, one row per step.  The value before it on its line stays
 // in a register, that of line t - 1 comes by a lane shift, between waves through
-// LDS: wave w is w groups of kG steps behind the first, one barrier per group.
+// LDS: wave w is w groups of kG steps behind the first, one barrier per group (kG 4,
+// or 3 where 4 would make the kernel spill registers).
 // All operands are loaded kG steps ahead; an old value is loaded before the step
 // that writes its cell, by the same wave or by one a group behind.
 template <bool TR, int kG>
@@ -163,7 +177,8 @@ __device__ __forceinline__ void FirstSweeps(int a, int b, const double2* __restr
                                             const double2* __restrict__ xn,
                                             const double2* __restrict__ ck, double* xf, double tol,
                                             int limit, double omega, long long slot, int* word,
-                                            double* head, unsigned long long* __restrict__ info) {
+                                            double* head, unsigned long long* __restrict__ info,
+                                            double* __restrict__ x) {
   constexpr int kRing = 16;
   __shared__ double edge[kSorThreads / 64][kRing];  // values of a wave's last lane, by step
   __shared__ double red[kSorThreads / 64];
@@ -238,6 +253,7 @@ __device__ __forceinline__ void FirstSweeps(int a, int b, const double2* __restr
         reinterpret_cast<long long*>(head)[1] = slot;
         __hip_atomic_fetch_min(word, kEndedFirst, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
+      if (x) CopyOut<TR>(a, b, xf, x, t, 64 * nw);
       return;
     }
     if (s + 1 == kFirstSweeps) return;
@@ -248,25 +264,29 @@ template <bool TR>
 __global__ void __launch_bounds__(kSorThreads)
 KSorPipe(int a, int b, int Q, int rounds, const double2* __restrict__ oc,
          const double2* __restrict__ xn, const double2* __restrict__ ck, double* ring, double* xf,
-         double tol, int limit, double omega, double* head,
-         unsigned long long* __restrict__ info) {
+         double tol, int limit, double omega, double* head, unsigned long long* __restrict__ info,
+         double* __restrict__ x) {
   // [2 step parities][Q][a + 2] values (first, second stage) with a zero
   // pad either side, then the sweeps' maxima
   extern __shared__ double2 lds2[];
   __shared__ int flag;  // 1 + the group of four steps in which a sweep ended the solve
+  __shared__ int result;  // its ring slot, if a sweep of this workgroup did
   const int W = a + 2;
   double2* const val = lds2;
   unsigned long long* const sd = reinterpret_cast<unsigned long long*>(lds2 + 2 * Q * W);
   const int P = 2 * Q, R = rounds * P;
   int* const word = reinterpret_cast<int*>(head);  // kNever until FirstSweeps ends the solve
   if (blockIdx.x == 1) {
-    FirstSweeps<TR, 4>(a, b, oc, xn, ck, xf, tol, limit, omega, R, word, head, info);
+    FirstSweeps<TR, 3>(a, b, oc, xn, ck, xf, tol, limit, omega, R, word, head, info, x);
     return;
   }
   const int tid = threadIdx.x;
   for (int z = tid; z < 2 * Q * W; z += blockDim.x) val[z] = double2{0., 0.};
   for (int z = tid; z < R; z += blockDim.x) sd[z] = 0ull;
-  if (tid == 0) flag = 0;
+  if (tid == 0) {
+    flag = 0;
+    result = -1;
+  }
   __syncthreads();
   const bool live = tid < Q * a;
   const int q = live ? tid / a : 0, t = live ? tid - q * a : 0;
@@ -330,6 +350,7 @@ KSorPipe(int a, int b, int Q, int rounds, const double2* __restrict__ oc,
   LoadPrev(g[0], m, slot, RowOn(off));
   double2* const mine = val + q * W + t;
   double ownA = 0., ownB = 0., oldA = 0., h1 = 0., h2 = 0., dA = 0., dB = 0.;
+  const int look = (a + b) / 4 + kFirstSweeps;
   int group = 0, ended = kNever;
   // sweep s (in ring slot `idx`) has just finished: the stop rule,
   // do { sweep } while (diff > tol && iter++ < limit), sweeps in order
@@ -343,11 +364,13 @@ KSorPipe(int a, int b, int Q, int rounds, const double2* __restrict__ oc,
       info[0] = (unsigned long long)(met ? s : s + 1);
       info[1] = bits;
       reinterpret_cast<long long*>(head)[1] = idx;
+      result = idx;
       flag = group + 1;
     }
   };
   for (;; ++group) {
-    if (tid == 0) {  // (as the group before found it: no wait)
+    // (from step a + b + 2 kFirstSweeps on this workgroup has decided them itself)
+    if (group < look && tid == 0) {  // as the group before found it
       if (ended != kNever && !flag) flag = group + 1;
       ended = AgentLoad(word);
     }
@@ -426,6 +449,11 @@ KSorPipe(int a, int b, int Q, int rounds, const double2* __restrict__ oc,
     const int f = flag;
     if (f != 0 && f <= group + 1) break;
   }
+  if (x) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // every wave's values are in the ring
+    __syncthreads();
+    if (result >= 0) CopyOut<TR>(a, b, ring + size_t(result) * (n8 / 8u), x, tid, blockDim.x);
+  }
 }
 
 // ---- several workgroups -----------------------------------------------------
@@ -469,7 +497,8 @@ KSorChain(SorChain ch, const double2* __restrict__ oc, const double2* __restrict
   const long log_n = long(le) * a;
   int G = ch.G, wg = blockIdx.x, limit = ch.limit;
   if (wg == G) {
-    FirstSweeps<TR, MAXT <= 512 ? 4 : 3>(a, b, oc, xn, ck, xf, tol, limit, omega, 1, stop, head, info);
+    FirstSweeps<TR, MAXT <= 512 ? 4 : 3>(a, b, oc, xn, ck, xf, tol, limit, omega, 1, stop, head, info,
+                                           nullptr);
     return;
   }
   // where the first stage's input comes from: the log of workgroup `src`, the
@@ -769,16 +798,17 @@ bool LaunchSor(hipStream_t st, int nx, int ny, Rows a, const double* k, double* 
     KSorUnpack<<<grid, 256, 0, st>>>(nx, ny, tr, out, ws, x);
     return true;
   }
+  double* const out = n <= kCopyOutCells ? x : nullptr;
   const int threads = (p.Q * p.a + 63) / 64 * 64;
   const size_t lds = size_t(2) * p.Q * (p.a + 2) * sizeof(double2) +
                      size_t(p.rounds) * 2 * p.Q * 8 + 16;
   if (p.tr)
-    KSorPipe<true><<<1 + first, threads, lds, st>>>(p.a, p.b, p.Q, p.rounds, oc, xn, ck, ring, xf, tol,
-                                            limit, omega, ws, info);
+    KSorPipe<true><<<1 + first, threads, lds, st>>>(p.a, p.b, p.Q, p.rounds, oc, xn, ck, ring, xf,
+                                                    tol, limit, omega, ws, info, out);
   else
-    KSorPipe<false><<<1 + first, threads, lds, st>>>(p.a, p.b, p.Q, p.rounds, oc, xn, ck, ring, xf, tol,
-                                             limit, omega, ws, info);
-  KSorUnpack<<<grid, 256, 0, st>>>(nx, ny, tr, ring, ws, x);
+    KSorPipe<false><<<1 + first, threads, lds, st>>>(p.a, p.b, p.Q, p.rounds, oc, xn, ck, ring, xf,
+                                                     tol, limit, omega, ws, info, out);
+  if (!out) KSorUnpack<<<grid, 256, 0, st>>>(nx, ny, tr, ring, ws, x);
   return false;
 }
 

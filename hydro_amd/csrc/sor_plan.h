@@ -17,6 +17,7 @@ constexpr int kSorMaxQ = 32;
 constexpr int kSorHeader = 32;  // doubles before the arrays: [0] kNever, [1] the result's slot
 constexpr int kFirstSweeps = 2;  // of FirstSweeps
 constexpr int kEndedFirst = -2;
+constexpr long kCopyOutCells = 4096;
 
 // (several workgroups, below)
 constexpr int kLag = 20;
