@@ -157,7 +157,7 @@ __device__ __forceinline__ double SorCell(const SorRow& r, double own, double cr
 // after another in xf; if the stop rule is met within them it ends the solve:
 // info, the result's slot, `word` lowered to kEndedFirst.  The pipeline leaves
 // when it sees that.  Where both end the solve they do at the same sweep, with
-// the same values.
+// the same values.  Neither waits for the other.
 //
 // Device time in us of a solve that ends in its first and second sweep (launches
 // and the read back of info, about 40, in all of them): a sweep at a time in place,
